@@ -140,7 +140,7 @@ typedef struct ovfcc_request ovfcc_request; /* one HIP stream + staging + split-
 /* kernel families, as reported by ovfcc_last_kernel_info and accepted by ovfcc_request_force_kernel */
 enum ovfcc_kernel {
     OVFCC_KERNEL_AUTO = 0,
-    OVFCC_KERNEL_PLAIN = 1,  /* any shape, OpenVINO layout, one wave per output channel */
+    OVFCC_KERNEL_PLAIN = 1,  /* shapes that do not tile: any N, K and group size */
     OVFCC_KERNEL_DECODE = 2, /* M <= 48: the streaming and the small-batch kernel over the tiled layout */
     OVFCC_KERNEL_PREFILL = 3 /* more rows: MFMA tile kernels over the tiled layout (N % 128 == 0) */
 };
@@ -209,7 +209,7 @@ int ovfcc_weights_glu(const ovfcc_weights* gate, const ovfcc_weights* up, int gl
 int ovfcc_weights_mlp(const ovfcc_weights* gate_up, const ovfcc_weights* down, ovfcc_weights** out);
 /* device bytes held by the repacked node */
 int64_t ovfcc_weights_device_bytes(const ovfcc_weights* w);
-/* 1 when the node uses the tiled layout (fast kernels), 0 for the OpenVINO-layout fallback */
+/* 1 when the node uses the tiled layout, 0 when its shape does not tile */
 int ovfcc_weights_is_tiled(const ovfcc_weights* w);
 
 /* The node in its device form as one relocatable host blob, and back: what ICompiledModel::export_model /

@@ -179,6 +179,33 @@ void fill_args(const ovfcc_weights* w, const void* x, void* y, int64_t M, ovfcc:
     a->layout = w->layout;
 }
 
+// The weights of a ragged node, wb bytes as OpenVINO packs them: uploaded, and brought into the order its kernels read
+// on the device.
+constexpr size_t kArrangeMax = (size_t)16 << 20;
+int upload_ragged(ovfcc_weights* W, const void* w, size_t wb) {
+    ovfcc_ctx* c = W->ctx;
+    HIP_TRY(hipMalloc(&W->d_w, W->layout.w_bytes));
+    W->bytes += W->layout.w_bytes;
+    std::unique_lock<std::mutex> lock(c->arrange_mu, std::defer_lock);
+    void* given = nullptr;
+    if (wb <= kArrangeMax) {
+        lock.lock();
+        int rc = grow(&c->d_arrange, &c->arrange_cap, wb);
+        if (rc)
+            return rc;
+        given = c->d_arrange;
+    } else {
+        HIP_TRY(hipMalloc(&given, wb));
+    }
+    hipError_t e = hipMemcpy(given, w, wb, hipMemcpyHostToDevice);
+    if (e == hipSuccess)
+        e = (hipError_t)ovfcc::launch_ragged_repack(W->desc, W->layout, given, W->d_w, nullptr);
+    const hipError_t done = hipStreamSynchronize(nullptr);
+    if (!lock.owns_lock())
+        (void)hipFree(given);
+    return e != hipSuccess ? hip_fail(e, "arranging the weights") : done != hipSuccess ? hip_fail(done, "arranging the weights") : OVFCC_OK;
+}
+
 // Last step of every way a node comes into being: tiled 4-bit nodes with groups of 128 inputs get channel-major
 // copies of their scales and zero-point table, [N/16][16][K/128], which the matrix-vector kernel reads.
 int finish_weights(ovfcc_weights* W) {
@@ -444,6 +471,20 @@ int enqueue_rows(ovfcc_request* r, const ovfcc_weights* w, const void* x, void* 
         shown.grid[0] = (unsigned)(w->desc.N / 256), shown.grid[1] = (unsigned)((M + 127) / 128);
         shown.name = grouped ? "fcc_prefill_i8_w4_grouped" : "fcc_prefill_i8_w4";
         record(r, shown);
+        return OVFCC_OK;
+    }
+    if ((force == OVFCC_KERNEL_AUTO || force == OVFCC_KERNEL_PLAIN) && L0.ragged) {
+        ovfcc::LaunchPlan p;
+        ovfcc::plan_ragged(a, r->ctx->n_cus, &p);
+        int rc = split_buffers(r, p, static_scratch, &a);
+        if (rc)
+            return rc;
+        int e = ovfcc::launch_ragged(a, p, r->stream);
+        if (e)
+            return hip_fail((hipError_t)e, "kernel launch");
+        if (static_scratch && (rc = static_scratch_released(r, a)))
+            return rc;
+        record(r, p);
         return OVFCC_OK;
     }
     bool chunked = w->layout.tiled && M > ovfcc::kDecodeMaxRows &&
@@ -869,6 +910,8 @@ int ovfcc_init(int device, ovfcc_ctx** out) {
 void ovfcc_destroy(ovfcc_ctx* ctx) {
     if (ctx && ctx->coop_done)
         (void)hipEventDestroy(ctx->coop_done);
+    if (ctx && ctx->d_arrange)
+        (void)hipFree(ctx->d_arrange);
     delete ctx;
 }
 
@@ -939,7 +982,7 @@ int ovfcc_weights_create(ovfcc_ctx* ctx, const ovfcc_fc_desc* desc, const void* 
     } else {
         const bool four = desc->w_type == OVFCC_U4 || desc->w_type == OVFCC_I4;
         const size_t wb = four ? (size_t)(N * K + 1) / 2 : (size_t)N * K;
-        rc = upload(&W->d_w, w, wb);
+        rc = L.ragged ? upload_ragged(W, w, wb) : upload(&W->d_w, w, wb);
         if (!rc)
             rc = upload(&W->d_scale, scales, (size_t)N * ng * 2);
         if (!rc && desc->zp_type != OVFCC_NONE) {
@@ -970,7 +1013,7 @@ int ovfcc_weights_create(ovfcc_ctx* ctx, const ovfcc_fc_desc* desc, const void* 
         const auto t_end = std::chrono::steady_clock::now();
         std::fprintf(stderr, "ovfcc: weights N=%lld K=%lld group=%lld w_type=%d zp_type=%d%s: %s layout, %zu bytes on the "
                      "device, repack %.2f ms, upload %.2f ms\n", (long long)N, (long long)K, (long long)desc->group_size,
-                     desc->w_type, desc->zp_type, desc->zp_scalar ? " (scalar)" : "", L.tiled ? "tiled" : "OpenVINO",
+                     desc->w_type, desc->zp_type, desc->zp_scalar ? " (scalar)" : "", L.tiled ? "tiled" : L.ragged ? "ragged" : "OpenVINO",
                      W->bytes, ms(t_repacked - t_start).count(), ms(t_end - t_repacked).count());
     }
     *out = W;
@@ -1009,7 +1052,7 @@ int ovfcc_weights_clone(const ovfcc_weights* src, ovfcc_weights** out) {
         sb = L.scale_bytes;
         zb = L.zp_bytes;
     } else {
-        wb = four ? (size_t)(N * K + 1) / 2 : (size_t)N * K;
+        wb = L.ragged ? L.w_bytes : four ? (size_t)(N * K + 1) / 2 : (size_t)N * K;
         sb = (size_t)N * ng * 2;
         if (src->desc.zp_type != OVFCC_NONE) {
             const size_t cnt = src->desc.zp_scalar ? 1 : (size_t)N * ng;
@@ -1241,7 +1284,7 @@ struct BlobHeader {
     int32_t tiled;        // kBlobTiled | kBlobHasDown
     uint64_t w_bytes, scale_bytes, zp_bytes, bias_bytes;
 };
-constexpr uint32_t kBlobVersion = 2;
+constexpr uint32_t kBlobVersion = 3;
 constexpr int32_t kBlobTiled = 1, kBlobHasDown = 2;  // bits of BlobHeader::tiled; HasDown: another node's blob follows
 const char kBlobMagic[8] = {'O', 'V', 'F', 'C', 'C', 'W', 0, 0};
 
@@ -1255,7 +1298,7 @@ void device_sizes(const ovfcc_fc_desc& d, const ovfcc::Layout& L, uint64_t out[4
     if (L.tiled) {
         out[0] = L.w_bytes, out[1] = L.scale_bytes, out[2] = L.zp_bytes;
     } else {
-        out[0] = L.bits == 4 ? (uint64_t)(N * K + 1) / 2 : (uint64_t)N * K;
+        out[0] = L.ragged ? L.w_bytes : L.bits == 4 ? (uint64_t)(N * K + 1) / 2 : (uint64_t)N * K;
         out[1] = (uint64_t)N * ng * 2;
         out[2] = 0;
         if (d.zp_type != OVFCC_NONE) {

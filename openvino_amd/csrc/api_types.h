@@ -18,6 +18,11 @@ struct ovfcc_ctx {
     // their kind: each waits, on its stream, for the event recorded behind the one before it.
     std::mutex coop_mu;
     hipEvent_t coop_done = nullptr;
+    // Where the constants of ragged nodes lie as given until they are arranged: up to kArrangeMax bytes, kept between
+    // nodes (an allocation and a release cost more than arranging a small node), given back with the context.
+    std::mutex arrange_mu;
+    void* d_arrange = nullptr;
+    size_t arrange_cap = 0;
 };
 
 struct ovfcc_weights {

@@ -1,4 +1,5 @@
-// Fallback kernel for shapes that keep OpenVINO's constant layout, and the small helper kernels of the routed calls.
+// Kernel for nodes that keep OpenVINO's constant layout (several groups per channel, or a gated linear unit, at widths
+// that do not tile), and the small helper kernels of the routed calls.
 // Semantics: the scalar reference kernel of the OpenVINO Intel-GPU plugin
 // (src/plugins/intel_gpu/src/kernel_selector/cl_kernels/fully_connected_gpu_bfyx_ref.cl:88-160).
 #include "device_common.h"

@@ -55,6 +55,12 @@ struct Layout {
     bool glu_gate_second = false;
     int gemv_c = 0;         // k-blocks per wave of the matrix-vector kernel, fixed when the node's channel-major
                             // parameter tables are written (0: the node has none)
+    // Nodes that fit no tile but have one scale per channel and no gated linear unit: the weights alone are repacked,
+    // into operand order with N padded to 16 channels and K to 128 inputs (codes unsigned as in a tile, padding zero),
+    // [N/16][K/128][step j of 32 inputs][lane][8 weights]: lane l holds channel l & 15, inputs 32 j + 8 (l >> 4) + e of
+    // the k-block -- the bytes of two dwords (8-bit) or the dword (4-bit) that a tile keeps for it.  A wave that
+    // contracts one step of every k-block reads 512 (256) contiguous bytes.  Scales, zero-points and bias stay as given.
+    bool ragged = false;
     bool dynquant = false;  // the node allows int8 activations (OVFCC_DYNQUANT_I8) where a kernel exists
     bool dynquant_grouped = false;  // ... quantised per group of 128 inputs rather than per token (4-bit nodes)
     bool dynquant_asym = false;     // ... as unsigned bytes with a zero-point per token (8-bit per-channel nodes)
@@ -179,6 +185,11 @@ unsigned env_generation();
 // Enqueues on `stream` (a hipStream_t passed as void*); returns a HIP error code (0 = success).
 int launch_fc(const FcDeviceArgs& a, const LaunchPlan& plan, void* stream);
 int launch_plain(const FcDeviceArgs& a, const LaunchPlan& plan, void* stream);
+// Decomposition and launch of a call on a node with Layout::ragged (kernel_ragged.hip).
+// launch_ragged_repack brings the constants into that layout (w as OpenVINO packs it, w_out L.w_bytes, both on the device).
+int launch_ragged_repack(const ovfcc_fc_desc& d, const Layout& L, const void* w, void* w_out, void* stream);
+void plan_ragged(const FcDeviceArgs& a, int n_cus, LaunchPlan* plan);
+int launch_ragged(const FcDeviceArgs& a, const LaunchPlan& plan, void* stream);
 int launch_decode(const FcDeviceArgs& a, const LaunchPlan& plan, void* stream);
 int launch_batch(const FcDeviceArgs& a, const LaunchPlan& plan, void* stream);
 int launch_gemv(const FcDeviceArgs& a, const LaunchPlan& plan, void* stream);

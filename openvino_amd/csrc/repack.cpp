@@ -107,6 +107,11 @@ Layout make_layout(const ovfcc_fc_desc& d) {
         L.w_bytes = (size_t)L.n_tiles * L.k_blocks * L.tiles_per_kblock * kTileBytes;
         L.scale_bytes = (size_t)L.n_tiles * L.groups * kTileRows * 2;
         L.zp_bytes = L.zp_table ? (size_t)L.n_tiles * L.groups * kTileRows : 0;
+    } else if (L.groups == 1 && !L.glu && d.K >= 8) {  // (eight inputs: one 16-byte load of activations)
+        L.ragged = true;
+        L.n_tiles = (d.N + kTileRows - 1) / kTileRows;
+        L.k_blocks = (d.K + kBlockK - 1) / kBlockK;
+        L.w_bytes = (size_t)L.n_tiles * L.k_blocks * kTileRows * kBlockK * L.bits / 8;
     }
     return L;
 }
@@ -366,7 +371,7 @@ int ovfcc_tiled_sizes(const ovfcc_fc_desc* desc, size_t* w_bytes, size_t* scale_
     if (rc != OVFCC_OK)
         return rc;
     const ovfcc::Layout L = ovfcc::make_layout(*desc);
-    *w_bytes = L.w_bytes;
+    *w_bytes = L.tiled ? L.w_bytes : 0;
     *scale_bytes = L.scale_bytes;
     *zp_bytes = L.zp_bytes;
     return OVFCC_OK;

@@ -1,0 +1,77 @@
+"""GPU parity of nodes with one scale per channel whose widths fit no tile (OpenVINO layout, matrix-core kernels that
+read the constants as they lie) against the CPU oracle: tails of K and N, row tiles of 16 and 64 rows and their edges,
+K split over workgroups, every zero-point form, both output types.  Weights are exact integers in the kernels and the
+products are summed in f32, so f32 outputs agree with a float64 sum to K 2^-24 of the sum of magnitudes, here bounded
+as 1e-5 relative in the 2-norm; f16 outputs add their own rounding (the bounds of tests/parity.py)."""
+import numpy as np
+import pytest
+
+from openvino_amd import datagen, fc
+from parity import check_parity, oracle_y
+
+pytestmark = pytest.mark.gpu
+
+MS = [1, 15, 16, 17, 32, 33, 63, 64, 65, 130]
+
+
+@pytest.fixture(scope="module")
+def dev():
+    d = fc.Device(0)
+    yield d
+    d.close()
+
+
+@pytest.fixture()
+def req(dev):
+    r = fc.InferRequest(dev)
+    yield r
+    r.close()
+
+
+@pytest.mark.parametrize("wt,zt,N,K,bias,out,scalar", [
+    ("i8", "none", 1000, 2048, True, "f32", False),   # a classifier head: N % 16 == 8
+    ("u8", "u8", 40, 200, False, "f16", False),       # K % 128 != 0
+    ("i8", "u8", 67, 1161, True, "f16", False),       # both odd: single halves at the end of a row, 2-byte rows
+    ("u8", "none", 5, 8, False, "f32", False),        # one chunk of eight inputs
+    ("i8", "none", 63, 9, True, "f32", False),
+    ("u8", "u8", 130, 4300, True, "f16", True),       # long K: split over workgroups
+    ("i4", "none", 65, 1160, True, "f32", False),     # nibbles
+    ("u4", "u4", 33, 650, False, "f16", False),
+    ("i4", "u8", 17, 4102, False, "f32", False),
+    ("u4", "u4", 300, 130, True, "f16", True),
+])
+def test_widths_that_fit_no_tile(oracle, dev, req, wt, zt, N, K, bias, out, scalar):
+    c = datagen.make_case(2100 + N, max(MS), K, N, wt, K, zt, with_bias=bias)
+    if scalar:
+        c.zp = c.zp[:1].copy()
+        c.zp_scalar = True
+    ref = oracle_y(oracle, c)
+    w = fc.CompressedWeights.from_case(dev, c, output_type=out)
+    try:
+        assert not w.tiled
+        for M in MS:
+            print(f"ragged {wt}/{zt} N={N} K={K} M={M}", flush=True)
+            y = req.infer(w, c.x[:M])
+            check_parity(oracle, y, ref[:M], K, f"{wt}/{zt} N={N} K={K} M={M}", output_rounding_slack=True)
+            if out == "f32":
+                assert oracle.rel_l2(y, ref[:M]) < 1e-5
+            assert np.array_equal(y, req.infer(w, c.x[:M]))
+    finally:
+        w.close()
+
+
+def test_rows_keep_to_themselves(dev, req):
+    """A row's result does not see its neighbours: what a lane loads beyond the end of a row is the next row, here
+    infinities and NaNs."""
+    for M in (3, 40):
+        c = datagen.make_case(2200, M, 203, 50, "i8", 203, "none")
+        w = fc.CompressedWeights.from_case(dev, c, output_type="f32")
+        try:
+            clean = req.infer(w, c.x)
+            x = c.x.copy()
+            x[1::2] = np.inf
+            x[1, 0] = np.nan
+            dirty = req.infer(w, x)
+            assert np.array_equal(clean[0::2], dirty[0::2]) and not np.isfinite(dirty[1::2]).any()
+        finally:
+            w.close()
