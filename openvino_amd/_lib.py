@@ -207,6 +207,15 @@ def load() -> ctypes.CDLL:
     return L
 
 
+# every override the library's table holds (csrc/plan.cpp)
+ENV_NAMES = tuple("OVFCC_" + n for n in (
+    "DECODE_WAVES DECODE_RT DECODE_XLDS DECODE_BATCH GEMV GEMV_C GEMV16 GEMV16_GRID GEMV16_SPLIT GEMV16_STREAM "
+    "GEMV16_STREAM_TILES PREFILL_DIRECT PREFILL_ASYNC PREFILL_WIDE PREFILL_BIG PREFILL_TAIL PREFILL_ROWS "
+    "MOE_HOST_ROUTING MLP_FUSED MLP_SPIN_LIMIT MLP_GRID VERBOSE").split())
+# os.environ decodes every entry it hands out: at 18 us a look it cost more than a decode launch.  The mapping
+# underneath it holds the encoded entries, and a handful of lookups there take 1 us.
+_env_raw = getattr(os.environ, "_data", None)
+_env_keys = None if _env_raw is None else tuple(os.environ.encodekey(n) for n in ENV_NAMES)
 _env_seen = None
 
 
@@ -214,9 +223,9 @@ def sync_env() -> None:
     """The library reads its OVFCC_* overrides once; a Python host that changes os.environ afterwards (tests,
     experiments) has them read again before its next call."""
     global _env_seen
-    now = tuple(sorted((k, v) for k, v in os.environ.items() if k.startswith("OVFCC_")))
+    now = tuple(map(os.environ.get, ENV_NAMES)) if _env_raw is None else tuple(map(_env_raw.get, _env_keys))
     if now != _env_seen:
-        if _env_seen is not None or now:
+        if _env_seen is not None or any(v is not None for v in now):
             load().ovfcc_env_reload()
         _env_seen = now
 

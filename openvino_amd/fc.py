@@ -309,14 +309,13 @@ class InferRequest:
         X = np.ascontiguousarray(X, dtype=np.float16)
         if X.shape[-1] != weights.K:
             raise OvfccError(_lib.EINVAL, f"last dimension of X is {X.shape[-1]}, expected K = {weights.K}")
-        M = int(np.prod(X.shape[:-1], dtype=np.int64))
+        M = X.size // weights.K
         Y = np.empty(X.shape[:-1] + (weights.N_out,), dtype=np.float32 if weights.out_f32 else np.float16)
-        check(self.device.lib.ovfcc_fc_run(self.handle, weights.handle, _vp(X), _vp(Y), M))
+        check(self.device.lib.ovfcc_fc_run(self.handle, weights.handle, X.ctypes.data, Y.ctypes.data, M))
         return Y
 
     def infer_device(self, weights: CompressedWeights, x_ptr: int, y_ptr: int, M: int) -> None:
-        check(self.device.lib.ovfcc_fc_run_device(self.handle, weights.handle, ctypes.c_void_p(x_ptr),
-                                                  ctypes.c_void_p(y_ptr), M))
+        check(self.device.lib.ovfcc_fc_run_device(self.handle, weights.handle, x_ptr, y_ptr, M))
 
     def infer_device_static(self, weights: CompressedWeights, x_ptr: int, y_ptr: int, M: int) -> None:
         """infer_device through the entry point that allocates nothing (fixed scratch array instead of buffers of
