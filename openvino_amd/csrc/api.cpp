@@ -371,7 +371,24 @@ int enqueue(ovfcc_request* r, const ovfcc_weights* w, const void* x, void* y, in
     return OVFCC_OK;
 }
 
-// plan_launch for a call of the node on its own (fill_args's arguments, nothing set by a grouped run), through the
+// The plan of one launch: plan_launch's, or the weight-streaming kernel's where that takes the call and nothing forces
+// another.
+int plan_call(const ovfcc_request* r, const ovfcc::FcDeviceArgs& a, int force, ovfcc::LaunchPlan* p) {
+    int rc = ovfcc::plan_launch(a, force, r->force_split, r->ctx->n_cus, p);
+    if (rc)
+        return rc;
+    if ((force == OVFCC_KERNEL_AUTO || force == OVFCC_KERNEL_DECODE) && r->force_split == 0 &&
+        ovfcc::env_int("OVFCC_DECODE_BATCH", -1) < 0 && ovfcc::env_int("OVFCC_GEMV16_SPLIT", 0) == 0 &&
+        ovfcc::env_int("OVFCC_GEMV16_STREAM", -1) < 0 && ovfcc::stream_preferred(a, *p))
+        ovfcc::plan_stream(a, r->ctx->n_cus, p);
+    return OVFCC_OK;
+}
+
+int launch_call(const ovfcc::FcDeviceArgs& a, const ovfcc::LaunchPlan& p, void* stream) {
+    return p.stream ? ovfcc::launch_stream(a, p, stream) : ovfcc::launch_fc(a, p, stream);
+}
+
+// plan_call for a call of the node on its own (fill_args's arguments, nothing set by a grouped run), through the
 // node's cache: the plan depends on the node, M, the request's overrides, the chip and the environment overrides.
 int cached_plan(const ovfcc_request* r, const ovfcc_weights* w, const ovfcc::FcDeviceArgs& a, int force,
                 ovfcc::LaunchPlan* p) {
@@ -385,7 +402,7 @@ int cached_plan(const ovfcc_request* r, const ovfcc_weights* w, const ovfcc::FcD
                 return OVFCC_OK;
             }
     }
-    int rc = ovfcc::plan_launch(a, force, r->force_split, r->ctx->n_cus, p);
+    int rc = plan_call(r, a, force, p);
     if (rc)
         return rc;
     std::lock_guard<std::mutex> lock(w->plan_mu);
@@ -505,13 +522,13 @@ int enqueue_rows(ovfcc_request* r, const ovfcc_weights* w, const void* x, void* 
             fill_args(w, static_cast<const char*>(x) + (size_t)m0 * w->desc.K * 2,
                       static_cast<char*>(y) + (size_t)m0 * out_channels(w) * (w->desc.out_type == OVFCC_F32 ? 4 : 2), rows, &a);
             ovfcc::LaunchPlan p;
-            int rc = ovfcc::plan_launch(a, OVFCC_KERNEL_DECODE, r->force_split, r->ctx->n_cus, &p);
+            int rc = plan_call(r, a, OVFCC_KERNEL_DECODE, &p);
             if (rc)
                 return rc;
             rc = split_buffers(r, p, static_scratch, &a);
             if (rc)
                 return rc;
-            int e = ovfcc::launch_fc(a, p, r->stream);
+            int e = launch_call(a, p, r->stream);
             if (e)
                 return hip_fail((hipError_t)e, "kernel launch");
             if (static_scratch && (rc = static_scratch_released(r, a)))
@@ -527,7 +544,7 @@ int enqueue_rows(ovfcc_request* r, const ovfcc_weights* w, const void* x, void* 
     rc = split_buffers(r, p, static_scratch, &a);
     if (rc)
         return rc;
-    int e = ovfcc::launch_fc(a, p, r->stream);
+    int e = launch_call(a, p, r->stream);
     if (e)
         return hip_fail((hipError_t)e, "kernel launch");
     if (static_scratch && (rc = static_scratch_released(r, a)))

@@ -164,6 +164,7 @@ struct LaunchPlan {
     int gemv_c = 0;             // ... and its k-blocks per wave (2, 4 or 8)
     bool gemv16 = false;        // decode family: its 16-row sibling with stationary activations (5 <= M <= 48)
     bool gemv16_stream = false; // decode family: the 16-row kernel that streams its activations (long K, 5 <= M <= 16)
+    bool stream = false;        // decode family: the weight-streaming kernel (launched by launch_stream, not launch_fc)
     int tiles_x = 0, tiles_y = 0;  // async prefill kernel: the tile grid; its launch is 1-D
     int full_tiles = 0;         // ... of which this many run unsplit (the rest in split_k parts each)
     unsigned grid[3] = {1, 1, 1};
@@ -190,6 +191,11 @@ int launch_plain(const FcDeviceArgs& a, const LaunchPlan& plan, void* stream);
 int launch_ragged_repack(const ovfcc_fc_desc& d, const Layout& L, const void* w, void* w_out, void* stream);
 void plan_ragged(const FcDeviceArgs& a, int n_cus, LaunchPlan* plan);
 int launch_ragged(const FcDeviceArgs& a, const LaunchPlan& plan, void* stream);
+// The weight-streaming kernel for up to 48 rows of large tiled nodes (kernel_stream.hip): whether it takes a call from
+// the kernel plan_launch chose, its decomposition, its launch.
+bool stream_preferred(const FcDeviceArgs& a, const LaunchPlan& plan);
+void plan_stream(const FcDeviceArgs& a, int n_cus, LaunchPlan* plan);
+int launch_stream(const FcDeviceArgs& a, const LaunchPlan& plan, void* stream);
 int launch_decode(const FcDeviceArgs& a, const LaunchPlan& plan, void* stream);
 int launch_batch(const FcDeviceArgs& a, const LaunchPlan& plan, void* stream);
 int launch_gemv(const FcDeviceArgs& a, const LaunchPlan& plan, void* stream);
