@@ -598,6 +598,14 @@ bool plan_routed(ovfcc_request* r, const ovfcc_weights* w0, int64_t R, int n_exp
     p.counter_count = parked ? (size_t)p.tiles_x * n : 0;
     out->cap = cap;
     out->n_slices = (int)n;
+    // few rows per expert: the weight-streaming kernel, over lower slices
+    ovfcc::LaunchPlan few;
+    if (r->force_split == 0 && ovfcc::env_int("OVFCC_PREFILL_ROWS", 0) == 0 &&
+        ovfcc::plan_stream_routed(out->args, R, n_experts, r->ctx->n_cus, &few, &cap)) {
+        p = few;
+        out->cap = cap;
+        out->n_slices = (int)((R + cap - 1) / cap + n_experts);
+    }
     return true;
 }
 
@@ -630,11 +638,14 @@ int launch_routed(ovfcc_request* r, RoutedLaunch& L, const ovfcc::RoutedHeader* 
     L.args.workspace = r->workspace;
     L.args.counters = r->counters;
     const ovfcc::BatchGroupTable none{};
-    const int e = ovfcc::launch_prefill_async_grouped(none, L.n_slices, L.args, L.plan, r->stream, d_table, d_header);
+    const int e = L.plan.stream
+                      ? ovfcc::launch_stream_grouped(d_table, L.args, L.plan, r->stream)
+                      : ovfcc::launch_prefill_async_grouped(none, L.n_slices, L.args, L.plan, r->stream, d_table, d_header);
     if (e)
         return hip_fail((hipError_t)e, "grouped kernel launch");
     ovfcc::LaunchPlan shown = L.plan;
-    shown.name = "fcc_prefill_async_grouped_w4";
+    if (!shown.stream)
+        shown.name = "fcc_prefill_async_grouped_w4";
     record(r, shown);
     return OVFCC_OK;
 }

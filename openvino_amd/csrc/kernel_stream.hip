@@ -17,6 +17,7 @@
 // partial sum of a group multiplied by its scale in f32 -- once at the end where a channel has one scale.  Split parts
 // are parked with device-scope stores and added in order by the last to arrive.
 #include <algorithm>
+#include <cmath>
 
 #include "device_common.h"
 
@@ -328,6 +329,30 @@ __global__ __launch_bounds__(512) void fcc_stream_kernel(StreamItem it, StreamSh
     stream_body<BITS, MT, ZP_TABLE, MODE>(it, sh, ws, counters);
 }
 
+// Slice blockIdx.z of the table that the routing kernel wrote: at most 16 MT rows of one expert.  Slices in use come
+// first in the table; the others have no rows.  Bound by the weights that the reached experts have: 6 rows through eight
+// experts of 4096 / 14336 (6.6 of them reached on average, 0.62 GB) take 152 us with routing and the weighted sum,
+// 4 TB/s.  The grouped prefill kernel, whose slices are 64 rows high at least, multiplies and unpacks for rows that are
+// not there and took 216.
+template <int MT, bool ZP_TABLE, int MODE>
+__global__ __launch_bounds__(512) void fcc_stream_grouped_kernel(const BatchGroupItem* __restrict__ tab, StreamShape sh,
+                                                                 float* __restrict__ ws, unsigned* __restrict__ counters,
+                                                                 const int* __restrict__ row_map, int64_t x_rows) {
+    const BatchGroupItem t = tab[blockIdx.z];
+    const int rows = __builtin_amdgcn_readfirstlane(t.M);
+    if (rows <= 0)
+        return;
+    // the same for every lane, which the compiler cannot tell (kernel_prefill_async.hip)
+    StreamItem it;
+    it.w = (const uint4_t*)uniform_ptr(t.w), it.scale = (const half_t*)uniform_ptr(t.scale);
+    it.zp = (const uint8_t*)uniform_ptr(t.zp), it.bias = (const half_t*)uniform_ptr(t.bias);
+    it.x = (const half_t*)uniform_ptr(t.x), it.y = const_cast<void*>(uniform_ptr(t.y));
+    it.row_map = row_map ? row_map + __builtin_amdgcn_readfirstlane(t.reserved) : nullptr;
+    it.M = rows, it.x_rows = row_map ? x_rows : rows;
+    const size_t at = (size_t)blockIdx.z * gridDim.x;
+    stream_body<4, MT, ZP_TABLE, MODE>(it, sh, ws + at * sh.split_k * (SR_WAVES * MT * 256), counters + at);
+}
+
 bool stream_applies(const FcDeviceArgs& a) {
     const Layout& L = a.layout;
     return L.tiled && a.M > 0 && a.M <= kDecodeMaxRows && a.M * a.K * 2 < ((int64_t)1 << 31) &&
@@ -360,14 +385,9 @@ bool stream_preferred(const FcDeviceArgs& a, const LaunchPlan& p) {
     return (a.M > 4 && L.w_bytes >= ((size_t)10 << 20)) || (L.bits == 8 && !p.x_in_lds && L.w_bytes >= ((size_t)64 << 20));
 }
 
-void plan_stream(const FcDeviceArgs& a, int n_cus, LaunchPlan* plan) {
-    const Layout& L = a.layout;
-    LaunchPlan p;
-    p.kernel = OVFCC_KERNEL_DECODE;
-    p.stream = true;
-    p.name = L.bits == 4 ? "fcc_stream_w4" : "fcc_stream_w8";
-    const int64_t groups = (L.n_tiles + SR_WAVES - 1) / SR_WAVES, stages = (L.k_blocks + 1) / 2;
-    const int mt = (int)((a.M + 15) / 16);
+// Parts along K for a launch of `groups` workgroups per part, and the stages of a part.
+static void stream_parts(const Layout& L, int64_t groups, int n_cus, int64_t* split_out, int64_t* per_out) {
+    const int64_t stages = (L.k_blocks + 1) / 2;
     // Parts along K: as many as make the launch shortest, counted in stages -- rounds of workgroups over the compute
     // units times a part's stages and two more for its start and end.  (Two workgroups fit a compute unit, but a second
     // round costs a round all the same: 8192 -> 10240 u8 at 16 rows, 80 groups, takes 17.8 us in 3 parts, 22.5 in 4.)
@@ -384,6 +404,19 @@ void plan_stream(const FcDeviceArgs& a, int n_cus, LaunchPlan* plan) {
         if (best < 0 || cost < best)
             best = cost, split = parts, per = n;
     }
+    *split_out = split, *per_out = per;
+}
+
+void plan_stream(const FcDeviceArgs& a, int n_cus, LaunchPlan* plan) {
+    const Layout& L = a.layout;
+    LaunchPlan p;
+    p.kernel = OVFCC_KERNEL_DECODE;
+    p.stream = true;
+    p.name = L.bits == 4 ? "fcc_stream_w4" : "fcc_stream_w8";
+    const int64_t groups = (L.n_tiles + SR_WAVES - 1) / SR_WAVES;
+    const int mt = (int)((a.M + 15) / 16);
+    int64_t split, per;
+    stream_parts(L, groups, n_cus, &split, &per);
     p.split_k = (int)split, p.kblocks_per_split = (int)(2 * per);
     p.grid[0] = (unsigned)groups, p.grid[1] = (unsigned)split;
     p.block = 64 * SR_WAVES;
@@ -391,6 +424,43 @@ void plan_stream(const FcDeviceArgs& a, int n_cus, LaunchPlan* plan) {
     p.workspace_bytes = split > 1 ? (size_t)groups * split * SR_WAVES * mt * 1024 : 0;
     p.counter_count = split > 1 ? (size_t)groups : 0;
     *plan = p;
+}
+
+bool plan_stream_routed(const FcDeviceArgs& a, int64_t pairs, int n_experts, int n_cus, LaunchPlan* plan, int* cap) {
+    const Layout& L = a.layout;
+    // The counts stay on the device: slices of the average bucket plus twice its square root (what random routing stays
+    // under), up to 32 rows.  Expert block of eight experts, hidden size 4096, MLP width 14336, top two, against the
+    // grouped prefill kernel: 1 row 79 / 57 us, 6 rows 216 / 152, 40 rows (slices of 32) 237 / 198, 80 rows 248 / 213;
+    // with slices of 48 rows it loses (100 rows 244 / 277).  Sixteen experts of 2048 x 2048, top four: 1 row 46 / 27,
+    // 80 rows 60 / 49.  (Nodes under 1 MiB were not measured and keep the prefill kernel.)
+    const double avg = (double)pairs / n_experts;
+    const int64_t likely = (int64_t)std::ceil(avg + 2.0 * std::sqrt(avg));
+    const int mt = (int)((likely + 15) / 16);
+    if (!L.tiled || L.bits != 4 || mt > 2 || L.w_bytes < ((size_t)1 << 20) || L.groups * 32 >= ((int64_t)1 << 31) ||
+        L.k_blocks * kTileBytes >= ((int64_t)1 << 31) || a.K * 2 * 16 * mt >= ((int64_t)1 << 31))
+        return false;
+    const int64_t slices = std::min(pairs, (pairs + 16 * mt - 1) / (16 * mt) + n_experts);
+    if (slices > 65535)
+        return false;
+    LaunchPlan p;
+    p.kernel = OVFCC_KERNEL_DECODE;
+    p.stream = true;
+    p.name = "fcc_stream_grouped_w4";
+    p.n_cus = n_cus;
+    const int64_t groups = (L.n_tiles + SR_WAVES - 1) / SR_WAVES;
+    const double reached = n_experts * (1.0 - std::pow(1.0 - 1.0 / n_experts, (double)pairs));
+    int64_t split, per;
+    stream_parts(L, groups * std::max<int64_t>(1, std::llround(reached)), n_cus, &split, &per);
+    p.split_k = (int)split, p.kblocks_per_split = (int)(2 * per);
+    p.grid[0] = (unsigned)groups, p.grid[1] = (unsigned)split, p.grid[2] = (unsigned)slices;
+    p.block = 64 * SR_WAVES;
+    p.tiles_x = (int)groups, p.tiles_y = (int)slices;
+    p.tile_m = 16 * mt, p.tile_n = 16 * SR_WAVES;
+    p.workspace_bytes = split > 1 ? (size_t)(slices * groups * split) * SR_WAVES * mt * 1024 : 0;
+    p.counter_count = split > 1 ? (size_t)(slices * groups) : 0;
+    *plan = p;
+    *cap = 16 * mt;
+    return true;
 }
 
 static StreamShape stream_shape(const FcDeviceArgs& a, const LaunchPlan& p) {
@@ -449,6 +519,31 @@ int launch_stream(const FcDeviceArgs& a, const LaunchPlan& p, void* stream) {
 #undef OVFCC_STREAM_MT
 #undef OVFCC_STREAM
     return (int)hipGetLastError();
+}
+
+template <bool ZP_TABLE, int MODE>
+static int launch_stream_grouped_mode(const BatchGroupItem* tab, const FcDeviceArgs& a, const LaunchPlan& p, hipStream_t s) {
+    const StreamShape sh = stream_shape(a, p);
+    const dim3 grid(p.grid[0], p.grid[1], p.grid[2]), block(p.block);
+    auto kern = p.tile_m == 16 ? fcc_stream_grouped_kernel<1, ZP_TABLE, MODE> : fcc_stream_grouped_kernel<2, ZP_TABLE, MODE>;
+    hipLaunchKernelGGL(kern, grid, block, 0, s, tab, sh, a.workspace, a.counters, a.row_map, a.x_rows);
+    return (int)hipGetLastError();
+}
+
+int launch_stream_grouped(const BatchGroupItem* tab, const FcDeviceArgs& a, const LaunchPlan& p, void* stream) {
+    const Layout& L = a.layout;
+    if (!tab || !p.stream || !L.tiled || L.bits != 4 || (int64_t)p.grid[0] * SR_WAVES < L.n_tiles ||
+        p.grid[1] != (unsigned)p.split_k || (int64_t)p.split_k * p.kblocks_per_split < L.k_blocks || (p.kblocks_per_split & 1) ||
+        (p.tile_m != 16 && p.tile_m != 32) || (p.split_k > 1 && !(a.workspace && a.counters)) ||
+        a.K * 2 * p.tile_m >= ((int64_t)1 << 31) ||
+        (a.row_map && (a.x_rows < 1 || a.x_rows * a.K * 2 >= ((int64_t)1 << 31))))
+        return (int)hipErrorInvalidValue;
+    hipStream_t s = static_cast<hipStream_t>(stream);
+    const int mode = L.groups == 1 ? 0 : L.groups_per_kblock;
+#define OVFCC_STREAM_MODE(G) \
+    (L.zp_table ? launch_stream_grouped_mode<true, G>(tab, a, p, s) : launch_stream_grouped_mode<false, G>(tab, a, p, s))
+    return mode == 0 ? OVFCC_STREAM_MODE(0) : mode == 1 ? OVFCC_STREAM_MODE(1) : mode == 2 ? OVFCC_STREAM_MODE(2) : OVFCC_STREAM_MODE(4);
+#undef OVFCC_STREAM_MODE
 }
 
 }  // namespace ovfcc

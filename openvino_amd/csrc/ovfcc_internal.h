@@ -283,6 +283,11 @@ int rows_cap_for(const int64_t* rows, int n, bool mid_ok);
 int launch_prefill_async_grouped(const BatchGroupTable& tab, int n_items, const FcDeviceArgs& a, const LaunchPlan& plan,
                                  void* stream, const BatchGroupItem* dev_tab = nullptr,
                                  const RoutedHeader* dev_hdr = nullptr);
+// The weight-streaming kernel over the slices of a routed launch (few rows per expert; 4-bit nodes): whether it takes
+// `pairs` rows spread over the experts (a: a node's arguments), its plan and the slice height; its launch over the
+// table in device memory, whose slices in use come first.
+bool plan_stream_routed(const FcDeviceArgs& a, int64_t pairs, int n_experts, int n_cus, LaunchPlan* plan, int* cap);
+int launch_stream_grouped(const BatchGroupItem* tab, const FcDeviceArgs& a, const LaunchPlan& plan, void* stream);
 // Routing of a mixture-of-experts layer on the device: buckets the R = M * top_k (row, selection) pairs of
 // indices [M, top_k] (device memory) by expert, ascending inside a bucket, and writes the row maps and the slice
 // table that the gather kernel and the grouped launch read -- first[slot] = row of A that bucket slot `slot`
