@@ -1309,11 +1309,13 @@ struct BlobHeader {
     uint32_t header_bytes;
     ovfcc_fc_desc desc;
     int32_t zp_const;
-    int32_t tiled;        // kBlobTiled | kBlobHasDown
+    int32_t tiled;        // kBlobTiled | kBlobHasDown | kBlobRagged
     uint64_t w_bytes, scale_bytes, zp_bytes, bias_bytes;
 };
 constexpr uint32_t kBlobVersion = 3;
-constexpr int32_t kBlobTiled = 1, kBlobHasDown = 2;  // bits of BlobHeader::tiled; HasDown: another node's blob follows
+// bits of BlobHeader::tiled; HasDown: another node's blob follows; Ragged: the weights of a node that fits no tile are in
+// operand order (blobs written before there was such an order have them as OpenVINO packs them, and no such bit)
+constexpr int32_t kBlobTiled = 1, kBlobHasDown = 2, kBlobRagged = 4;
 const char kBlobMagic[8] = {'O', 'V', 'F', 'C', 'C', 'W', 0, 0};
 
 size_t pad16(size_t n) {
@@ -1375,7 +1377,7 @@ int ovfcc_weights_export(const ovfcc_weights* w, void* blob, size_t bytes) {
     h.header_bytes = (uint32_t)sizeof(BlobHeader);
     h.desc = w->desc;
     h.zp_const = w->layout.zp_const;
-    h.tiled = (w->layout.tiled ? kBlobTiled : 0) | (w->mlp_down ? kBlobHasDown : 0);
+    h.tiled = (w->layout.tiled ? kBlobTiled : 0) | (w->layout.ragged ? kBlobRagged : 0) | (w->mlp_down ? kBlobHasDown : 0);
     h.w_bytes = sz[0], h.scale_bytes = sz[1], h.zp_bytes = sz[2], h.bias_bytes = sz[3];
     char* at = static_cast<char*>(blob);
     std::memset(at, 0, need);
@@ -1406,10 +1408,14 @@ int ovfcc_weights_import(ovfcc_ctx* ctx, const void* blob, size_t bytes, ovfcc_w
     ovfcc::Layout L = ovfcc::make_layout(h.desc);
     uint64_t sz[4];
     device_sizes(h.desc, L, sz);
+    const bool as_given = L.ragged && !(h.tiled & kBlobRagged);
+    if (as_given)
+        sz[0] = L.bits == 4 ? (uint64_t)(h.desc.N * h.desc.K + 1) / 2 : (uint64_t)(h.desc.N * h.desc.K);
     // a scalar zero-point lives in zp_const; everything else must be exactly what the descriptor implies
     const int zp_lo = L.zp_offset, zp_hi = L.zp_offset + 255;
     const size_t need = pad16(sizeof(BlobHeader)) + pad16(sz[0]) + pad16(sz[1]) + pad16(sz[2]) + pad16(sz[3]);
-    if ((h.tiled & ~(kBlobTiled | kBlobHasDown)) != 0 || ((h.tiled & kBlobTiled) != 0) != L.tiled || h.w_bytes != sz[0] || h.scale_bytes != sz[1] || h.zp_bytes != sz[2] ||
+    if ((h.tiled & ~(kBlobTiled | kBlobHasDown | kBlobRagged)) != 0 || ((h.tiled & kBlobTiled) != 0) != L.tiled ||
+        ((h.tiled & kBlobRagged) != 0 && !L.ragged) || h.w_bytes != sz[0] || h.scale_bytes != sz[1] || h.zp_bytes != sz[2] ||
         h.bias_bytes != sz[3] || h.zp_const < zp_lo || h.zp_const > zp_hi ||
         bytes < need)
         return fail(OVFCC_EINVAL, "blob sizes do not match its descriptor");
@@ -1422,7 +1428,9 @@ int ovfcc_weights_import(ovfcc_ctx* ctx, const void* blob, size_t bytes, ovfcc_w
     const char* at = static_cast<const char*>(blob) + pad16(sizeof(BlobHeader));
     void** dst[4] = {&W->d_w, &W->d_scale, &W->d_zp, &W->d_bias};
     for (int i = 0; i < 4 && !rc; ++i) {
-        if (sz[i]) {
+        if (i == 0 && as_given) {
+            rc = upload_ragged(W, at, sz[0]);
+        } else if (sz[i]) {
             hipError_t e = hipMalloc(dst[i], sz[i]);
             if (e == hipSuccess)
                 e = hipMemcpy(*dst[i], at, sz[i], hipMemcpyHostToDevice);

@@ -75,3 +75,35 @@ def test_rows_keep_to_themselves(dev, req):
             assert np.array_equal(clean[0::2], dirty[0::2]) and not np.isfinite(dirty[1::2]).any()
         finally:
             w.close()
+
+
+@pytest.mark.parametrize("wt,zt,N,K", [("i8", "u8", 128, 256),    # as many bytes in operand order as in OpenVINO's
+                                       ("u8", "u8", 67, 1161), ("i4", "none", 65, 1160)])
+def test_blob_with_the_weights_as_given(dev, req, wt, zt, N, K):
+    """A blob written before these nodes had an order of their own holds the weights as OpenVINO packs them and no bit
+    that says otherwise: it gives the same node, as does a blob in operand order."""
+    c = datagen.make_case(2250 + N, 20, K, N, wt, K, zt, with_bias=True)
+    w = fc.CompressedWeights.from_case(dev, c, output_type="f32")
+    blob = np.asarray(w.export_blob()).copy()
+    head = int(blob[12:16].view(np.uint32)[0])
+    flags, w_at = blob[head - 36:head - 32].view(np.int32), blob[head - 32:head - 24].view(np.uint64)
+    assert flags[0] == 4
+    pad = lambda n: (n + 15) // 16 * 16
+    rest = blob[pad(head) + pad(int(w_at[0])):]
+    given = np.ascontiguousarray(c.w).view(np.uint8).reshape(-1)
+    start = blob[:pad(head)].copy()
+    start[head - 36:head - 32].view(np.int32)[0] = 0
+    start[head - 32:head - 24].view(np.uint64)[0] = given.size
+    old = np.concatenate([start, given, np.zeros(pad(given.size) - given.size, np.uint8), rest])
+    nodes = [w]
+    try:
+        y = req.infer(w, c.x)
+        for b in (blob, old):
+            nodes.append(fc.CompressedWeights.import_blob(dev, b))
+            assert np.array_equal(req.infer(nodes[-1], c.x), y)
+        blob[head - 36:head - 32].view(np.int32)[0] = 1    # tiled: not what the descriptor implies
+        with pytest.raises(fc.OvfccError):
+            fc.CompressedWeights.import_blob(dev, blob)
+    finally:
+        for n in nodes:
+            n.close()
