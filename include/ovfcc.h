@@ -217,9 +217,10 @@ int ovfcc_weights_is_tiled(const ovfcc_weights* w);
  * template plugin's pair: src/plugins/template/src/compiled_model.cpp:173-192, plugin.cpp:230-311) store per node so
  * that a cached model skips the repack (ov::cache_dir, src/inference/src/dev/core_impl.cpp:858-897).
  * ovfcc_weights_export_size gives the blob's size; ovfcc_weights_export fills a host buffer of at least that size;
- * ovfcc_weights_import rebuilds the node on ctx's device.  A blob is valid for this library version only: import
- * checks magic, version, descriptor and every size against what the descriptor implies and fails with
- * OVFCC_EINVAL otherwise. */
+ * ovfcc_weights_import rebuilds the node on ctx's device.  Import reads blobs of this
+ * layout version and of the one before it (which held the weights of nodes that fit no tile as OpenVINO packs them);
+ * it checks magic, version, descriptor and every size against what these imply and fails with OVFCC_EINVAL
+ * otherwise. */
 int ovfcc_weights_export_size(const ovfcc_weights* w, size_t* bytes);
 int ovfcc_weights_export(const ovfcc_weights* w, void* blob, size_t bytes);
 int ovfcc_weights_import(ovfcc_ctx* ctx, const void* blob, size_t bytes, ovfcc_weights** out);

@@ -1312,9 +1312,11 @@ struct BlobHeader {
     int32_t tiled;        // kBlobTiled | kBlobHasDown | kBlobRagged
     uint64_t w_bytes, scale_bytes, zp_bytes, bias_bytes;
 };
-constexpr uint32_t kBlobVersion = 3;
-// bits of BlobHeader::tiled; HasDown: another node's blob follows; Ragged: the weights of a node that fits no tile are in
-// operand order (blobs written before there was such an order have them as OpenVINO packs them, and no such bit)
+// Version 2 differs in one thing: it knows no operand order of nodes that fit no tile, whose weights it holds as OpenVINO
+// packs them.  Both versions are read.
+constexpr uint32_t kBlobVersion = 3, kBlobVersionAsGiven = 2;
+// bits of BlobHeader::tiled; HasDown: another node's blob follows; Ragged: the weights are in operand order (in version 3
+// every node with Layout::ragged, and no other)
 constexpr int32_t kBlobTiled = 1, kBlobHasDown = 2, kBlobRagged = 4;
 const char kBlobMagic[8] = {'O', 'V', 'F', 'C', 'C', 'W', 0, 0};
 
@@ -1400,7 +1402,8 @@ int ovfcc_weights_import(ovfcc_ctx* ctx, const void* blob, size_t bytes, ovfcc_w
         return fail(OVFCC_EINVAL, "blob is shorter than its header");
     BlobHeader h;
     std::memcpy(&h, blob, sizeof(h));
-    if (std::memcmp(h.magic, kBlobMagic, 8) != 0 || h.version != kBlobVersion || h.header_bytes != sizeof(BlobHeader))
+    if (std::memcmp(h.magic, kBlobMagic, 8) != 0 || (h.version != kBlobVersion && h.version != kBlobVersionAsGiven) ||
+        h.header_bytes != sizeof(BlobHeader))
         return fail(OVFCC_EINVAL, "not a weight blob of this library version");
     int rc = ovfcc::validate_desc(&h.desc);
     if (rc)
@@ -1408,14 +1411,14 @@ int ovfcc_weights_import(ovfcc_ctx* ctx, const void* blob, size_t bytes, ovfcc_w
     ovfcc::Layout L = ovfcc::make_layout(h.desc);
     uint64_t sz[4];
     device_sizes(h.desc, L, sz);
-    const bool as_given = L.ragged && !(h.tiled & kBlobRagged);
+    const bool as_given = L.ragged && h.version == kBlobVersionAsGiven;
     if (as_given)
         sz[0] = L.bits == 4 ? (uint64_t)(h.desc.N * h.desc.K + 1) / 2 : (uint64_t)(h.desc.N * h.desc.K);
     // a scalar zero-point lives in zp_const; everything else must be exactly what the descriptor implies
     const int zp_lo = L.zp_offset, zp_hi = L.zp_offset + 255;
     const size_t need = pad16(sizeof(BlobHeader)) + pad16(sz[0]) + pad16(sz[1]) + pad16(sz[2]) + pad16(sz[3]);
     if ((h.tiled & ~(kBlobTiled | kBlobHasDown | kBlobRagged)) != 0 || ((h.tiled & kBlobTiled) != 0) != L.tiled ||
-        ((h.tiled & kBlobRagged) != 0 && !L.ragged) || h.w_bytes != sz[0] || h.scale_bytes != sz[1] || h.zp_bytes != sz[2] ||
+        ((h.tiled & kBlobRagged) != 0) != (L.ragged && !as_given) || h.w_bytes != sz[0] || h.scale_bytes != sz[1] || h.zp_bytes != sz[2] ||
         h.bias_bytes != sz[3] || h.zp_const < zp_lo || h.zp_const > zp_hi ||
         bytes < need)
         return fail(OVFCC_EINVAL, "blob sizes do not match its descriptor");

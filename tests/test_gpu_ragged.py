@@ -77,33 +77,76 @@ def test_rows_keep_to_themselves(dev, req):
             w.close()
 
 
+def blob_fields(blob, at=0):
+    """(version, flags, bytes of the weights) of the header that begins at byte `at`, as views into the blob."""
+    head = int(blob[at + 12:at + 16].view(np.uint32)[0])
+    return (blob[at + 8:at + 12].view(np.uint32), blob[at + head - 36:at + head - 32].view(np.int32),
+            blob[at + head - 32:at + head - 24].view(np.uint64))
+
+
+def pad16(n):
+    return (n + 15) // 16 * 16
+
+
+def version_2(blob, given):
+    """The blob of a node that fits no tile as version 2 wrote it: the weights as given, no flag."""
+    head = int(blob[12:16].view(np.uint32)[0])
+    old = blob[:pad16(head)].copy()
+    rest = blob[pad16(head) + pad16(int(blob_fields(blob)[2][0])):]
+    version, flags, w_bytes = blob_fields(old)
+    version[0], flags[0], w_bytes[0] = 2, 0, given.size
+    return np.concatenate([old, given, np.zeros(pad16(given.size) - given.size, np.uint8), rest])
+
+
 @pytest.mark.parametrize("wt,zt,N,K", [("i8", "u8", 128, 256),    # as many bytes in operand order as in OpenVINO's
-                                       ("u8", "u8", 67, 1161), ("i4", "none", 65, 1160)])
+                                       ("u8", "u8", 67, 1161), ("i4", "none", 65, 1160), ("u4", "u4", 33, 651)])
 def test_blob_with_the_weights_as_given(dev, req, wt, zt, N, K):
-    """A blob written before these nodes had an order of their own holds the weights as OpenVINO packs them and no bit
-    that says otherwise: it gives the same node, as does a blob in operand order."""
+    """A blob of version 2, written before these nodes had an order of their own, holds the weights as OpenVINO packs
+    them: it gives the same node, as does a blob of version 3 in operand order.  Each version's flag is held to."""
     c = datagen.make_case(2250 + N, 20, K, N, wt, K, zt, with_bias=True)
     w = fc.CompressedWeights.from_case(dev, c, output_type="f32")
     blob = np.asarray(w.export_blob()).copy()
-    head = int(blob[12:16].view(np.uint32)[0])
-    flags, w_at = blob[head - 36:head - 32].view(np.int32), blob[head - 32:head - 24].view(np.uint64)
-    assert flags[0] == 4
-    pad = lambda n: (n + 15) // 16 * 16
-    rest = blob[pad(head) + pad(int(w_at[0])):]
-    given = np.ascontiguousarray(c.w).view(np.uint8).reshape(-1)
-    start = blob[:pad(head)].copy()
-    start[head - 36:head - 32].view(np.int32)[0] = 0
-    start[head - 32:head - 24].view(np.uint64)[0] = given.size
-    old = np.concatenate([start, given, np.zeros(pad(given.size) - given.size, np.uint8), rest])
+    version, flags, _ = blob_fields(blob)
+    assert version[0] == 3 and flags[0] == 4
+    old = version_2(blob, np.ascontiguousarray(c.w).view(np.uint8).reshape(-1))
     nodes = [w]
     try:
         y = req.infer(w, c.x)
         for b in (blob, old):
             nodes.append(fc.CompressedWeights.import_blob(dev, b))
             assert np.array_equal(req.infer(nodes[-1], c.x), y)
-        blob[head - 36:head - 32].view(np.int32)[0] = 1    # tiled: not what the descriptor implies
+        assert np.array_equal(np.asarray(nodes[-1].export_blob()), blob)
+        blob_fields(old)[1][0] = 4          # version 2 with the flag of version 3
         with pytest.raises(fc.OvfccError):
-            fc.CompressedWeights.import_blob(dev, blob)
+            fc.CompressedWeights.import_blob(dev, old)
+        # version 3 without it (operand order, as one would write before there was a flag), tiled, or as version 1 or 4
+        for v, f in ((3, 0), (3, 1), (3, 5), (1, 4), (4, 4)):
+            version[0], flags[0] = v, f
+            with pytest.raises(fc.OvfccError):
+                fc.CompressedWeights.import_blob(dev, blob)
+    finally:
+        for n in nodes:
+            n.close()
+
+
+def test_version_2_blobs_of_other_nodes(dev, req):
+    """Tiled nodes, MLP nodes and nodes with several groups per channel have the same blob in both versions."""
+    plain = datagen.make_case(2260, 6, 200, 40, "u4", 50, "u4")
+    tiled = datagen.make_case(2261, 6, 512, 256, "i4", 128, "none", with_bias=True)
+    gate_up = fc.CompressedWeights.from_case(dev, datagen.make_case(2262, 6, 512, 512, "u4", 128, "u4"), glu="swish")
+    down = fc.CompressedWeights.from_case(dev, datagen.make_case(2263, 6, 256, 128, "u4", 128, "u4"))
+    nodes = [gate_up, down, fc.CompressedWeights.from_case(dev, plain), fc.CompressedWeights.from_case(dev, tiled)]
+    try:
+        nodes.append(fc.CompressedWeights.mlp(gate_up, down))
+        for w in list(nodes[2:]):
+            x = np.random.default_rng(2264).standard_normal((6, w.K)).astype(np.float16)
+            blob = np.asarray(w.export_blob()).copy()
+            magic, at = blob[:8].tobytes(), 0
+            while at >= 0:                  # an MLP node: its down projection's blob as well
+                blob_fields(blob, at)[0][0] = 2
+                at = blob.tobytes().find(magic, at + 8)
+            nodes.append(fc.CompressedWeights.import_blob(dev, blob))
+            assert np.array_equal(req.infer(nodes[-1], x), req.infer(w, x))
     finally:
         for n in nodes:
             n.close()
