@@ -372,14 +372,14 @@ int enqueue(ovfcc_request* r, const ovfcc_weights* w, const void* x, void* y, in
 }
 
 // The plan of one launch: plan_launch's, or the weight-streaming kernel's where that takes the call and nothing forces
-// another.
+// another (OVFCC_STREAM, or an override about the kernel that plan_launch chose).
 int plan_call(const ovfcc_request* r, const ovfcc::FcDeviceArgs& a, int force, ovfcc::LaunchPlan* p) {
     int rc = ovfcc::plan_launch(a, force, r->force_split, r->ctx->n_cus, p);
-    if (rc)
+    if (rc || (force != OVFCC_KERNEL_AUTO && force != OVFCC_KERNEL_DECODE) || r->force_split != 0 ||
+        p->kernel != OVFCC_KERNEL_DECODE)
         return rc;
-    if ((force == OVFCC_KERNEL_AUTO || force == OVFCC_KERNEL_DECODE) && r->force_split == 0 &&
-        ovfcc::env_int("OVFCC_DECODE_BATCH", -1) < 0 && ovfcc::env_int("OVFCC_GEMV16_SPLIT", 0) == 0 &&
-        ovfcc::env_int("OVFCC_GEMV16_STREAM", -1) < 0 && ovfcc::stream_preferred(a, *p))
+    const int wish = ovfcc::env_int("OVFCC_STREAM", -1);
+    if (wish == 1 ? ovfcc::stream_applies(a) : wish != 0 && !ovfcc::decode_overridden() && ovfcc::stream_preferred(a, *p))
         ovfcc::plan_stream(a, r->ctx->n_cus, p);
     return OVFCC_OK;
 }
@@ -600,7 +600,7 @@ bool plan_routed(ovfcc_request* r, const ovfcc_weights* w0, int64_t R, int n_exp
     out->n_slices = (int)n;
     // few rows per expert: the weight-streaming kernel, over lower slices
     ovfcc::LaunchPlan few;
-    if (r->force_split == 0 && ovfcc::env_int("OVFCC_PREFILL_ROWS", 0) == 0 &&
+    if (r->force_split == 0 && ovfcc::env_int("OVFCC_PREFILL_ROWS", 0) == 0 && ovfcc::env_int("OVFCC_STREAM", -1) != 0 &&
         ovfcc::plan_stream_routed(out->args, R, n_experts, r->ctx->n_cus, &few, &cap)) {
         p = few;
         out->cap = cap;

@@ -181,6 +181,8 @@ int plan_launch(const FcDeviceArgs& a, int force_kernel, int force_split, int n_
 // OVFCC_* overrides of the process environment: cached at the first use, re-read by env_reload only.
 // env_generation changes with every (re)read; plans cached under an older generation are stale.
 int env_int(const char* name, int fallback);
+// whether an override that chooses or shapes one of the older decode kernels is set
+bool decode_overridden();
 void env_reload();
 unsigned env_generation();
 // Enqueues on `stream` (a hipStream_t passed as void*); returns a HIP error code (0 = success).
@@ -191,8 +193,9 @@ int launch_plain(const FcDeviceArgs& a, const LaunchPlan& plan, void* stream);
 int launch_ragged_repack(const ovfcc_fc_desc& d, const Layout& L, const void* w, void* w_out, void* stream);
 void plan_ragged(const FcDeviceArgs& a, int n_cus, LaunchPlan* plan);
 int launch_ragged(const FcDeviceArgs& a, const LaunchPlan& plan, void* stream);
-// The weight-streaming kernel for up to 48 rows of large tiled nodes (kernel_stream.hip): whether it takes a call from
-// the kernel plan_launch chose, its decomposition, its launch.
+// The weight-streaming kernel for up to 48 rows of large tiled nodes (kernel_stream.hip): whether it can run a call,
+// whether it takes it from the kernel plan_launch chose, its decomposition, its launch.
+bool stream_applies(const FcDeviceArgs& a);
 bool stream_preferred(const FcDeviceArgs& a, const LaunchPlan& plan);
 void plan_stream(const FcDeviceArgs& a, int n_cus, LaunchPlan* plan);
 int launch_stream(const FcDeviceArgs& a, const LaunchPlan& plan, void* stream);

@@ -23,6 +23,8 @@ namespace ovfcc {
 //            OVFCC_GEMV16_GRID = n (its workgroups per row tile), OVFCC_GEMV16_SPLIT = 1 | 2 | 4 | 8 (parts it cuts K in),
 //            OVFCC_GEMV16_STREAM = 0 | 1 (the 16-row kernel that streams its activations, 5-16 rows),
 //            OVFCC_GEMV16_STREAM_TILES = 1 | 2 | 4 (its channel tiles per workgroup),
+//            OVFCC_STREAM = 0 | 1 (the weight-streaming kernel nowhere, wherever it can run; without it any of the
+//            overrides above keeps the kernel that they are about),
 //            OVFCC_PREFILL_{DIRECT, ASYNC, WIDE, BIG, TAIL} = 0 | 1, OVFCC_PREFILL_ROWS = 64 | 128,
 //            OVFCC_MOE_HOST_ROUTING = 1, OVFCC_MLP_FUSED = 1 (an MLP node of up to four rows as one launch instead of two),
 //            OVFCC_MLP_GRID = n (its workgroups), OVFCC_MLP_SPIN_LIMIT = n (polls after which that launch's wait for its workgroups gives up; tests);
@@ -30,28 +32,35 @@ namespace ovfcc {
 namespace {
 struct EnvEntry {
     const char* name;
+    bool decode;  // chooses or shapes one of the older decode kernels
     std::atomic<int> set{0};
     std::atomic<int> value{0};
-    explicit EnvEntry(const char* n) : name(n) {}
+    explicit EnvEntry(const char* n, bool d = false) : name(n), decode(d) {}
 };
-EnvEntry g_env[] = {EnvEntry("OVFCC_DECODE_WAVES"),   EnvEntry("OVFCC_DECODE_RT"),      EnvEntry("OVFCC_DECODE_XLDS"),
-                    EnvEntry("OVFCC_DECODE_BATCH"),   EnvEntry("OVFCC_GEMV"),           EnvEntry("OVFCC_GEMV_C"),
-                    EnvEntry("OVFCC_GEMV16"),         EnvEntry("OVFCC_GEMV16_GRID"),    EnvEntry("OVFCC_GEMV16_SPLIT"),
-                    EnvEntry("OVFCC_GEMV16_STREAM"),  EnvEntry("OVFCC_GEMV16_STREAM_TILES"),
+EnvEntry g_env[] = {EnvEntry("OVFCC_DECODE_WAVES", true),   EnvEntry("OVFCC_DECODE_RT", true),
+                    EnvEntry("OVFCC_DECODE_XLDS", true),    EnvEntry("OVFCC_DECODE_BATCH", true),
+                    EnvEntry("OVFCC_GEMV", true),           EnvEntry("OVFCC_GEMV_C", true),
+                    EnvEntry("OVFCC_GEMV16", true),         EnvEntry("OVFCC_GEMV16_GRID", true),
+                    EnvEntry("OVFCC_GEMV16_SPLIT", true),   EnvEntry("OVFCC_GEMV16_STREAM", true),
+                    EnvEntry("OVFCC_GEMV16_STREAM_TILES", true), EnvEntry("OVFCC_STREAM"),
                     EnvEntry("OVFCC_PREFILL_DIRECT"), EnvEntry("OVFCC_PREFILL_ASYNC"),  EnvEntry("OVFCC_PREFILL_WIDE"),
                     EnvEntry("OVFCC_PREFILL_BIG"),    EnvEntry("OVFCC_PREFILL_TAIL"),   EnvEntry("OVFCC_PREFILL_ROWS"),
                     EnvEntry("OVFCC_MOE_HOST_ROUTING"), EnvEntry("OVFCC_MLP_FUSED"),      EnvEntry("OVFCC_MLP_SPIN_LIMIT"),
                     EnvEntry("OVFCC_MLP_GRID"),
                     EnvEntry("OVFCC_VERBOSE")};
+std::atomic<bool> g_decode_overridden{false};
 std::atomic<unsigned> g_env_generation{0};
 std::once_flag g_env_once;
 
 void env_read_all() {
+    bool decode = false;
     for (EnvEntry& e : g_env) {
         const char* v = std::getenv(e.name);
         e.value.store(v ? std::atoi(v) : 0, std::memory_order_relaxed);
         e.set.store(v ? 1 : 0, std::memory_order_release);
+        decode |= v && e.decode;
     }
+    g_decode_overridden.store(decode, std::memory_order_release);
     g_env_generation.fetch_add(1, std::memory_order_acq_rel);
 }
 }  // namespace
@@ -64,6 +73,11 @@ void env_reload() {
 unsigned env_generation() {
     std::call_once(g_env_once, env_read_all);
     return g_env_generation.load(std::memory_order_acquire);
+}
+
+bool decode_overridden() {
+    std::call_once(g_env_once, env_read_all);
+    return g_decode_overridden.load(std::memory_order_acquire);
 }
 
 int env_int(const char* name, int fallback) {

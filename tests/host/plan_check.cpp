@@ -179,6 +179,18 @@ static void check_env_cache() {
     unsetenv("OVFCC_PREFILL_ROWS");
     ovfcc::env_reload();
     CHECK(ovfcc::env_int("OVFCC_PREFILL_ROWS", 7) == 7, "and its removal");
+    // overrides of the older decode kernels are told from the others
+    for (const char* name : {"OVFCC_STREAM", "OVFCC_PREFILL_BIG", "OVFCC_VERBOSE", "OVFCC_DECODE_WAVES", "OVFCC_DECODE_RT",
+                             "OVFCC_DECODE_XLDS", "OVFCC_DECODE_BATCH", "OVFCC_GEMV", "OVFCC_GEMV16", "OVFCC_GEMV16_GRID",
+                             "OVFCC_GEMV16_SPLIT", "OVFCC_GEMV16_STREAM", "OVFCC_GEMV16_STREAM_TILES"}) {
+        const bool decode = std::strstr(name, "DECODE") || std::strstr(name, "GEMV");
+        setenv(name, "0", 1);
+        ovfcc::env_reload();
+        CHECK(ovfcc::decode_overridden() == decode, "%s", name);
+        unsetenv(name);
+        ovfcc::env_reload();
+        CHECK(!ovfcc::decode_overridden(), "%s removed", name);
+    }
 }
 
 int main() {

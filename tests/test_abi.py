@@ -52,6 +52,13 @@ def test_version_and_error_string():
     assert b"group_size" in L.ovfcc_last_error()
 
 
+def test_every_override_is_looked_at():
+    """The Python mirror has the library read its overrides again when one of them changes: it looks at the names of
+    csrc/plan.cpp's table."""
+    text = open(os.path.join(ROOT, "openvino_amd", "csrc", "plan.cpp")).read()
+    assert sorted(re.findall(r'EnvEntry\("(\w+)"', text)) == sorted(_lib.ENV_NAMES)
+
+
 @pytest.mark.parametrize("mutate,code", [
     (dict(N=0), _lib.EINVAL), (dict(K=-4), _lib.EINVAL), (dict(group_size=0), _lib.EINVAL),
     (dict(group_size=96), _lib.EINVAL), (dict(w_type=_lib.F16), _lib.EUNSUPPORTED),

@@ -78,3 +78,27 @@ def test_gated_linear_unit(oracle, dev, req, wt, zt, N, K, G, kind, second):
             check_parity(oracle, y, ref[:M], K, f"{req.last_kernel()}", output_rounding_slack=True, limit_scale=amp)
     finally:
         w.close()
+
+
+@pytest.mark.parametrize("env,M,name,block", [
+    ({}, 32, "fcc_stream_w4", 512),
+    ({"OVFCC_STREAM": "0"}, 32, "fcc_batch_w4", 512),
+    ({"OVFCC_GEMV16": "0"}, 32, "fcc_batch_w4", 512),           # any override about an older kernel keeps it
+    ({"OVFCC_DECODE_WAVES": "4"}, 32, "fcc_batch_w4", 256),
+    ({"OVFCC_DECODE_RT": "2"}, 32, "fcc_batch_w4", 512),
+    ({"OVFCC_DECODE_XLDS": "0"}, 3, "fcc_decode_w4", None),
+    ({"OVFCC_STREAM": "1"}, 3, "fcc_stream_w4", 512),
+    ({"OVFCC_STREAM": "1", "OVFCC_GEMV16": "0"}, 32, "fcc_stream_w4", 512),
+])
+def test_overrides(oracle, dev, req, monkeypatch, env, M, name, block):
+    c = datagen.make_case(2450, M, 1024, 1024, "u4", 64, "u4")
+    w = fc.CompressedWeights.from_case(dev, c)
+    try:
+        for k, v in env.items():
+            monkeypatch.setenv(k, v)
+        print(f"overrides {env} M={M}", flush=True)
+        y, info = req.infer(w, c.x), req.last_kernel()
+        assert info["name"] == name and block in (None, info["block"]), info
+        check_parity(oracle, y, oracle_y(oracle, c), 1024, f"{info}", output_rounding_slack=True)
+    finally:
+        w.close()
