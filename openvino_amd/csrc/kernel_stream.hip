@@ -77,7 +77,10 @@ __device__ __forceinline__ void stream_body(const StreamItem& it, const StreamSh
         const_cast<uint8_t*>(ZP_TABLE ? it.zp + t0 * sh.ng * 16 : it.zp), 0, ZP_TABLE && mine ? sh.ng * 16 : 0, kRsrcFlags);
     const __amdgpu_buffer_rsrc_t rx = __builtin_amdgcn_make_buffer_rsrc(
         const_cast<half_t*>(it.x), 0, (int)(it.x_rows * sh.K * 2), kRsrcFlags);
-    const unsigned g_mul = sh.kb_per_group == 1 ? 0u : (unsigned)((0x100000000ull + sh.kb_per_group - 1) / sh.kb_per_group);
+    // kb / kb_per_group as the high word of 2 kb ceil(2^31 / kb_per_group): exact for kb kb_per_group < 2^31 (a node has
+    // fewer than 2^16 k-blocks, a group at most half of them), and without a branch -- two loads of one register on two
+    // sides of a branch made every stage wait for all weights in flight
+    const unsigned g_mul = (unsigned)((0x80000000ull + sh.kb_per_group - 1) / sh.kb_per_group);
 
     // ---- activations: chunk i of the thread is eight inputs of row 16 i + (tid >> 5) ----
     unsigned x_ofs[MT];
@@ -132,7 +135,7 @@ __device__ __forceinline__ void stream_body(const StreamItem& it, const StreamSh
 #pragma unroll
             for (int b = 0; b < 2; ++b) {
                 const unsigned kb = (unsigned)(kb_begin + 2 * s + b);
-                const unsigned g = sh.kb_per_group == 1 ? kb : __umulhi(kb, g_mul);
+                const unsigned g = __umulhi(2 * kb, g_mul);
                 const unsigned idx = MODE == 1 ? g * 16u + col : (kb * 16u + col) * GPB;
                 if constexpr (GPB == 1)
                     q.scale[b][0] = __builtin_amdgcn_raw_buffer_load_b16(rs, (idx * 2u) | past, 0, 0);
