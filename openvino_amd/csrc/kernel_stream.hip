@@ -326,8 +326,10 @@ __device__ __forceinline__ void stream_body(const StreamItem& it, const StreamSh
 
 }  // namespace
 
+// Two workgroups share a compute unit: four waves per SIMD, 128 registers each (48 rows of nodes with a zero-point table
+// would take 130).
 template <int BITS, int MT, bool ZP_TABLE, int MODE>
-__global__ __launch_bounds__(512) void fcc_stream_kernel(StreamItem it, StreamShape sh, float* __restrict__ ws,
+__global__ __launch_bounds__(512, 4) void fcc_stream_kernel(StreamItem it, StreamShape sh, float* __restrict__ ws,
                                                          unsigned* __restrict__ counters) {
     stream_body<BITS, MT, ZP_TABLE, MODE>(it, sh, ws, counters);
 }
