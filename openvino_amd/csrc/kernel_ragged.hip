@@ -33,8 +33,7 @@ namespace ovfcc {
 
 namespace {
 
-constexpr int RG_BM = 64, RG_BN = 64;
-constexpr int RG_PITCH = kBlockK + 8;  // halves per staged row: 16 bytes of padding spread the rows over the banks
+constexpr int RG_BM = kRaggedTile, RG_BN = kRaggedTile, RG_PITCH = kRaggedPitch;
 constexpr int RG_STAGE_HALVES = RG_BM * RG_PITCH;
 
 template <class T>
@@ -173,9 +172,6 @@ __device__ __forceinline__ void finish4(const RaggedNode& a, int m, int n, float
 }  // namespace
 
 // grid = (ceil(N / 16), ceil(M / (16 MT))), block = 64 waves, dynamic LDS = waves * ragged_wave_lds(MT).
-constexpr int ragged_wave_lds(int mt) {
-    return mt * 16 * RG_PITCH * 2;
-}
 template <int BITS, int MT>
 __global__ __launch_bounds__(1024) void fcc_ragged_rows_kernel(RaggedNode a, int kb_total) {
     constexpr int WD = BITS / 4;            // dwords of a lane's eight weights
@@ -478,42 +474,6 @@ int launch_ragged_repack(const ovfcc_fc_desc& d, const Layout& L, const void* w,
     hipLaunchKernelGGL(fcc_ragged_repack_kernel, dim3((unsigned)groups), dim3(256), 0, static_cast<hipStream_t>(stream),
                        (const uint8_t*)w, (uint8_t*)w_out, (int)d.N, (int)d.K, units, (int)(L.k_blocks * 4), L.bits, flip);
     return (int)hipGetLastError();
-}
-
-void plan_ragged(const FcDeviceArgs& a, int n_cus, LaunchPlan* plan) {
-    LaunchPlan p;
-    p.kernel = OVFCC_KERNEL_PLAIN;
-    p.name = "fcc_plain";
-    const int64_t kb = a.layout.k_blocks;
-    // The rows kernel up to 16 rows, and up to the row count at which its workgroups (32 rows each) still fit the chip
-    // in one round: N = 1000, K = 1160 at 128 rows (252 workgroups) 6.0 us against 8.8 for the tile kernel, at 192 rows
-    // (378) 10.3 against 8.8; N = 2000 at 64 rows 5.8 against 8.7, at 96 rows 10.1 against 8.9; N = 4300 at 32 rows (269)
-    // 10.0 against 8.9.
-    const int mt = a.M <= 16 ? 1 : 2;
-    if (a.M <= 16 || (a.N + 15) / 16 * ((a.M + 31) / 32) <= n_cus) {
-        const int64_t waves = kb < 16 ? kb : 16;
-        p.grid[0] = (unsigned)((a.N + 15) / 16), p.grid[1] = (unsigned)((a.M + 16 * mt - 1) / (16 * mt));
-        p.block = (unsigned)(64 * waves);
-        p.tile_m = 16 * mt, p.tile_n = 16;
-        p.dynamic_lds = (unsigned)(waves * ragged_wave_lds(mt));
-    } else {
-        p.tiles_x = (int)((a.N + RG_BN - 1) / RG_BN), p.tiles_y = (int)((a.M + RG_BM - 1) / RG_BM);
-        // three workgroups fit a compute unit: K is split until the launch has about that many, four k-blocks at least
-        // to each (1160 -> 1160 at 577 rows, 190 tiles, two parts)
-        const int64_t tiles = (int64_t)p.tiles_x * p.tiles_y;
-        int64_t split = 1;
-        while (split < 8 && tiles * split * 2 <= 3 * (int64_t)n_cus && kb / (split * 2) >= 4)
-            split *= 2;
-        const int64_t per = (kb + split - 1) / split;
-        split = (kb + per - 1) / per;
-        p.split_k = (int)split, p.kblocks_per_split = (int)per;
-        p.grid[0] = (unsigned)((tiles + 7) / 8 * 8 * split);
-        p.block = 256;
-        p.tile_m = RG_BM, p.tile_n = RG_BN;
-        p.workspace_bytes = split > 1 ? (size_t)tiles * split * RG_BM * RG_BN * sizeof(float) : 0;
-        p.counter_count = split > 1 ? (size_t)tiles : 0;
-    }
-    *plan = p;
 }
 
 int launch_ragged(const FcDeviceArgs& a, const LaunchPlan& p, void* stream) {

@@ -16,16 +16,13 @@
 // Arithmetic as in the small-batch kernel: exact halves q - zp, v_mfma_f32_16x16x32_f16 with A = activations, the f32
 // partial sum of a group multiplied by its scale in f32 -- once at the end where a channel has one scale.  Split parts
 // are parked with device-scope stores and added in order by the last to arrive.
-#include <algorithm>
-#include <cmath>
-
 #include "device_common.h"
 
 namespace ovfcc {
 
 namespace {
 
-constexpr int SR_WAVES = 8;
+constexpr int SR_WAVES = kStreamWaves;
 constexpr int SR_PITCH = 2 * kBlockK + 8;  // halves per staged row; 16 bytes of padding spread the rows over the banks
 
 // What a workgroup multiplies: one node, or one slice of a grouped launch.
@@ -356,116 +353,6 @@ __global__ __launch_bounds__(512) void fcc_stream_grouped_kernel(const BatchGrou
     it.M = rows, it.x_rows = row_map ? x_rows : rows;
     const size_t at = (size_t)blockIdx.z * gridDim.x;
     stream_body<4, MT, ZP_TABLE, MODE>(it, sh, ws + at * sh.split_k * (SR_WAVES * MT * 256), counters + at);
-}
-
-bool stream_applies(const FcDeviceArgs& a) {
-    const Layout& L = a.layout;
-    return L.tiled && a.M > 0 && a.M <= kDecodeMaxRows && a.M * a.K * 2 < ((int64_t)1 << 31) &&
-           L.k_blocks * L.tiles_per_kblock * kTileBytes < ((int64_t)1 << 31) && L.groups * 32 < ((int64_t)1 << 31);
-}
-
-// Which calls it takes from the kernel that plan_launch chose (figures: that kernel against this one, us).
-bool stream_preferred(const FcDeviceArgs& a, const LaunchPlan& p) {
-    const Layout& L = a.layout;
-    // (nodes under 256 KiB stay where they are: their launches cost the same wherever they run)
-    if (p.kernel != OVFCC_KERNEL_DECODE || !stream_applies(a) || L.w_bytes < ((size_t)256 << 10))
-        return false;
-    // All of the small-batch kernel's: u8 8192 -> 57344 at 24 rows 110 / 83, 28672 -> 8192 71 / 44; i4 in groups of 64,
-    // 4096 -> 28672 at 24 rows 28.1 / 20.4, at 48 39.1 / 26.4; i8 1024 -> 1024 at 32 rows 8.9 / 5.8.  (The one
-    // exception costs it 5 %: u4 6144 -> 38912 at 5 rows 30.0 / 31.3.)
-    if (p.batch)
-        return true;
-    // The 16-row kernel with stationary activations where it streams many weights once per row tile, or cuts K in two
-    // and adds the parts in a second launch: 4096 -> 28672 at 40 rows 32.6 / 26.4, 6144 -> 9216 at 24 rows 15.3 / 13.7, at
-    // 48 rows 22.4 / 17.1.  It stays for 4096 -> 28672 at 32 rows (19.5 / 20.6) and for smaller nodes (4096 -> 6144 at
-    // 48 rows 11.7 / 12.1, 4096 -> 4096 8.7 / 10.9); with K in four parts (14336 -> 4096 at 24 rows 17.1 / 14.4) the
-    // planner's choice is fixed by tests.
-    if (p.gemv16)
-        return a.M > 16 && ((p.split_k == 2 && L.w_bytes >= ((size_t)8 << 20)) || (p.split_k == 1 && a.M > 32 && L.w_bytes >= ((size_t)32 << 20)));
-    if (p.gemv || p.gemv16_stream)
-        return false;
-    // The streaming kernel of one channel tile per workgroup: from five rows on for nodes of 10 MB and more (i4 in
-    // groups of 64, 4096 -> 6144 at 8 rows 10.6 / 8.2; 4096 -> 4096, 8 MB, at 5 rows 6.3 / 7.3, at 16 rows 7.8 / 7.3),
-    // and for 8-bit nodes whose K is too long for its LDS (u8 28672 -> 8192 at 1 row 42.8 / 38.5).
-    return (a.M > 4 && L.w_bytes >= ((size_t)10 << 20)) || (L.bits == 8 && !p.x_in_lds && L.w_bytes >= ((size_t)64 << 20));
-}
-
-// Parts along K for a launch of `groups` workgroups per part, and the stages of a part.
-static void stream_parts(const Layout& L, int64_t groups, int n_cus, int64_t* split_out, int64_t* per_out) {
-    const int64_t stages = (L.k_blocks + 1) / 2;
-    // Parts along K: as many as make the launch shortest, counted in stages -- rounds of workgroups over the compute
-    // units times a part's stages and two more for its start and end.  (Two workgroups fit a compute unit, but a second
-    // round costs a round all the same: 8192 -> 10240 u8 at 16 rows, 80 groups, takes 17.8 us in 3 parts, 22.5 in 4.)
-    const int64_t stage_bytes = 2 * L.tiles_per_kblock * kTileBytes;
-    int64_t split = 1, per = stages, best = -1;
-    for (int64_t s = 1; s <= 16 && s <= stages; ++s) {
-        int64_t n = (stages + s - 1) / s;
-        // a part that begins a multiple of 32 KiB into its tile makes all streams of the launch meet in the same
-        // memory channels (8192 -> 8192 u8 at 16 rows: parts of 8 stages 20.5 us, of 10 15.4)
-        if (s > 1 && n * stage_bytes % (32 * 1024) == 0)
-            n += 2;
-        const int64_t parts = (stages + n - 1) / n;
-        const int64_t cost = (groups * parts + n_cus - 1) / n_cus * (n + 2);
-        if (best < 0 || cost < best)
-            best = cost, split = parts, per = n;
-    }
-    *split_out = split, *per_out = per;
-}
-
-void plan_stream(const FcDeviceArgs& a, int n_cus, LaunchPlan* plan) {
-    const Layout& L = a.layout;
-    LaunchPlan p;
-    p.kernel = OVFCC_KERNEL_DECODE;
-    p.stream = true;
-    p.name = L.bits == 4 ? "fcc_stream_w4" : "fcc_stream_w8";
-    const int64_t groups = (L.n_tiles + SR_WAVES - 1) / SR_WAVES;
-    const int mt = (int)((a.M + 15) / 16);
-    int64_t split, per;
-    stream_parts(L, groups, n_cus, &split, &per);
-    p.split_k = (int)split, p.kblocks_per_split = (int)(2 * per);
-    p.grid[0] = (unsigned)groups, p.grid[1] = (unsigned)split;
-    p.block = 64 * SR_WAVES;
-    p.tile_m = 16 * mt, p.tile_n = 16 * SR_WAVES;
-    p.workspace_bytes = split > 1 ? (size_t)groups * split * SR_WAVES * mt * 1024 : 0;
-    p.counter_count = split > 1 ? (size_t)groups : 0;
-    *plan = p;
-}
-
-bool plan_stream_routed(const FcDeviceArgs& a, int64_t pairs, int n_experts, int n_cus, LaunchPlan* plan, int* cap) {
-    const Layout& L = a.layout;
-    // The counts stay on the device: slices of the average bucket plus twice its square root (what random routing stays
-    // under), up to 32 rows.  Expert block of eight experts, hidden size 4096, MLP width 14336, top two, against the
-    // grouped prefill kernel: 1 row 79 / 57 us, 6 rows 216 / 152, 40 rows (slices of 32) 237 / 198, 80 rows 248 / 213;
-    // with slices of 48 rows it loses (100 rows 244 / 277).  Sixteen experts of 2048 x 2048, top four: 1 row 46 / 27,
-    // 80 rows 60 / 49.  (Nodes under 1 MiB were not measured and keep the prefill kernel.)
-    const double avg = (double)pairs / n_experts;
-    const int64_t likely = (int64_t)std::ceil(avg + 2.0 * std::sqrt(avg));
-    const int mt = (int)((likely + 15) / 16);
-    if (!L.tiled || L.bits != 4 || mt > 2 || L.w_bytes < ((size_t)1 << 20) || L.groups * 32 >= ((int64_t)1 << 31) ||
-        L.k_blocks * kTileBytes >= ((int64_t)1 << 31) || a.K * 2 * 16 * mt >= ((int64_t)1 << 31))
-        return false;
-    const int64_t slices = std::min(pairs, (pairs + 16 * mt - 1) / (16 * mt) + n_experts);
-    if (slices > 65535)
-        return false;
-    LaunchPlan p;
-    p.kernel = OVFCC_KERNEL_DECODE;
-    p.stream = true;
-    p.name = "fcc_stream_grouped_w4";
-    p.n_cus = n_cus;
-    const int64_t groups = (L.n_tiles + SR_WAVES - 1) / SR_WAVES;
-    const double reached = n_experts * (1.0 - std::pow(1.0 - 1.0 / n_experts, (double)pairs));
-    int64_t split, per;
-    stream_parts(L, groups * std::max<int64_t>(1, std::llround(reached)), n_cus, &split, &per);
-    p.split_k = (int)split, p.kblocks_per_split = (int)(2 * per);
-    p.grid[0] = (unsigned)groups, p.grid[1] = (unsigned)split, p.grid[2] = (unsigned)slices;
-    p.block = 64 * SR_WAVES;
-    p.tiles_x = (int)groups, p.tiles_y = (int)slices;
-    p.tile_m = 16 * mt, p.tile_n = 16 * SR_WAVES;
-    p.workspace_bytes = split > 1 ? (size_t)(slices * groups * split) * SR_WAVES * mt * 1024 : 0;
-    p.counter_count = split > 1 ? (size_t)(slices * groups) : 0;
-    *plan = p;
-    *cap = 16 * mt;
-    return true;
 }
 
 static StreamShape stream_shape(const FcDeviceArgs& a, const LaunchPlan& p) {

@@ -188,13 +188,19 @@ unsigned env_generation();
 // Enqueues on `stream` (a hipStream_t passed as void*); returns a HIP error code (0 = success).
 int launch_fc(const FcDeviceArgs& a, const LaunchPlan& plan, void* stream);
 int launch_plain(const FcDeviceArgs& a, const LaunchPlan& plan, void* stream);
-// Decomposition and launch of a call on a node with Layout::ragged (kernel_ragged.hip).
+// Decomposition and launch of a call on a node with Layout::ragged (kernel_ragged.hip): square tiles of the tile kernel,
+// halves per staged row (16 bytes of padding spread the rows over the banks), LDS of a wave of the rows kernel.
+constexpr int kRaggedTile = 64, kRaggedPitch = kBlockK + 8;
+constexpr int ragged_wave_lds(int mt) {
+    return mt * 16 * kRaggedPitch * 2;
+}
 // launch_ragged_repack brings the constants into that layout (w as OpenVINO packs it, w_out L.w_bytes, both on the device).
 int launch_ragged_repack(const ovfcc_fc_desc& d, const Layout& L, const void* w, void* w_out, void* stream);
 void plan_ragged(const FcDeviceArgs& a, int n_cus, LaunchPlan* plan);
 int launch_ragged(const FcDeviceArgs& a, const LaunchPlan& plan, void* stream);
 // The weight-streaming kernel for up to 48 rows of large tiled nodes (kernel_stream.hip): whether it can run a call,
 // whether it takes it from the kernel plan_launch chose, its decomposition, its launch.
+constexpr int kStreamWaves = 8;
 bool stream_applies(const FcDeviceArgs& a);
 bool stream_preferred(const FcDeviceArgs& a, const LaunchPlan& plan);
 void plan_stream(const FcDeviceArgs& a, int n_cus, LaunchPlan* plan);

@@ -1,6 +1,7 @@
 // Host-logic check, built with AddressSanitizer and UBSan by tests/test_host_logic.py: descriptor gate, layout,
 // repack round trips on exactly sized buffers, and the invariants every launch plan must satisfy before a kernel
 // may be launched with it.  No GPU: the kernel launchers are stubbed out (launch_stubs.h) and never called.
+#include <algorithm>
 #include <cstdio>
 #include <cstdlib>
 #include <cstring>
@@ -165,6 +166,103 @@ static void check_plan(const ovfcc_fc_desc& d, int64_t M, int force, int force_s
     }
 }
 
+static ovfcc::FcDeviceArgs node_args(const ovfcc_fc_desc& d, int64_t M) {
+    ovfcc::FcDeviceArgs a{};
+    a.M = M, a.N = d.N, a.K = d.K, a.group_size = d.group_size, a.w_type = d.w_type, a.zp_type = d.zp_type;
+    a.layout = ovfcc::make_layout(d);
+    a.N_out = a.layout.glu ? d.N / 2 : d.N;
+    return a;
+}
+
+// What every launch that cuts K must hold: parts that cover K, none of them empty, buffers exactly when there are parts.
+static void check_parts(const ovfcc::LaunchPlan& p, int64_t kb, const char* what) {
+    CHECK(p.split_k >= 1 && (int64_t)p.split_k * p.kblocks_per_split >= kb && (int64_t)(p.split_k - 1) * p.kblocks_per_split < kb,
+          "%s split=%d per=%d", what, p.split_k, p.kblocks_per_split);
+    CHECK((p.split_k > 1) == (p.workspace_bytes > 0) && (p.split_k > 1) == (p.counter_count > 0), "%s", what);
+    CHECK(p.grid[0] >= 1 && p.grid[1] >= 1 && p.grid[2] >= 1 && p.grid[1] < 65536 && p.grid[2] < 65536 &&
+              (uint64_t)p.grid[0] * p.grid[1] * p.grid[2] < (1ull << 31), "%s", what);
+}
+
+// The streaming kernel's plan of a call (launch_stream's assumptions); its scratch fits the fixed array.
+static bool check_stream(const ovfcc_fc_desc& d, int64_t M, int n_cus) {
+    const ovfcc::FcDeviceArgs a = node_args(d, M);
+    if (!ovfcc::stream_applies(a))
+        return false;
+    const ovfcc::Layout& L = a.layout;
+    ovfcc::LaunchPlan p;
+    ovfcc::plan_stream(a, n_cus, &p);
+    char what[160];
+    std::snprintf(what, sizeof(what), "%s M=%ld N=%ld K=%ld G=%ld cus=%d", p.name, (long)M, (long)d.N, (long)d.K,
+                  (long)d.group_size, n_cus);
+    check_parts(p, L.k_blocks, what);
+    CHECK(p.stream && p.kernel == OVFCC_KERNEL_DECODE && p.block == 64u * ovfcc::kStreamWaves, "%s", what);
+    CHECK(p.tile_m % 16 == 0 && p.tile_m >= M && p.tile_m < M + 16 && p.tile_m <= 48, "%s tile_m=%d", what, p.tile_m);
+    CHECK((int64_t)p.grid[0] * ovfcc::kStreamWaves >= L.n_tiles && p.grid[1] == (unsigned)p.split_k && p.grid[2] == 1, "%s", what);
+    CHECK(p.split_k == 1 || p.kblocks_per_split % 2 == 0, "%s per=%d", what, p.kblocks_per_split);
+    if (p.split_k > 1)
+        CHECK(p.workspace_bytes == (size_t)p.grid[0] * p.split_k * ovfcc::kStreamWaves * p.tile_m * 64 && p.counter_count == p.grid[0],
+              "%s ws=%zu", what, p.workspace_bytes);
+    CHECK(p.workspace_bytes <= ovfcc::kStaticWorkspaceBytes && p.counter_count * sizeof(unsigned) <= ovfcc::kStaticCounterBytes,
+          "%s needs %zu bytes and %zu counters of the fixed array", what, p.workspace_bytes, p.counter_count);
+    return true;
+}
+
+// The streaming kernel's plan of a routed launch: a slice for whatever the buckets can become.
+static bool check_stream_routed(const ovfcc_fc_desc& d, int64_t pairs, int experts, int n_cus) {
+    const ovfcc::FcDeviceArgs a = node_args(d, 1);
+    const ovfcc::Layout& L = a.layout;
+    ovfcc::LaunchPlan p;
+    int cap = -1;
+    if (!ovfcc::plan_stream_routed(a, pairs, experts, n_cus, &p, &cap)) {
+        CHECK(cap == -1, "a refused plan leaves the slice height alone");
+        return false;
+    }
+    char what[160];
+    std::snprintf(what, sizeof(what), "%s pairs=%ld experts=%d N=%ld K=%ld", p.name, (long)pairs, experts, (long)d.N, (long)d.K);
+    check_parts(p, L.k_blocks, what);
+    CHECK((cap == 16 || cap == 32) && p.tile_m == cap && p.kblocks_per_split % 2 == 0, "%s cap=%d", what, cap);
+    CHECK((int64_t)p.grid[0] * ovfcc::kStreamWaves >= L.n_tiles && p.tiles_x == (int)p.grid[0] && p.grid[1] == (unsigned)p.split_k, "%s", what);
+    // most slices: one pair in as many experts as there are, the rest in one of them
+    const int64_t lone = std::min<int64_t>(experts, pairs) - 1, worst = lone + (pairs - lone + cap - 1) / cap;
+    CHECK(p.grid[2] >= (unsigned)worst && p.tiles_y == (int)p.grid[2] && (int64_t)p.grid[2] <= (pairs + cap - 1) / cap + experts,
+          "%s slices=%u worst=%ld", what, p.grid[2], (long)worst);
+    if (p.split_k > 1)
+        CHECK(p.workspace_bytes == (size_t)p.grid[2] * p.grid[0] * p.split_k * ovfcc::kStreamWaves * cap * 64 &&
+                  p.counter_count == (size_t)p.grid[2] * p.grid[0], "%s ws=%zu", what, p.workspace_bytes);
+    return true;
+}
+
+// The plans of the kernels for nodes that fit no tile (launch_ragged's assumptions).
+static bool check_ragged(const ovfcc_fc_desc& d, int64_t M, int n_cus, int* tile_kernels) {
+    const ovfcc::FcDeviceArgs a = node_args(d, M);
+    const ovfcc::Layout& L = a.layout;
+    if (!L.ragged)
+        return false;
+    ovfcc::LaunchPlan p;
+    ovfcc::plan_ragged(a, n_cus, &p);
+    char what[160];
+    std::snprintf(what, sizeof(what), "%s M=%ld N=%ld K=%ld cus=%d", p.name, (long)M, (long)d.N, (long)d.K, n_cus);
+    CHECK(!L.tiled && p.kernel == OVFCC_KERNEL_PLAIN && L.w_bytes == (size_t)((d.N + 15) / 16 * 16) * ((d.K + 127) / 128 * 128) * L.bits / 8,
+          "%s", what);
+    if (p.tile_n == 16) {
+        CHECK(p.split_k == 1 && p.workspace_bytes == 0 && p.counter_count == 0, "%s", what);
+        CHECK((int64_t)p.grid[0] * 16 >= d.N && (int64_t)p.grid[1] * p.tile_m >= M && p.grid[1] < 65536 && p.grid[2] == 1, "%s", what);
+        CHECK(p.block >= 64 && p.block <= 1024 && (int64_t)(p.block / 64) <= L.k_blocks && (p.tile_m == 16 || p.tile_m == 32), "%s", what);
+        CHECK(p.dynamic_lds == p.block / 64 * ovfcc::ragged_wave_lds(p.tile_m / 16) && p.dynamic_lds <= 160 * 1024, "%s", what);
+        return true;
+    }
+    ++*tile_kernels;
+    const int64_t tiles = (int64_t)p.tiles_x * p.tiles_y;
+    check_parts(p, L.k_blocks, what);
+    CHECK(p.tile_m == ovfcc::kRaggedTile && p.tile_n == ovfcc::kRaggedTile && p.block == 256, "%s", what);
+    CHECK((int64_t)p.tiles_x * ovfcc::kRaggedTile >= d.N && (int64_t)p.tiles_y * ovfcc::kRaggedTile >= M, "%s", what);
+    CHECK(p.grid[0] == (unsigned)((tiles + 7) / 8 * 8 * p.split_k) && p.grid[1] == 1 && p.grid[2] == 1, "%s", what);
+    if (p.split_k > 1)
+        CHECK(p.workspace_bytes == (size_t)tiles * p.split_k * ovfcc::kRaggedTile * ovfcc::kRaggedTile * 4 && p.counter_count == (size_t)tiles, "%s", what);
+    CHECK(p.workspace_bytes <= ovfcc::kStaticWorkspaceBytes && p.counter_count * sizeof(unsigned) <= ovfcc::kStaticCounterBytes, "%s", what);
+    return true;
+}
+
 // The environment overrides are read once and again only on request.
 static void check_env_cache() {
     unsetenv("OVFCC_PREFILL_ROWS");
@@ -221,7 +319,39 @@ int main() {
                                         ++plans;
                                     }
                     }
-    // untiled shapes: plain kernel only
+    // the streaming kernel, over the shapes above and wide nodes with long K
+    int streamed = 0, routed = 0, ragged = 0, tile_kernels = 0;
+    const int64_t wide_Ns[] = {16640, 32896, 37504, 43776, 57344, 264000}, long_Ks[] = {8192, 28672, 65536, 122880, 524288};
+    auto each_M = [&](const ovfcc_fc_desc& d) {
+        for (int64_t M : {1, 3, 4, 5, 16, 17, 32, 33, 48, 49})
+            for (int cus : {256, 64})
+                streamed += check_stream(d, M, cus);
+    };
+    for (int t : types) {
+        const int zp = (t == OVFCC_U4) ? OVFCC_U4 : (t == OVFCC_U8 ? OVFCC_U8 : OVFCC_NONE);
+        for (int64_t N : Ns)
+            for (int64_t K : Ks)
+                for (int64_t G : {(int64_t)64, (int64_t)128, K}) {
+                    const ovfcc_fc_desc d = desc(N, K, G, t, zp, 0);
+                    if (ovfcc::validate_desc(&d) != 0)
+                        continue;
+                    each_M(d);
+                    for (int64_t pairs : {1, 2, 7, 16, 33, 100, 160, 257, 1000, 2048})
+                        for (int experts : {1, 2, 8, 16, 64})
+                            routed += check_stream_routed(d, pairs, experts, 256);
+                }
+        for (int64_t N : wide_Ns)
+            for (int64_t K : long_Ks)
+                each_M(desc(N, K, K, t, zp, 0));
+        for (int64_t N : {1, 5, 15, 16, 17, 40, 63, 65, 260, 1000, 1160, 3480, 4300, 32003, 100003})
+            for (int64_t K : {8, 9, 127, 129, 200, 514, 1160, 1161, 4300, 20001, 100000})
+                for (int64_t M : {1, 15, 16, 17, 32, 33, 64, 65, 128, 256, 577, 641, 1500, 5003, 65535})
+                    for (int cus : {256, 64})
+                        ragged += check_ragged(desc(N, K, K, t, zp, 0), M, cus, &tile_kernels);
+    }
+    CHECK(streamed > 5000 && routed > 1000 && ragged > 10000 && tile_kernels > 5000, "%d %d %d %d", streamed, routed, ragged, tile_kernels);
+    plans += streamed + routed + ragged;
+    // untiled shapes of several groups: plain kernel only
     for (int fl : flags) {
         const ovfcc_fc_desc d = desc(40, 200, 50, OVFCC_U4, OVFCC_U4, fl);
         CHECK(ovfcc::validate_desc(&d) == 0 && !ovfcc::make_layout(d).tiled, "untiled");
