@@ -129,9 +129,9 @@ int plan_launch(const FcDeviceArgs& a, int force_kernel, int force_split, int n_
     if (kernel == OVFCC_KERNEL_AUTO)
         kernel = !L.tiled ? OVFCC_KERNEL_PLAIN : (a.M <= kDecodeMaxRows ? OVFCC_KERNEL_DECODE : OVFCC_KERNEL_PREFILL);
     if (kernel != OVFCC_KERNEL_PLAIN && !L.tiled)
-        return fail(OVFCC_EUNSUPPORTED, "this node keeps the OpenVINO layout; only the plain kernel can run it");
+        return fail(OVFCC_EUNSUPPORTED, "this node fits no tile; only the plain family can run it");
     if (kernel == OVFCC_KERNEL_PLAIN && L.tiled)
-        return fail(OVFCC_EUNSUPPORTED, "this node was repacked into tiles; the plain kernel needs the OpenVINO layout");
+        return fail(OVFCC_EUNSUPPORTED, "this node was repacked into tiles; the plain family runs nodes that fit no tile");
     if (kernel == OVFCC_KERNEL_DECODE && a.M > kDecodeMaxRows)
         return fail(OVFCC_EUNSUPPORTED, "the decode kernels handle at most 48 rows per launch");
     if (kernel == OVFCC_KERNEL_PREFILL && (a.N % kPrefillTileN) != 0)
@@ -698,7 +698,7 @@ bool plan_stream_routed(const FcDeviceArgs& a, int64_t pairs, int n_experts, int
 void plan_ragged(const FcDeviceArgs& a, int n_cus, LaunchPlan* plan) {
     LaunchPlan p;
     p.kernel = OVFCC_KERNEL_PLAIN;
-    p.name = "fcc_plain";
+    const bool four = a.layout.bits == 4;
     const int64_t kb = a.layout.k_blocks;
     // The rows kernel up to 16 rows, and up to the row count at which its workgroups (32 rows each) still fit the chip
     // in one round: N = 1000, K = 1160 at 128 rows (252 workgroups) 6.0 us against 8.8 for the tile kernel, at 192 rows
@@ -710,6 +710,7 @@ void plan_ragged(const FcDeviceArgs& a, int n_cus, LaunchPlan* plan) {
         p.grid[0] = (unsigned)((a.N + 15) / 16), p.grid[1] = (unsigned)((a.M + 16 * mt - 1) / (16 * mt));
         p.block = (unsigned)(64 * waves);
         p.tile_m = 16 * mt, p.tile_n = 16;
+        p.name = four ? "fcc_ragged_rows_w4" : "fcc_ragged_rows_w8";
         p.dynamic_lds = (unsigned)(waves * ragged_wave_lds(mt));
     } else {
         p.tiles_x = (int)((a.N + kRaggedTile - 1) / kRaggedTile), p.tiles_y = (int)((a.M + kRaggedTile - 1) / kRaggedTile);
@@ -725,6 +726,7 @@ void plan_ragged(const FcDeviceArgs& a, int n_cus, LaunchPlan* plan) {
         p.grid[0] = (unsigned)((tiles + 7) / 8 * 8 * split);
         p.block = 256;
         p.tile_m = kRaggedTile, p.tile_n = kRaggedTile;
+        p.name = four ? "fcc_ragged_tile_w4" : "fcc_ragged_tile_w8";
         p.workspace_bytes = split > 1 ? (size_t)tiles * split * kRaggedTile * kRaggedTile * sizeof(float) : 0;
         p.counter_count = split > 1 ? (size_t)tiles : 0;
     }

@@ -244,6 +244,8 @@ static bool check_ragged(const ovfcc_fc_desc& d, int64_t M, int n_cus, int* tile
     std::snprintf(what, sizeof(what), "%s M=%ld N=%ld K=%ld cus=%d", p.name, (long)M, (long)d.N, (long)d.K, n_cus);
     CHECK(!L.tiled && p.kernel == OVFCC_KERNEL_PLAIN && L.w_bytes == (size_t)((d.N + 15) / 16 * 16) * ((d.K + 127) / 128 * 128) * L.bits / 8,
           "%s", what);
+    const std::string kernel = std::string("fcc_ragged_") + (p.tile_n == 16 ? "rows_w" : "tile_w") + (L.bits == 4 ? "4" : "8");
+    CHECK(kernel == p.name, "%s is not %s", what, kernel.c_str());
     if (p.tile_n == 16) {
         CHECK(p.split_k == 1 && p.workspace_bytes == 0 && p.counter_count == 0, "%s", what);
         CHECK((int64_t)p.grid[0] * 16 >= d.N && (int64_t)p.grid[1] * p.tile_m >= M && p.grid[1] < 65536 && p.grid[2] == 1, "%s", what);

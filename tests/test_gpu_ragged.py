@@ -52,6 +52,9 @@ def test_widths_that_fit_no_tile(oracle, dev, req, wt, zt, N, K, bias, out, scal
         for M in MS:
             print(f"ragged {wt}/{zt} N={N} K={K} M={M}", flush=True)
             y = req.infer(w, c.x[:M])
+            info = req.last_kernel()
+            kernel = "rows" if info["tile_n"] == 16 else "tile"
+            assert info["name"] == f"fcc_ragged_{kernel}_w{wt[1]}", info
             check_parity(oracle, y, ref[:M], K, f"{wt}/{zt} N={N} K={K} M={M}", output_rounding_slack=True)
             if out == "f32":
                 assert oracle.rel_l2(y, ref[:M]) < 1e-5
