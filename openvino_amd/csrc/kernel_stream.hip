@@ -14,8 +14,10 @@
 // 64, 4096 -> 6144 at 24 rows 12.3 -> 9.8 us.
 //
 // Arithmetic as in the small-batch kernel: exact halves q - zp, v_mfma_f32_16x16x32_f16 with A = activations, the f32
-// partial sum of a group multiplied by its scale in f32 -- once at the end where a channel has one scale.  Split parts
-// are parked with device-scope stores and added in order by the last to arrive.
+// partial sum of a group multiplied by its scale in f32 -- once at the end where a channel has one scale, whose k-blocks
+// are summed from zero each and then added (one chain of MFMAs over a whole part of K rounds worse: u8 28672 -> 1024 at
+// 24 rows 2.4e-7 from 64 bits against 1.0e-7, the small-batch kernel 1.2e-7; the times do not differ).  Split parts are
+// parked with device-scope stores and added by the last to arrive, always in the same order, four at a time.
 #include "device_common.h"
 
 namespace ovfcc {
@@ -188,7 +190,7 @@ __device__ __forceinline__ void stream_body(const StreamItem& it, const StreamSh
                 float4_t part[MT];
 #pragma unroll
                 for (int t = 0; t < MT; ++t)
-                    part[t] = MODE == 0 ? acc[t] : float4_t{0.f, 0.f, 0.f, 0.f};
+                    part[t] = float4_t{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
                 for (int j = gi * (4 / GPB); j < (gi + 1) * (4 / GPB); ++j) {
                     Frag8 f;
@@ -204,7 +206,7 @@ __device__ __forceinline__ void stream_body(const StreamItem& it, const StreamSh
                 if constexpr (MODE == 0) {
 #pragma unroll
                     for (int t = 0; t < MT; ++t)
-                        acc[t] = part[t];
+                        acc[t] += part[t];
                 } else {
                     const float scale = (float)__builtin_bit_cast(half_t, (uint16_t)(q.scale[b][gi >> 1] >> (16 * (gi & 1))));
 #pragma unroll
@@ -271,12 +273,10 @@ __device__ __forceinline__ void stream_body(const StreamItem& it, const StreamSh
                     v[u][t] = __builtin_bit_cast(float4_t, __builtin_amdgcn_raw_buffer_load_b128(
                                                                rp, (unsigned)(z0 + u) * kPart + at + t * 1024u, 0, kAuxDeviceScope));
 #pragma unroll
-            for (int u = 0; u < 4; ++u)
+            for (int t = 0; t < MT; ++t)
 #pragma unroll
-                for (int t = 0; t < MT; ++t)
-#pragma unroll
-                    for (int q = 0; q < 4; ++q)
-                        sum[t][q] += v[u][t][q];
+                for (int q = 0; q < 4; ++q)
+                    sum[t][q] += (v[0][t][q] + v[1][t][q]) + (v[2][t][q] + v[3][t][q]);
         }
         if (tid == 0)
             __hip_atomic_store(counters + grp, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);

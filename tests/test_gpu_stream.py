@@ -80,6 +80,27 @@ def test_gated_linear_unit(oracle, dev, req, wt, zt, N, K, G, kind, second):
         w.close()
 
 
+@pytest.mark.parametrize("wt,zt,K,G", [("u8", "u8", 8192, 8192), ("i8", "none", 28672, 28672), ("u4", "u4", 14336, 14336),
+                                       ("u4", "u4", 8192, 64)])
+def test_sums_are_no_less_precise_than_the_small_batch_kernels(oracle, dev, req, monkeypatch, wt, zt, K, G):
+    """Both kernels sum exact products in f32, in different orders; 12 288 results, whose mean error varies by 1 %."""
+    c = datagen.make_case(2460, 24, K, 512, wt, G, zt)
+    exact = oracle_y(oracle, c, acc_f64=True).astype(np.float64)
+    w = fc.CompressedWeights.from_case(dev, c, output_type="f32")
+    try:
+        error = {}
+        for stream in ("0", "1"):
+            monkeypatch.setenv("OVFCC_STREAM", stream)
+            print(f"precision {wt}/{zt} K={K} G={G} OVFCC_STREAM={stream}", flush=True)
+            y = req.infer(w, c.x).astype(np.float64)
+            assert req.last_kernel()["name"].startswith("fcc_stream" if stream == "1" else "fcc_batch"), req.last_kernel()
+            error[stream] = np.linalg.norm(y - exact) / np.linalg.norm(exact)
+        print(error)
+        assert error["1"] <= 1.1 * error["0"], error
+    finally:
+        w.close()
+
+
 @pytest.mark.parametrize("env,M,name,block", [
     ({}, 32, "fcc_stream_w4", 512),
     ({"OVFCC_STREAM": "0"}, 32, "fcc_batch_w4", 512),
