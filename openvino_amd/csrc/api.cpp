@@ -46,7 +46,19 @@ int grow(void** p, size_t* cap, size_t need) {
     return OVFCC_OK;
 }
 
+// While any stream is under capture (another library's: nobody can capture a request's own stream), the runtime refuses
+// allocations on the threads that the capture's mode names and ends the capture.  Memory that no captured work uses may be
+// allocated all the same: the thread says so for as long as this lives.
+struct AllocateUnderCapture {
+    hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
+    AllocateUnderCapture() { (void)hipThreadExchangeStreamCaptureMode(&mode); }
+    ~AllocateUnderCapture() { (void)hipThreadExchangeStreamCaptureMode(&mode); }
+};
+
 int ensure_split_buffers(ovfcc_request* r, const ovfcc::LaunchPlan& plan) {
+    if (plan.workspace_bytes <= r->ws_cap && plan.counter_count <= r->counter_cap)
+        return OVFCC_OK;
+    AllocateUnderCapture relaxed;
     if (plan.workspace_bytes > r->ws_cap) {
         HIP_TRY(hipStreamSynchronize(r->stream));
         int rc = grow(reinterpret_cast<void**>(&r->workspace), &r->ws_cap, plan.workspace_bytes);
