@@ -391,7 +391,7 @@ int plan_call(const ovfcc_request* r, const ovfcc::FcDeviceArgs& a, int force, o
         p->kernel != OVFCC_KERNEL_DECODE)
         return rc;
     const int wish = ovfcc::env_int("OVFCC_STREAM", -1);
-    if (wish == 1 ? ovfcc::stream_applies(a) : wish != 0 && !ovfcc::decode_overridden() && ovfcc::stream_preferred(a, *p))
+    if (wish == 1 ? ovfcc::stream_applies(a) : wish != 0 && !ovfcc::decode_overridden() && ovfcc::stream_preferred(a, *p, r->ctx->n_cus))
         ovfcc::plan_stream(a, r->ctx->n_cus, p);
     return OVFCC_OK;
 }

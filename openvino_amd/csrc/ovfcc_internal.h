@@ -202,7 +202,7 @@ int launch_ragged(const FcDeviceArgs& a, const LaunchPlan& plan, void* stream);
 // whether it takes it from the kernel plan_launch chose, its decomposition, its launch.
 constexpr int kStreamWaves = 8;
 bool stream_applies(const FcDeviceArgs& a);
-bool stream_preferred(const FcDeviceArgs& a, const LaunchPlan& plan);
+bool stream_preferred(const FcDeviceArgs& a, const LaunchPlan& plan, int n_cus);
 void plan_stream(const FcDeviceArgs& a, int n_cus, LaunchPlan* plan);
 int launch_stream(const FcDeviceArgs& a, const LaunchPlan& plan, void* stream);
 int launch_decode(const FcDeviceArgs& a, const LaunchPlan& plan, void* stream);

@@ -583,29 +583,38 @@ bool stream_applies(const FcDeviceArgs& a) {
 }
 
 // Which calls it takes from the kernel that plan_launch chose (figures: that kernel against this one, us).
-bool stream_preferred(const FcDeviceArgs& a, const LaunchPlan& p) {
+bool stream_preferred(const FcDeviceArgs& a, const LaunchPlan& p, int n_cus) {
     const Layout& L = a.layout;
     // (nodes under 256 KiB stay where they are: their launches cost the same wherever they run)
     if (p.kernel != OVFCC_KERNEL_DECODE || !stream_applies(a) || L.w_bytes < ((size_t)256 << 10))
         return false;
     // All of the small-batch kernel's: u8 8192 -> 57344 at 24 rows 110 / 83, 28672 -> 8192 71 / 44; i4 in groups of 64,
-    // 4096 -> 28672 at 24 rows 28.1 / 20.4, at 48 39.1 / 26.4; i8 1024 -> 1024 at 32 rows 8.9 / 5.8.  (The one
-    // exception costs it 5 %: u4 6144 -> 38912 at 5 rows 30.0 / 31.3.)
+    // 4096 -> 28672 at 24 rows 28.1 / 20.4, at 48 39.1 / 26.4; i8 1024 -> 1024 at 32 rows 8.9 / 5.8.  (Over 60 drawn nodes
+    // the worst are 4-bit ones of groups of 128 with a zero-point table, up to 8 rows: 11648 -> 3584 11.6 / 11.9, 7296 ->
+    // 6896 12.4 / 12.7.)
     if (p.batch)
         return true;
-    // The 16-row kernel with stationary activations where it streams many weights once per row tile, or cuts K in two
-    // and adds the parts in a second launch: 4096 -> 28672 at 40 rows 32.6 / 26.4, 6144 -> 9216 at 24 rows 15.3 / 13.7, at
-    // 48 rows 22.4 / 17.1.  It stays for 4096 -> 28672 at 32 rows (19.5 / 20.6) and for smaller nodes (4096 -> 6144 at
-    // 48 rows 11.7 / 12.1, 4096 -> 4096 8.7 / 10.9); with K in four parts (14336 -> 4096 at 24 rows 17.1 / 14.4) the
-    // planner's choice is fixed by tests.
+    // The 16-row kernel with stationary activations where it streams many weights once per row tile, or cuts K of a
+    // large node in two and adds the parts in a second launch: 4096 -> 28672 at 40 rows 32.6 / 26.4, 6144 -> 9216 at 24
+    // rows 15.3 / 13.7, at 48 rows 22.4 / 17.1.  It stays for 4096 -> 28672 at 32 rows (19.5 / 20.6), for smaller nodes
+    // (4096 -> 6144 at 48 rows 11.7 / 12.1; two parts of 8 to 17 MB at 40 rows: 7680 -> 2368 12.4 / 14.5, 7168 -> 3824 12.9 /
+    // 14.5, 5632 -> 6304 14.7 / 15.5, with a few the other way: 4608 -> 6864 15.0 / 13.3) and with K in four parts.
     if (p.gemv16)
-        return a.M > 16 && ((p.split_k == 2 && L.w_bytes >= ((size_t)8 << 20)) || (p.split_k == 1 && a.M > 32 && L.w_bytes >= ((size_t)32 << 20)));
+        return a.M > 16 && ((p.split_k == 2 && L.w_bytes >= ((size_t)20 << 20)) || (p.split_k == 1 && a.M > 32 && L.w_bytes >= ((size_t)32 << 20)));
     if (p.gemv || p.gemv16_stream)
         return false;
-    // The streaming kernel of one channel tile per workgroup: from five rows on for nodes of 10 MB and more (i4 in
-    // groups of 64, 4096 -> 6144 at 8 rows 10.6 / 8.2; 4096 -> 4096, 8 MB, at 5 rows 6.3 / 7.3, at 16 rows 7.8 / 7.3),
-    // and for 8-bit nodes whose K is too long for its LDS (u8 28672 -> 8192 at 1 row 42.8 / 38.5).
-    return (a.M > 4 && L.w_bytes >= ((size_t)10 << 20)) || (L.bits == 8 && !p.x_in_lds && L.w_bytes >= ((size_t)64 << 20));
+    // The streaming kernel of one channel tile per workgroup: 8-bit nodes whose K is too long for its LDS (u8 28672 ->
+    // 8192 at 1 row 42.8 / 38.5, 15104 -> 4416 18.3 / 15.8), and from five rows on nodes of 10 MB and more (larger ones
+    // than 16 MB are the small-batch kernel's).  There its time grows with the rows and with K, which one workgroup
+    // contracts, while this kernel's is what its many parts and their sum take, 8 to 10 us: 3552 channels of 8 bits, K =
+    // 4096, 6.5 / 8.5 at 5 rows, 8.4 / 8.6 at 16; 5376 -> 2256 7.4 / 8.6 at 5 rows, 8.3 / 8.6 at 10; 7936 -> 2032 9.7 / 10.2
+    // at 8; 9728 -> 1584 12.6 / 9.8 at 16; i4 in groups of 128, 7808 -> 3472 8.3 / 9.5 at 5; in groups of 32, 7424 -> 2944 9.3
+    // / 9.8 at 6, even at 9.  Where its workgroups need a second round and its groups cost it most (several to a k-block,
+    // or 4-bit ones with a zero-point table), all move: i4 in groups of 64, 4096 -> 6144 at 8 rows 10.6 / 8.2.
+    if (L.bits == 8 && !p.x_in_lds && L.w_bytes >= ((size_t)64 << 20))
+        return true;
+    const bool slow_rounds = L.n_tiles > n_cus && (L.groups_per_kblock != 1 || (L.bits == 4 && L.zp_table && L.groups > 1));
+    return a.M > 4 && L.w_bytes >= ((size_t)10 << 20) && (slow_rounds || a.K * (a.M + 10) >= 145000);
 }
 
 constexpr int64_t kStreamMaxParts = 16;

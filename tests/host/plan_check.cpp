@@ -232,6 +232,37 @@ static bool check_stream_routed(const ovfcc_fc_desc& d, int64_t pairs, int exper
     return true;
 }
 
+// Which calls the streaming kernel takes from the kernel that plan_launch chose, on both sides of each line (256 compute
+// units; times of both in stream_preferred).
+static void check_stream_rule() {
+    const struct { int64_t N, K, G, M; int w, zp; const char* from; bool taken; } calls[] = {
+        {3552, 4096, 4096, 5, OVFCC_U8, OVFCC_U8, "fcc_decode_w8", false},      // 8 bits, 10 to 16 MB
+        {3552, 4096, 4096, 16, OVFCC_I8, OVFCC_NONE, "fcc_decode_w8", false},
+        {2176, 6016, 6016, 6, OVFCC_U8, OVFCC_U8, "fcc_decode_w8", false},
+        {1584, 9728, 9728, 16, OVFCC_I8, OVFCC_NONE, "fcc_decode_w8", true},
+        {8192, 28672, 28672, 1, OVFCC_U8, OVFCC_U8, "fcc_decode_w8", true},
+        {57344, 8192, 8192, 24, OVFCC_U8, OVFCC_U8, "fcc_batch_w8", true},
+        {2944, 7424, 32, 6, OVFCC_I4, OVFCC_NONE, "fcc_decode_w4", false},      // one round of its workgroups
+        {6144, 4096, 64, 8, OVFCC_I4, OVFCC_NONE, "fcc_decode_w4", true},       // two
+        {3472, 7808, 128, 5, OVFCC_I4, OVFCC_NONE, "fcc_decode_w4", false},
+        {2368, 7680, 128, 40, OVFCC_I4, OVFCC_NONE, "fcc_gemv16_w4", false},    // K in two parts
+        {9216, 6144, 128, 24, OVFCC_U4, OVFCC_U4, "fcc_gemv16_w4", true},
+        {28672, 4096, 128, 32, OVFCC_U4, OVFCC_U4, "fcc_gemv16_w4", false},
+        {28672, 4096, 128, 40, OVFCC_U4, OVFCC_U4, "fcc_gemv16_w4", true},
+    };
+    for (const auto& c : calls) {
+        ovfcc::FcDeviceArgs a = node_args(desc(c.N, c.K, c.G, c.w, c.zp, 0), c.M);
+        if (c.G == 128) {  // what the channel-major tables of such a node make possible
+            a.layout.gemv_c = ovfcc::gemv_kblocks_per_wave(a.layout, 256);
+            a.scale_cm = a.layout.gemv_c ? &a : nullptr;
+        }
+        ovfcc::LaunchPlan p;
+        CHECK(ovfcc::plan_launch(a, OVFCC_KERNEL_AUTO, 0, 256, &p) == OVFCC_OK && std::string(p.name) == c.from &&
+                  ovfcc::stream_preferred(a, p, 256) == c.taken,
+              "%s M=%ld N=%ld K=%ld G=%ld", p.name, (long)c.M, (long)c.N, (long)c.K, (long)c.G);
+    }
+}
+
 // The plans of the kernels for nodes that fit no tile (launch_ragged's assumptions).
 static bool check_ragged(const ovfcc_fc_desc& d, int64_t M, int n_cus, int* tile_kernels) {
     const ovfcc::FcDeviceArgs a = node_args(d, M);
@@ -295,6 +326,7 @@ static void check_env_cache() {
 
 int main() {
     check_env_cache();
+    check_stream_rule();
     std::mt19937 rng(12345);
     const int64_t Ns[] = {16, 32, 48, 96, 128, 256, 272, 1024, 4096, 14336};
     const int64_t Ks[] = {128, 256, 384, 1024, 4096, 14336};
