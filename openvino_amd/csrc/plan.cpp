@@ -713,7 +713,8 @@ void plan_ragged(const FcDeviceArgs& a, int n_cus, LaunchPlan* plan) {
     // in one round: N = 1000, K = 1160 at 128 rows (252 workgroups) 6.0 us against 8.8 for the tile kernel, at 192 rows
     // (378) 10.3 against 8.8; N = 2000 at 64 rows 5.8 against 8.7, at 96 rows 10.1 against 8.9; N = 4300 at 32 rows (269)
     // 10.0 against 8.9.
-    const int mt = a.M <= 16 ? 1 : 2;
+    // Row tiles of 16 as long as they fit in one round: each wave has half of the rows to stage.
+    const int mt = a.M <= 16 || (a.N + 15) / 16 * ((a.M + 15) / 16) <= n_cus ? 1 : 2;
     if (a.M <= 16 || (a.N + 15) / 16 * ((a.M + 31) / 32) <= n_cus) {
         const int64_t waves = kb < 16 ? kb : 16;
         p.grid[0] = (unsigned)((a.N + 15) / 16), p.grid[1] = (unsigned)((a.M + 16 * mt - 1) / (16 * mt));

@@ -281,6 +281,8 @@ static bool check_ragged(const ovfcc_fc_desc& d, int64_t M, int n_cus, int* tile
         CHECK(p.split_k == 1 && p.workspace_bytes == 0 && p.counter_count == 0, "%s", what);
         CHECK((int64_t)p.grid[0] * 16 >= d.N && (int64_t)p.grid[1] * p.tile_m >= M && p.grid[1] < 65536 && p.grid[2] == 1, "%s", what);
         CHECK(p.block >= 64 && p.block <= 1024 && (int64_t)(p.block / 64) <= L.k_blocks && (p.tile_m == 16 || p.tile_m == 32), "%s", what);
+        // taller row tiles only where the low ones need a second round
+        CHECK((p.tile_m == 16) == (M <= 16 || (d.N + 15) / 16 * ((M + 15) / 16) <= n_cus), "%s tile_m=%d", what, p.tile_m);
         CHECK(p.dynamic_lds == p.block / 64 * ovfcc::ragged_wave_lds(p.tile_m / 16) && p.dynamic_lds <= 160 * 1024, "%s", what);
         return true;
     }
