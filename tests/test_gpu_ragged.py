@@ -1,8 +1,9 @@
-"""GPU parity of nodes with one scale per channel whose widths fit no tile (OpenVINO layout, matrix-core kernels that
-read the constants as they lie) against the CPU oracle: tails of K and N, row tiles of 16 and 64 rows and their edges,
-K split over workgroups, every zero-point form, both output types.  Weights are exact integers in the kernels and the
-products are summed in f32, so f32 outputs agree with a float64 sum to K 2^-24 of the sum of magnitudes, here bounded
-as 1e-5 relative in the 2-norm; f16 outputs add their own rounding (the bounds of tests/parity.py)."""
+"""GPU parity of nodes with one scale per channel whose widths fit no tile (matrix-core kernels over weights in operand
+order, activations as given) against the CPU oracle: tails of K and N, the rows kernel and the tile kernel with the
+edges of their row tiles, K split over workgroups (the tile kernel only), every zero-point form, both output types.
+Weights are exact integers in the kernels and the products are summed in f32, so f32 outputs agree with a float64 sum
+to K 2^-24 of the sum of magnitudes, here bounded as 1e-5 relative in the 2-norm; f16 outputs add their own rounding
+(the bounds of tests/parity.py)."""
 import numpy as np
 import pytest
 
@@ -34,7 +35,7 @@ def req(dev):
     ("i8", "u8", 67, 1161, True, "f16", False),       # both odd: single halves at the end of a row, 2-byte rows
     ("u8", "none", 5, 8, False, "f32", False),        # one chunk of eight inputs
     ("i8", "none", 63, 9, True, "f32", False),
-    ("u8", "u8", 130, 4300, True, "f16", True),       # long K: split over workgroups
+    ("u8", "u8", 130, 4300, True, "f16", True),       # long K: three k-blocks to a wave
     ("i4", "none", 65, 1160, True, "f32", False),     # nibbles
     ("u4", "u4", 33, 650, False, "f16", False),
     ("i4", "u8", 17, 4102, False, "f32", False),
@@ -63,14 +64,51 @@ def test_widths_that_fit_no_tile(oracle, dev, req, wt, zt, N, K, bias, out, scal
         w.close()
 
 
+@pytest.mark.parametrize("wt,zt,N,K,bias,out,scalar,runs", [
+    # runs: {M: parts of K}.  One channel of the last tile of 64, one row of the last row tile, tails of K.
+    ("i8", "none", 1160, 1160, True, "f16", False, {577: 2, 640: 2, 641: 2}),    # parts of five k-blocks
+    ("u8", "u8", 1161, 1161, True, "f32", False, {577: 2, 1300: 1}),             # ten k-blocks, the last of nine inputs
+    ("u4", "u4", 1160, 4300, False, "f32", False, {577: 4}),                     # parts of 9, 9, 9 and 7 k-blocks
+    ("i4", "none", 100, 4302, True, "f32", False, {1500: 7}),                    # parts of five, the last of four
+    ("i8", "u8", 1161, 200, False, "f16", False, {577: 1}),
+    ("i4", "none", 1160, 8, True, "f16", False, {577: 1}),                       # one chunk of one k-block
+    ("u4", "u8", 2113, 300, True, "f32", False, {63: 1, 64: 1, 65: 1, 577: 1}),  # three k-blocks
+    ("u8", "none", 4300, 394, False, "f16", False, {17: 1, 33: 1}),              # less than one row tile
+    ("u8", "u8", 1089, 1161, False, "f16", True, {577: 2}),
+    ("u4", "u4", 1090, 650, True, "f32", True, {577: 1}),
+])
+def test_tiles(oracle, dev, req, wt, zt, N, K, bias, out, scalar, runs):
+    """The tile kernel, unsplit and with K split, over even and odd numbers of k-blocks."""
+    c = datagen.make_case(2150 + N + K, max(runs), K, N, wt, K, zt, with_bias=bias)
+    if scalar:
+        c.zp = c.zp[:1].copy()
+        c.zp_scalar = True
+    w = fc.CompressedWeights.from_case(dev, c, output_type=out)
+    try:
+        for M, parts in runs.items():
+            print(f"ragged tiles {wt}/{zt} N={N} K={K} M={M}", flush=True)
+            y, info = req.infer(w, c.x[:M]), req.last_kernel()
+            assert info["name"] == f"fcc_ragged_tile_w{wt[1]}" and (info["tile_m"], info["tile_n"]) == (64, 64), info
+            assert info["split_k"] == parts, info
+            rows = np.unique(np.clip(np.r_[0:M:37, 60:68, M - 66:M], 0, M - 1))
+            ref = oracle_y(oracle, c, x=c.x[rows])
+            check_parity(oracle, y[rows], ref, K, f"{wt}/{zt} N={N} K={K} M={M}", output_rounding_slack=True)
+            if out == "f32":
+                assert oracle.rel_l2(y[rows], ref) < 1e-5
+            assert np.array_equal(y, req.infer(w, c.x[:M]))
+    finally:
+        w.close()
+
+
 def test_rows_keep_to_themselves(dev, req):
     """A row's result does not see its neighbours: what a lane loads beyond the end of a row is the next row, here
     infinities and NaNs."""
-    for M in (3, 40):
-        c = datagen.make_case(2200, M, 203, 50, "i8", 203, "none")
+    for N, M, kernel in ((50, 3, "rows"), (50, 40, "rows"), (1161, 577, "tile")):
+        c = datagen.make_case(2200, M, 203, N, "i8", 203, "none")
         w = fc.CompressedWeights.from_case(dev, c, output_type="f32")
         try:
             clean = req.infer(w, c.x)
+            assert req.last_kernel()["name"] == f"fcc_ragged_{kernel}_w8"
             x = c.x.copy()
             x[1::2] = np.inf
             x[1, 0] = np.nan

@@ -1,5 +1,5 @@
-"""GPU parity of the weight-streaming kernel (5-48 rows of large tiled nodes) against the CPU oracle, where it can go
-wrong: a last workgroup with channels for some of its waves only, an odd number of k-blocks (half a stage), K split over
+"""GPU parity of the weight-streaming kernel (up to 48 rows of large tiled nodes) against the CPU oracle, where it can
+go wrong: a last workgroup with channels for some of its waves only, an odd number of k-blocks (half a stage), K split over
 workgroups with a short last part, row tiles and their edges, every group size and zero-point form, the gated linear
 unit, both output types.  Bounds of tests/parity.py; f32 outputs add no rounding of their own and the weights are exact
 in the kernel, so they stay within 1e-5 of the oracle's f32 sums."""
@@ -43,8 +43,7 @@ CASES = [
 ]
 
 
-@pytest.mark.parametrize("wt,zt,N,K,G,bias,out,rows", CASES)
-def test_parity(oracle, dev, req, wt, zt, N, K, G, bias, out, rows):
+def parity(oracle, dev, req, wt, zt, N, K, G, bias, out, rows):
     c = datagen.make_case(2300 + N, max(rows), K, N, wt, G, zt, with_bias=bias)
     ref = oracle_y(oracle, c)
     w = fc.CompressedWeights.from_case(dev, c, output_type=out)
@@ -59,6 +58,35 @@ def test_parity(oracle, dev, req, wt, zt, N, K, G, bias, out, rows):
                 assert oracle.rel_l2(y, ref[:M]) < 1e-5
             for _ in range(3):      # split parts are added in order: the same bits every time
                 assert np.array_equal(y, req.infer(w, c.x[:M]))
+    finally:
+        w.close()
+
+
+@pytest.mark.parametrize("wt,zt,N,K,G,bias,out,rows", CASES)
+def test_parity(oracle, dev, req, wt, zt, N, K, G, bias, out, rows):
+    parity(oracle, dev, req, wt, zt, N, K, G, bias, out, rows)
+
+
+@pytest.mark.parametrize("wt,zt,N,K,G,bias,out", [case[:7] for case in CASES[:10]])
+def test_one_to_four_rows(oracle, dev, req, monkeypatch, wt, zt, N, K, G, bias, out):
+    """Most nodes of these sizes run other kernels at so few rows; the kernel itself takes them all."""
+    monkeypatch.setenv("OVFCC_STREAM", "1")
+    parity(oracle, dev, req, wt, zt, N, K, G, bias, out, [1, 2, 3, 4])
+
+
+@pytest.mark.parametrize("wt,zt,N,K,G,glu", [
+    ("u8", "u8", 2400, 28672, 28672, None),      # 8 bits, K beyond the LDS of the kernel with one tile per workgroup
+    ("u4", "u4", 2080, 24576, 64, "swish")])     # a gated linear unit with long K
+def test_one_to_four_rows_of_long_nodes(oracle, dev, req, wt, zt, N, K, G, glu):
+    c = datagen.make_case(2500 + N, 4, K, N, wt, G, zt, with_bias=True)
+    ref, amp = glu_reference(oracle, c, glu) if glu else (oracle_y(oracle, c), 1.0)
+    w = fc.CompressedWeights.from_case(dev, c, glu=glu)
+    try:
+        for M in (1, 2, 4):
+            print(f"stream {wt}/{zt} N={N} K={K} G={G} glu={glu} M={M}", flush=True)
+            y, info = req.infer(w, c.x[:M]), req.last_kernel()
+            assert info["name"].startswith("fcc_stream"), info
+            check_parity(oracle, y, ref[:M], K, f"{info}", output_rounding_slack=True, limit_scale=amp)
     finally:
         w.close()
 
