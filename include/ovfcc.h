@@ -242,7 +242,8 @@ int ovfcc_fc_run(ovfcc_request* req, const ovfcc_weights* w, const void* x_host,
 
 /* Same with device-resident X and Y (a remote tensor in OpenVINO terms,
  * src/inference/dev_api/openvino/runtime/iremote_tensor.hpp): enqueues on the request's
- * stream and returns without waiting. */
+ * stream and returns without waiting -- except that a launch which needs more scratch than any before it on this
+ * request (K cut into parts, activations quantised) allocates it, after the request's earlier work. */
 int ovfcc_fc_run_device(ovfcc_request* req, const ovfcc_weights* w, const void* x_dev, void* y_dev, int64_t M);
 
 /* ovfcc_fc_run_device for callers that cannot allocate device memory (code under HIP graph capture, tight serving

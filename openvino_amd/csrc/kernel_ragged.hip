@@ -16,15 +16,17 @@
 //                           unpacked once per 64 rows and an activation operand read from LDS meets four MFMAs
 //                           (half of what LDS delivers at the matrix cores' rate; waves side by side along N would
 //                           need all of it).  Three workgroups share a compute unit and hide each other's loads,
-//                           which travel two k-blocks ahead through registers (rows of K halves start anywhere: no
-//                           direct-to-LDS load, which wants 16-byte pieces).  577 x 1160 -> 3480 (552 tiles) takes
-//                           18 us: 8 of launch, first loads and epilogue, then 1 us per k-block, of which the matrix
-//                           cores are busy 0.3 (29 % by the counter); a third workgroup on some compute units and two
-//                           on the others make the rest.
+//                           which travel two k-blocks ahead through registers: where K is no multiple of eight, rows
+//                           start anywhere and a direct-to-LDS load, which wants 16-byte pieces, cannot fetch them
+//                           (other K could; that form is not built).  577 x 1160 -> 3480 (552 tiles) takes
+//                           18 us (21 under the tracer): 8 of launch, first loads and epilogue, then 1 us per k-block
+//                           against 0.3 of matrix-core work (their pipe is busy 19 % of the launch by the counter;
+//                           a third of the waves' cycles are waits); a third workgroup on some compute units and
+//                           two on the others make the rest.
 // What a load costs the compute unit is the number of 64-byte pieces its 64 lanes name in lane order: weights read
 // where OpenVINO left them (neighbouring lanes in different rows) kept the cache's tag stage busy every cycle of the
 // launch -- 577 x 4640 -> 3480 took 61.6 us that way and takes 42.1 in operand order.
-// An encoder layer of hidden size 1160 (four nodes, 577 rows) takes 71 us where one wave per output took 7 840.
+// An encoder layer of hidden size 1160 (four nodes, 577 rows) takes 75 us where one wave per output took 7 850.
 #include <atomic>
 
 #include "device_common.h"
@@ -265,7 +267,7 @@ __global__ __launch_bounds__(256) void fcc_ragged_tile_kernel(RaggedNode a, int 
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int run = (tiles + 7) >> 3;
     const int tile = (int)(blockIdx.x & 7) * run + (int)((blockIdx.x >> 3) % run), part = (int)((blockIdx.x >> 3) / run);
-    if ((int)((blockIdx.x >> 3) % run) >= run || tile >= tiles)
+    if (tile >= tiles)
         return;
     const int n0 = tile / tiles_m * RG_BN, m0 = tile % tiles_m * RG_BM;
     const int kb_lo = part * kb_per_split, kb_hi = min(kb_total, kb_lo + kb_per_split);

@@ -2,7 +2,7 @@
 //
 //   grid = (ceil(N / 16 / 8), split along K, slices of a grouped launch), block = 512: eight waves, each with a channel
 //   tile of its own whose weights go straight from memory into the MFMA weight operand, a stage (two k-blocks) at a
-//   time, SR_DEPTH stages ahead.  The activations of a stage, 16 MT rows x 256 inputs, pass through registers into
+//   time, three stages ahead (four of 4-bit weights, which are half as large).  The activations of a stage, 16 MT rows x 256 inputs, pass through registers into
 //   one of two LDS buffers that all eight waves read: one barrier per stage, which waits for LDS only.
 //
 // The small-batch kernel (kernel_batch.hip) brings a workgroup's whole slice of X to LDS before the first product and
@@ -67,7 +67,7 @@ __device__ __forceinline__ void stream_body(const StreamItem& it, const StreamSh
     constexpr unsigned kOob = 0x80000000u;
     constexpr int kRsrcFlags = 0x00020000;
     const size_t t0 = mine ? (size_t)tile : 0;
-    // (the range ends with this part of K: a stage's second k-block past it reads zeros)
+    // (the range ends with this part of K: of a stage's second k-block past it every code reads as zero, a weight of -zp)
     const __amdgpu_buffer_rsrc_t rw = __builtin_amdgcn_make_buffer_rsrc(
         const_cast<uint4_t*>(it.w + t0 * sh.kb_total * TPB * 64), 0, mine ? kb_end * TPB * kTileBytes : 0, kRsrcFlags);
     const __amdgpu_buffer_rsrc_t rs = __builtin_amdgcn_make_buffer_rsrc(const_cast<half_t*>(it.scale + t0 * sh.ng * 16), 0,
@@ -96,7 +96,7 @@ __device__ __forceinline__ void stream_body(const StreamItem& it, const StreamSh
     uint4_t xr[MT];
     auto load_x = [&](int s) {
         const unsigned k = (unsigned)(kb_begin + 2 * s) * kBlockK;
-        // inputs past this part of K: the weights that meet them are zeros, but the activations need not be finite there
+        // inputs past this part of K are zeros, which is what makes half a stage right: the weights that meet them are -zp
         const unsigned oob = k + (tid & 31) * 8u >= (unsigned)kb_end * kBlockK ? kOob : 0u;
 #pragma unroll
         for (int i = 0; i < MT; ++i)
@@ -333,9 +333,9 @@ __global__ __launch_bounds__(512, 4) void fcc_stream_kernel(StreamItem it, Strea
 
 // Slice blockIdx.z of the table that the routing kernel wrote: at most 16 MT rows of one expert.  Slices in use come
 // first in the table; the others have no rows.  Bound by the weights that the reached experts have: 6 rows through eight
-// experts of 4096 / 14336 (6.6 of them reached on average, 0.62 GB) take 152 us with routing and the weighted sum,
-// 4 TB/s.  The grouped prefill kernel, whose slices are 64 rows high at least, multiplies and unpacks for rows that are
-// not there and took 216.
+// experts of 4096 / 14336, top two, take 139 us with routing and the weighted sum, the two projections fetching their
+// weights at 4.5 to 4.7 TB/s.  The grouped prefill kernel, whose slices are 64 rows high at least, multiplies and unpacks
+// for rows that are not there and took 195.
 template <int MT, bool ZP_TABLE, int MODE>
 __global__ __launch_bounds__(512) void fcc_stream_grouped_kernel(const BatchGroupItem* __restrict__ tab, StreamShape sh,
                                                                  float* __restrict__ ws, unsigned* __restrict__ counters,

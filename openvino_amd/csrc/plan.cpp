@@ -1,9 +1,11 @@
 // Kernel choice and launch decomposition (host only).
 //
-// Policy: shapes that keep OpenVINO's layout run the plain kernel; tiled nodes run a decode kernel for
-// M <= 48 (the streaming kernel for a few rows, the small-batch kernel above) and the prefill kernel for more
-// (the roofline ridge of int4 g128 sits near M = 83).  The caller cuts 48 < M <= 128 into decode launches:
-// a single 128-row prefill tile per column block leaves most of the chip idle.
+// Policy: nodes that fit no tile run the ragged kernels (one scale per channel; plan_ragged) or the plain kernel; tiled
+// nodes run a decode kernel for M <= 48 and a prefill kernel for more (the roofline ridge of int4 g128 sits near
+// M = 83).  plan_launch chooses among the decode kernels that keep their activations (one channel tile per workgroup,
+// matrix-vector, 16-row, small-batch); of its choices the weight-streaming kernel takes what stream_preferred names.
+// The caller cuts 48 < M <= 128 into decode launches: a single 128-row prefill tile per column block leaves most of
+// the chip idle.
 #include <algorithm>
 #include <atomic>
 #include <cmath>
@@ -669,7 +671,7 @@ bool plan_stream_routed(const FcDeviceArgs& a, int64_t pairs, int n_experts, int
     const Layout& L = a.layout;
     // The counts stay on the device: slices of the average bucket plus twice its square root (what random routing stays
     // under), up to 32 rows.  Expert block of eight experts, hidden size 4096, MLP width 14336, top two, against the
-    // grouped prefill kernel: 1 row 79 / 57 us, 6 rows 216 / 152, 40 rows (slices of 32) 237 / 198, 80 rows 248 / 213;
+    // grouped prefill kernel: 1 row 79 / 57 us, 40 rows (slices of 32) 237 / 198, 80 rows 248 / 213;
     // with slices of 48 rows it loses (100 rows 244 / 277).  Sixteen experts of 2048 x 2048, top four: 1 row 46 / 27,
     // 80 rows 60 / 49.  (Nodes under 1 MiB were not measured and keep the prefill kernel.)
     const double avg = (double)pairs / n_experts;
