@@ -15,9 +15,10 @@
 //
 // Arithmetic as in the small-batch kernel: exact halves q - zp, v_mfma_f32_16x16x32_f16 with A = activations, the f32
 // partial sum of a group multiplied by its scale in f32 -- once at the end where a channel has one scale, whose k-blocks
-// are summed from zero each and then added (one chain of MFMAs over a whole part of K rounds worse: u8 28672 -> 1024 at
-// 24 rows 2.4e-7 from 64 bits against 1.0e-7, the small-batch kernel 1.2e-7; the times do not differ).  Split parts are
-// parked with device-scope stores and added by the last to arrive, always in the same order, four at a time.
+// are summed from zero each and added two at a time.  (One chain of MFMAs over a whole part of K rounds worse: u8 28672
+// -> 1024 at 24 rows 2.4e-7 from 64 bits against 0.9e-7, the small-batch kernel 1.2e-7.  It was 3 % faster at 33-48 rows,
+// 1 % up to 16; a wait for the matrix cores after every k-block would cost 4 % and 1 %.)  Split parts are parked with
+// device-scope stores and added by the last to arrive, always in the same order, four at a time.
 #include "device_common.h"
 
 namespace ovfcc {
@@ -179,15 +180,17 @@ __device__ __forceinline__ void stream_body(const StreamItem& it, const StreamSh
 
     auto consume = [&](int buf, const Slot& q) {
         const half_t* xs = &stage_lds[buf][col * SR_PITCH + 8 * kq];
+        // one scale per channel: both k-blocks' sums first, so that the additions wait for the matrix cores once
+        float4_t sums[MODE == 0 ? 2 : 1][MT];
 #pragma unroll
         for (int b = 0; b < 2; ++b) {
+            auto& part = sums[MODE == 0 ? b : 0];
 #pragma unroll
             for (int gi = 0; gi < GPB; ++gi) {
                 float zpv = zp_uniform;
                 if constexpr (ZP_TABLE)
                     zpv = (float)(MODE == 0 ? chan_zp & 0xFFu : (q.zp[b] >> (8 * gi)) & 0xFFu);
                 const half2_t off = splat(1024.f + zpv), off_hi = splat(64.f + zpv);
-                float4_t part[MT];
 #pragma unroll
                 for (int t = 0; t < MT; ++t)
                     part[t] = float4_t{0.f, 0.f, 0.f, 0.f};
@@ -203,17 +206,18 @@ __device__ __forceinline__ void stream_body(const StreamItem& it, const StreamSh
                         part[t] = __builtin_amdgcn_mfma_f32_16x16x32_f16(
                             *reinterpret_cast<const half8_t*>(xs + 16 * t * SR_PITCH + b * kBlockK + 32 * j), f.v, part[t], 0, 0, 0);
                 }
-                if constexpr (MODE == 0) {
-#pragma unroll
-                    for (int t = 0; t < MT; ++t)
-                        acc[t] += part[t];
-                } else {
+                if constexpr (MODE != 0) {
                     const float scale = (float)__builtin_bit_cast(half_t, (uint16_t)(q.scale[b][gi >> 1] >> (16 * (gi & 1))));
 #pragma unroll
                     for (int t = 0; t < MT; ++t)
                         acc[t] += scale * part[t];
                 }
             }
+        }
+        if constexpr (MODE == 0) {
+#pragma unroll
+            for (int t = 0; t < MT; ++t)
+                acc[t] += sums[0][t] + sums[1][t];
         }
     };
 
