@@ -45,6 +45,10 @@
 // MFMA roles: A = weights (rows = channels), B = activations (columns = rows m of X); result lane holds
 // column m = lane & 15, channels 4 (lane >> 4) + r, so a lane stores four consecutive outputs of one row.
 //
+// A node that ends on half a tile (N an odd multiple of 128) multiplies zeros for the channels that are not there:
+// their weight loads have no range, two of the four wave columns store nothing (block of 4224 / 1024 / 11008, u4 in
+// groups of 64, 371 rows: 594 us with the square kernel, which ran such nodes before, 251 here).
+//
 // Weights: (q - zp) * s rounded once to f16 for grouped scales; with one group per channel the exact
 // integers q - zp go to the matrix cores and the scale multiplies the f32 result.
 #include "device_common.h"
@@ -110,18 +114,19 @@ __device__ __forceinline__ void prefill_async_body(const uint4_t* __restrict__ w
     // advances with the k-block is uniform and travels in the scalar operand, which is not checked -- a load for a
     // k-block past kb_hi uses a descriptor of length zero instead.  That keeps the loop free of vector address
     // arithmetic.
-    const int nt0 = n0 / 16;  // the workgroup's 16 channel tiles
+    const int nt0 = n0 / 16;                // the workgroup's 16 channel tiles,
+    const int nts = min(16, N / 16 - nt0);  // eight of them in the last column of a node that ends on half a tile
+    const int w_len = 2 * wave < nts ? 16 * kb_total * kTileBytes : 0;  // (the tiles 2 wave, 2 wave + 1 that the wave copies)
     auto live = [&](int kb, int bytes) { return kb < kb_hi ? bytes : 0; };
 #define PA_DESC_X(kb) \
     __builtin_amdgcn_make_buffer_rsrc(const_cast<half_t*>(x), 0, live(kb, (row_map ? x_rows : M) * K * 2), kRsrcFlags)
-#define PA_DESC_W(kb)                                                                                  \
-    __builtin_amdgcn_make_buffer_rsrc(const_cast<uint4_t*>(wt + (size_t)nt0 * kb_total * 64), 0,        \
-                                      live(kb, 16 * kb_total * kTileBytes), kRsrcFlags)
+#define PA_DESC_W(kb) \
+    __builtin_amdgcn_make_buffer_rsrc(const_cast<uint4_t*>(wt + (size_t)nt0 * kb_total * 64), 0, live(kb, w_len), kRsrcFlags)
 #define PA_DESC_S(kb) \
-    __builtin_amdgcn_make_buffer_rsrc(const_cast<half_t*>(st + (size_t)nt0 * ng * 16), 0, live(kb, 16 * ng * 32), kRsrcFlags)
+    __builtin_amdgcn_make_buffer_rsrc(const_cast<half_t*>(st + (size_t)nt0 * ng * 16), 0, live(kb, nts * ng * 32), kRsrcFlags)
 #define PA_DESC_Z(kb)                                                                                       \
     __builtin_amdgcn_make_buffer_rsrc(const_cast<uint8_t*>(ZP_TABLE ? zt + (size_t)nt0 * ng * 16 : zt), 0, \
-                                      ZP_TABLE ? live(kb, 16 * ng * 16) : 0, kRsrcFlags)
+                                      ZP_TABLE ? live(kb, nts * ng * 16) : 0, kRsrcFlags)
     const unsigned g_mul = kb_per_group == 1 ? 0u : (unsigned)((0x100000000ull + kb_per_group - 1) / kb_per_group);
 
     // ---- activations: direct-to-LDS load i of the wave covers rows 4 AL wave + 4 i .. +3 of the tile (AL loads per
@@ -476,7 +481,7 @@ static int allow_lds(Kern kern, bool* done, unsigned bytes) {
 // remaining tile, parts that cover K.
 static bool async_plan_ok(const FcDeviceArgs& a, const LaunchPlan& p) {
     const int64_t tiles = (int64_t)p.tiles_x * p.tiles_y;
-    return (p.tile_m == 128 || p.tile_m == 96 || p.tile_m == 80 || p.tile_m == 64) && p.tiles_x == a.N / PA_BN && p.tiles_y >= 1 && p.full_tiles >= 0 && p.full_tiles <= tiles && p.split_k >= 1 &&
+    return (p.tile_m == 128 || p.tile_m == 96 || p.tile_m == 80 || p.tile_m == 64) && p.tiles_x == (a.N + PA_BN - 1) / PA_BN && a.N % (PA_BN / 2) == 0 && p.tiles_y >= 1 && p.full_tiles >= 0 && p.full_tiles <= tiles && p.split_k >= 1 &&
            (int64_t)p.kblocks_per_split * p.split_k >= a.layout.k_blocks && (p.full_tiles == tiles || p.kblocks_per_split >= 1) &&
            p.grid[0] == (unsigned)(p.full_tiles + (tiles - p.full_tiles) * p.split_k) && p.grid[1] == 1 && p.grid[2] == 1 &&
            (p.split_k == 1 || (a.workspace && a.counters));

@@ -65,13 +65,14 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1))) voi
     constexpr int kRsrcFlags = 0x00020000;
     // Every offset goes through the vector operand: the scalar offset of a buffer load is not range-checked.
     const __amdgpu_buffer_rsrc_t rx = __builtin_amdgcn_make_buffer_rsrc(const_cast<half_t*>(x), 0, M * K * 2, kRsrcFlags);
-    const int nt0 = n0 / 16 + 4 * wave;  // the wave's four channel tiles
+    const int nt0 = n0 / 16 + 4 * wave;  // the wave's four channel tiles,
+    const int nts = n0 + 64 * wave < N ? 4 : 0;  // none where the node ends on half a tile
     const __amdgpu_buffer_rsrc_t rw = __builtin_amdgcn_make_buffer_rsrc(
-        const_cast<uint4_t*>(wt + (size_t)nt0 * kb_total * 64), 0, 4 * kb_total * kTileBytes, kRsrcFlags);
+        const_cast<uint4_t*>(wt + (size_t)nt0 * kb_total * 64), 0, nts * kb_total * kTileBytes, kRsrcFlags);
     const __amdgpu_buffer_rsrc_t rs =
-        __builtin_amdgcn_make_buffer_rsrc(const_cast<half_t*>(st + (size_t)nt0 * ng * 16), 0, 4 * ng * 32, kRsrcFlags);
+        __builtin_amdgcn_make_buffer_rsrc(const_cast<half_t*>(st + (size_t)nt0 * ng * 16), 0, nts * ng * 32, kRsrcFlags);
     const __amdgpu_buffer_rsrc_t rz = __builtin_amdgcn_make_buffer_rsrc(
-        const_cast<uint8_t*>(ZP_TABLE ? zt + (size_t)nt0 * ng * 16 : zt), 0, ZP_TABLE ? 4 * ng * 16 : 0, kRsrcFlags);
+        const_cast<uint8_t*>(ZP_TABLE ? zt + (size_t)nt0 * ng * 16 : zt), 0, ZP_TABLE ? nts * ng * 16 : 0, kRsrcFlags);
     const unsigned g_mul = kb_per_group == 1 ? 0u : (unsigned)((0x100000000ull + kb_per_group - 1) / kb_per_group);
 
     // ---- activations: load i of the wave fills rows 64 wave + 8 i .. +7 of a stage; lane -> row 8 i + (lane >> 3)
@@ -306,6 +307,8 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1))) voi
     asm volatile("s_nop 15\n\ts_nop 15" ::: "memory");
 
     // ---- epilogue: per-channel scale, bias, gated linear unit, stores ----
+    if (nts == 0)
+        return;  // (no barrier from here on)
     auto channel_params = [&](int r, float (&sc)[4], float (&bs)[4]) {
         const int n = n0 + 64 * wave + 16 * r + 4 * kq;
 #pragma unroll
@@ -422,8 +425,8 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1))) voi
 // The launch must be what the kernel assumes: a 1-D grid of whole 256 x 256 tiles.
 static bool big_plan_ok(const FcDeviceArgs& a, const LaunchPlan& p) {
     const Layout& L = a.layout;
-    return L.tiled && L.bits == 4 && L.groups_per_kblock == 1 && a.N % PB_BN == 0 && p.tile_m == PB_BM &&
-           p.tile_n == PB_BN && p.tiles_x == a.N / PB_BN && p.tiles_y >= 1 && (int64_t)p.tiles_y * PB_BM >= a.M &&
+    return L.tiled && L.bits == 4 && L.groups_per_kblock == 1 && a.N % (PB_BN / 2) == 0 && p.tile_m == PB_BM &&
+           p.tile_n == PB_BN && p.tiles_x == (a.N + PB_BN - 1) / PB_BN && p.tiles_y >= 1 && (int64_t)p.tiles_y * PB_BM >= a.M &&
            p.split_k == 1 && p.full_tiles == p.tiles_x * p.tiles_y && p.grid[0] == (unsigned)(p.tiles_x * p.tiles_y) &&
            p.grid[1] == 1 && p.grid[2] == 1 && p.block == 256 && a.M * a.K * 2 < ((int64_t)1 << 31) &&
            (int64_t)4 * L.k_blocks * kTileBytes < ((int64_t)1 << 31);

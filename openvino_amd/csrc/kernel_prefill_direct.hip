@@ -81,13 +81,14 @@ __global__ __launch_bounds__(512) void fcc_prefill_direct_kernel(const uint4_t* 
     constexpr int kRsrcFlags = 0x00020000;
     // Every offset goes through the vector operand: the scalar offset of a buffer load is not range-checked.
     const __amdgpu_buffer_rsrc_t rx = __builtin_amdgcn_make_buffer_rsrc(const_cast<half_t*>(x), 0, M * K * 2, kRsrcFlags);
-    const int nt0 = n0 / 16 + 4 * wn;  // the wave's four channel tiles
+    const int nt0 = n0 / 16 + 4 * wn;  // the wave's four channel tiles,
+    const int nts = n0 + 64 * wn < N ? 4 : 0;  // none where the node ends on half a tile
     const __amdgpu_buffer_rsrc_t rw = __builtin_amdgcn_make_buffer_rsrc(
-        const_cast<uint4_t*>(wt + (size_t)nt0 * kb_total * TPB * 64), 0, 4 * kb_total * TPB * kTileBytes, kRsrcFlags);
+        const_cast<uint4_t*>(wt + (size_t)nt0 * kb_total * TPB * 64), 0, nts * kb_total * TPB * kTileBytes, kRsrcFlags);
     const __amdgpu_buffer_rsrc_t rs =
-        __builtin_amdgcn_make_buffer_rsrc(const_cast<half_t*>(st + (size_t)nt0 * ng * 16), 0, 4 * ng * 32, kRsrcFlags);
+        __builtin_amdgcn_make_buffer_rsrc(const_cast<half_t*>(st + (size_t)nt0 * ng * 16), 0, nts * ng * 32, kRsrcFlags);
     const __amdgpu_buffer_rsrc_t rz = __builtin_amdgcn_make_buffer_rsrc(
-        const_cast<uint8_t*>(ZP_TABLE ? zt + (size_t)nt0 * ng * 16 : zt), 0, ZP_TABLE ? 4 * ng * 16 : 0, kRsrcFlags);
+        const_cast<uint8_t*>(ZP_TABLE ? zt + (size_t)nt0 * ng * 16 : zt), 0, ZP_TABLE ? nts * ng * 16 : 0, kRsrcFlags);
     const unsigned g_mul = kb_per_group == 1 ? 0u : (unsigned)((0x100000000ull + kb_per_group - 1) / kb_per_group);
 
     // ---- activations: direct-to-LDS load i of the wave covers rows 16 wave + 4 i .. +3 of the tile; lane ->
@@ -316,7 +317,7 @@ int launch_prefill_direct(const FcDeviceArgs& a, const LaunchPlan& p, void* stre
     const int64_t tiles = (int64_t)p.tiles_x * p.tiles_y;
     if (L.groups_per_kblock != 1)
         return (int)hipErrorInvalidValue;  // groups below 128 inputs: the planner picks another kernel
-    if (p.tile_m != PD_BM || p.tiles_x != a.N / PD_BN || (int64_t)p.tiles_y * PD_BM < a.M || p.full_tiles < 0 ||
+    if (p.tile_m != PD_BM || p.tiles_x != (a.N + PD_BN - 1) / PD_BN || a.N % (PD_BN / 2) != 0 || (int64_t)p.tiles_y * PD_BM < a.M || p.full_tiles < 0 ||
         p.full_tiles > tiles || p.split_k < 1 || (int64_t)p.kblocks_per_split * p.split_k < L.k_blocks ||
         p.grid[0] != (unsigned)(p.full_tiles + (tiles - p.full_tiles) * p.split_k) || p.grid[1] != 1 || p.grid[2] != 1 ||
         (p.split_k > 1 && !(a.workspace && a.counters)))

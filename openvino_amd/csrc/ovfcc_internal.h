@@ -158,6 +158,7 @@ struct LaunchPlan {
     bool x_in_lds = false;      // decode kernel: activations staged in LDS
     bool direct = false;        // prefill family: the kernels that feed weights from registers
     bool async_dma = false;     // ... and of those the one whose operands all travel by direct-to-LDS loads
+    bool fills = false;         // ... and whether their grid covers half the chip
     bool big = false;           // prefill family: the 4-bit kernel with 256 x 256 tiles (whole tiles, no split-K)
     bool batch = false;         // decode family: the small-batch kernel (waves own channel tiles)
     bool gemv = false;          // decode family: the matrix-vector kernel for M <= 4 (4-bit weights, G = 128)

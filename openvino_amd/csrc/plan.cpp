@@ -407,28 +407,37 @@ int plan_launch(const FcDeviceArgs& a, int force_kernel, int force_split, int n_
         p.dynamic_lds = (unsigned)((size_t)nw * rt * mt * 256 * sizeof(float) + (xlds ? x_bytes : 0));
         p.name = L.bits == 4 ? "fcc_decode_w4" : "fcc_decode_w8";
     } else {
-        // The kernels with 128 x 256 tiles run when their grid still gives every second compute unit a tile;
-        // otherwise, or when N is not a multiple of 256, the square kernel's smaller tiles spread the work
-        // further.  Of the two, the register-fed kernel is the faster one; the LDS-dequantising one also needs
+        // The register-fed kernels with 256-channel tiles run whatever they can, however small the launch: they split K and
+        // keep their loads in flight, where the square kernel waits for every k-block (u4 in groups of 128, 129 rows:
+        // 2048 -> 2048 40.8 us there against 18.7, 14336 -> 512 268 / 27; u8 2048 -> 2048 40.7 / 27.2).  Nodes under 256 KiB,
+        // which would gain too (512 -> 256 16.5 / 9.8), stay: they are what calls the square kernel by default.
+        // A grouped run shares a launch only where that covers half the chip (its other slices run one by one), and
+        // p.fills tells a caller that could cut the rows into decode launches.  The LDS-dequantising kernel also needs
         // K % 256 == 0.  OVFCC_PREFILL_WIDE = 0 | 1 and OVFCC_PREFILL_DIRECT = 0 | 1 override for experiments.
         const int64_t m_tiles = (a.M + kPrefillTileM - 1) / kPrefillTileM;
         const int tiles_per_kb = L.bits == 4 ? 1 : 2;
-        const bool direct_ok = (a.N % kPrefillWideN) == 0 && a.M * a.K * 2 < ((int64_t)1 << 31) &&
+        // The register-fed kernels also run nodes that end on half a tile (its other half multiplies zeros: 1 / 46 of the
+        // work at N = 5760), except grouped launches.  A node of half a tile only stays with the square kernel.
+        const bool whole = (a.N % kPrefillWideN) == 0;
+        const bool direct_ok = (whole || ((a.N % kPrefillTileN) == 0 && a.N > kPrefillWideN && a.tile_rows == 0 && !a.want_async)) &&
+                               a.M * a.K * 2 < ((int64_t)1 << 31) &&
                                (int64_t)16 * L.k_blocks * tiles_per_kb * kTileBytes < ((int64_t)1 << 31);
-        const bool wide_ok = direct_ok && (a.K % 256) == 0;
+        const bool wide_ok = direct_ok && whole && (a.K % 256) == 0;
+        const int64_t n_wide = (a.N + kPrefillWideN - 1) / kPrefillWideN;
         // (the register-fed kernels can also split K, which multiplies their grid by up to eight)
         const bool may_split = direct_ok && env_int("OVFCC_PREFILL_DIRECT", 1) != 0;
         const bool may_async = may_split && L.bits == 4 && env_int("OVFCC_PREFILL_ASYNC", 1) != 0;
         // (and the 4-bit one has a form with 64-row tiles, which doubles the tile count of a grid that fits one round)
-        int64_t reach = (a.N / kPrefillWideN) * m_tiles;
+        int64_t reach = n_wide * m_tiles;
         if (may_split) {
-            const int64_t tiles64 = (a.N / kPrefillWideN) * ((a.M + 63) / 64);
+            const int64_t tiles64 = n_wide * ((a.M + 63) / 64);
             if (may_async && tiles64 <= n_cus)
                 reach = tiles64;
             for (int split = 1; split < 8 && reach * 2 <= n_cus && L.k_blocks / (split * 2) >= 8; split *= 2)
                 reach *= 2;
         }
-        bool big = reach * 2 >= n_cus || (a.want_async && may_async);
+        p.fills = reach * 2 >= n_cus;
+        bool big = p.fills || (a.want_async && may_async) || (a.tile_rows == 0 && may_split && L.w_bytes >= ((size_t)256 << 10));
         const int wide_env = env_int("OVFCC_PREFILL_WIDE", -1);
         if (wide_env >= 0)
             big = wide_env != 0;
@@ -441,7 +450,7 @@ int plan_launch(const FcDeviceArgs& a, int force_kernel, int force_split, int n_
         p.async_dma = p.direct && L.bits == 4 && env_int("OVFCC_PREFILL_ASYNC", 1) != 0;
         p.tile_m = kPrefillTileM;
         p.tile_n = wide ? kPrefillWideN : kPrefillTileN;
-        p.grid[0] = (unsigned)(a.N / p.tile_n);
+        p.grid[0] = (unsigned)(wide ? n_wide : a.N / kPrefillTileN);
         p.grid[1] = (unsigned)m_tiles;
         if (p.async_dma) {
             // 64-row tiles while they still fit the compute units in one round: a 64-row tile takes two thirds of
@@ -507,7 +516,7 @@ int plan_launch(const FcDeviceArgs& a, int force_kernel, int force_split, int n_
         // the kernel can run the node).  A grouped run (a.tile_rows set) keeps its one row tile per slice.
         if (p.async_dma && p.split_k == 1 && p.tile_m == kPrefillTileM && L.groups_per_kblock == 1 && force_split <= 0 &&
             a.tile_rows == 0) {
-            const int64_t big_tiles = (a.N / kPrefillWideN) * ((a.M + 255) / 256);
+            const int64_t big_tiles = n_wide * ((a.M + 255) / 256);
             const int64_t big_rounds = (big_tiles + n_cus - 1) / n_cus;
             const int64_t small_rounds = ((int64_t)p.tiles_x * p.tiles_y + n_cus - 1) / n_cus;
             const int big_env = env_int("OVFCC_PREFILL_BIG", -1);

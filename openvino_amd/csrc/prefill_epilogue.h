@@ -82,6 +82,10 @@ __device__ __forceinline__ void split_k_last_arrival(const __amdgpu_buffer_rsrc_
     __syncthreads();
     if (ticket_s != (unsigned)(split_k - 1))
         return;
+    if (tid == 0)  // (everyone has arrived: nobody draws from it any more)
+        __hip_atomic_store(counters + tile_id, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    if (n0 + 64 * wn >= N)
+        return;  // the node ends on half a tile
     // Last arrival: every wave adds up two of its k-group pair's four channel tiles (k-group kg takes tiles 2 kg and
     // 2 kg + 1 -- a gate tile and its up tile), all row tiles, parts in ascending order.  The loads of two parts,
     // 2 x 2 NT of them, are in flight together (a part index past split_k falls outside the descriptor's range
@@ -132,8 +136,6 @@ __device__ __forceinline__ void split_k_last_arrival(const __amdgpu_buffer_rsrc_
             for (int r2 = 0; r2 < 2; ++r2)
                 finish(2 * kg + r2, t, sum[r2][t], sc[r2], bs[r2]);
     }
-    if (tid == 0)
-        __hip_atomic_store(counters + tile_id, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
 // k-group 1 -> k-group 0 through LDS, two channel tiles at a time.  Without split-K k-group 0
@@ -229,7 +231,9 @@ __device__ __forceinline__ void tile_epilogue(float4_t (&acc)[4][NT], unsigned c
                 }
         }
         __syncthreads();
-        if (kg == 0 && glu && split_k == 1) {
+        if (n0 + 64 * wn >= N) {
+            // the node ends on half a tile
+        } else if (kg == 0 && glu && split_k == 1) {
             float scg[4], bsg[4], scu[4], bsu[4];
             channel_params(2 * hh, scg, bsg);
             channel_params(2 * hh + 1, scu, bsu);
@@ -333,6 +337,8 @@ __device__ __forceinline__ void tile_epilogue_shared(float4_t (&acc)[4][NT], uns
                 mine[(r * T0 + i) * 64] = acc[r][SLO + i];
     };
     auto run = [&](auto kg_const) {
+        if (n0 + 64 * wn >= N)
+            return;  // the node ends on half a tile
         constexpr int KG = decltype(kg_const)::value;
         constexpr int LO = KG == 0 ? 0 : T0, CNT = KG == 0 ? T0 : NT - T0;
         const float4_t* theirs = ex + (size_t)((wave ^ 4) * 4 * T0) * 64 + lane;
