@@ -178,13 +178,18 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1))) voi
     auto x_at = [&](int stage, int n) {
         return *(lds_frag_ptr)(lds3 + stage * PB_STAGE_BYTES + ((n & 15) * 16 + col) * 128 + ((((n >> 4) * 4 + kq) ^ x_sw) << 4));
     };
+    // Row tiles take the channel tiles there and back again (0 1 2 3, 3 2 1 0): from one MFMA to the next only one of the
+    // two operands changes, and a chip at its power limit pays for every operand bit that does.  A loop of nothing but
+    // MFMAs on random halves (4 x 8 accumulator tiles, two waves per SIMD) runs 1 388 TFLOP/s starting over and 1 456
+    // this way; here it is worth 0.8 % (8B block, 2048 rows: 779 -> 773 us).  The 128-row kernels, which are not at that
+    // limit, do not gain (117 rows: 108.8 / 109.7).  The sums are the same.
     auto half = [&](int stage, Frag8 (&wa)[4], Frag8 (&wb)[4], const WSlot& sa, int ja, WSlot& sb, int jb,
                     auto&& sync_next, auto&& mem) {
         auto slot = [&](int i) {
-            const int tt = i >> 2, r = i & 3;  // tt = 16 js + t
+            const int tt = i >> 2, r = (tt & 1) ? 3 - (i & 3) : i & 3;  // tt = 16 js + t
             if (i == PB_SYNC_SLOT)
                 sync_next();  // the next half's activations are in LDS for every wave
-            if (r == 0) {
+            if ((i & 3) == 0) {
                 constexpr int ahead = PB_XQ - 1;
                 xq[(tt + ahead) % PB_XQ] = tt + ahead < 32 ? x_at(stage, tt + ahead) : x_at((stage + 1) & 3, tt + ahead - 32);
             }
