@@ -16,17 +16,16 @@
 //                           unpacked once per 64 rows and an activation operand read from LDS meets four MFMAs
 //                           (half of what LDS delivers at the matrix cores' rate; waves side by side along N would
 //                           need all of it).  Three workgroups share a compute unit and hide each other's loads,
-//                           which travel two k-blocks ahead through registers: where K is no multiple of eight, rows
-//                           start anywhere and a direct-to-LDS load, which wants 16-byte pieces, cannot fetch them
-//                           (other K could; that form is not built).  577 x 1160 -> 3480 (552 tiles) takes
-//                           18 us (21 under the tracer): 8 of launch, first loads and epilogue, then 1 us per k-block
-//                           against 0.3 of matrix-core work (their pipe is busy 19 % of the launch by the counter;
-//                           a third of the waves' cycles are waits); a third workgroup on some compute units and
-//                           two on the others make the rest.
+//                           which travel two k-blocks ahead through registers: rows may start anywhere.
+//   fcc_ragged_tile_dma_kernel  the same tiles where rows start at dwords: the activations go to LDS without registers
+//                           or LDS stores.  577 x 1160 -> 3480 (552 tiles) 18.1 -> 15.2 us, 1160 -> 4300 18.4 -> 15.7, 4300
+//                           -> 1160 23.2 -> 18.9, 1500 x 1600 -> 4800 51.5 -> 46.1; a k-block of three workgroups takes 0.97 us
+//                           against 0.32 of matrix-core work: 32 load instructions a workgroup, 16 cycles of the
+//                           address path each, are 0.64.  A fourth stage leaves room for two workgroups only (17.8).
 // What a load costs the compute unit is the number of 64-byte pieces its 64 lanes name in lane order: weights read
 // where OpenVINO left them (neighbouring lanes in different rows) kept the cache's tag stage busy every cycle of the
 // launch -- 577 x 4640 -> 3480 took 61.6 us that way and takes 42.1 in operand order.
-// An encoder layer of hidden size 1160 (four nodes, 577 rows) takes 75 us where one wave per output took 7 850.
+// An encoder layer of hidden size 1160 (four nodes, 577 rows) takes 64 us where one wave per output took 7 850.
 #include <atomic>
 
 #include "device_common.h"
@@ -37,6 +36,7 @@ namespace {
 
 constexpr int RG_BM = kRaggedTile, RG_BN = kRaggedTile, RG_PITCH = kRaggedPitch;
 constexpr int RG_STAGE_HALVES = RG_BM * RG_PITCH;
+constexpr int RD_STAGES = 3;
 
 template <class T>
 __device__ __forceinline__ T load_unaligned(const void* p) {
@@ -169,6 +169,52 @@ __device__ __forceinline__ void finish4(const RaggedNode& a, int m, int n, float
     const float v[4] = {sum.x * (float)p.scale[0] + (float)p.bias[0], sum.y * (float)p.scale[1] + (float)p.bias[1],
                         sum.z * (float)p.scale[2] + (float)p.bias[2], sum.w * (float)p.scale[3] + (float)p.bias[3]};
     store4(a, m, n, v);
+}
+
+// The end of a 64 x 64 tile: out[r] holds channel tile r of row tile `wave` over this part of K.
+__device__ __forceinline__ void finish_tile(const RaggedNode& a, float* __restrict__ ws, unsigned* __restrict__ counters, int tile,
+                                            int split, int part, int m0, int n0, float4_t (&out)[4],
+                                            const ChannelParams (&params)[4], unsigned* ticket) {
+    const int lane = threadIdx.x & 63, col = lane & 15, kq = lane >> 4;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    if (split > 1) {
+        // partial tiles are parked with device-scope stores; the last part to arrive adds them in order
+        constexpr int kAuxDeviceScope = 16;
+        constexpr unsigned kTileFloats = RG_BM * RG_BN;
+        const __amdgpu_buffer_rsrc_t rp = __builtin_amdgcn_make_buffer_rsrc(ws + (size_t)tile * split * kTileFloats, 0,
+                                                                            split * (int)(kTileFloats * 4), 0x00020000);
+        const unsigned mine = (unsigned)(wave * 64 + lane) * 16u;
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+            __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(uint4_t, out[i]), rp,
+                                                   (unsigned)part * (kTileFloats * 4) + i * 4096u + mine, 0, kAuxDeviceScope);
+        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+        __syncthreads();
+        if (threadIdx.x == 0)
+            *ticket = __hip_atomic_fetch_add(counters + tile, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        __syncthreads();
+        if (*ticket != (unsigned)(split - 1))
+            return;
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+            out[i] = float4_t{0.f, 0.f, 0.f, 0.f};
+        for (int z = 0; z < split; ++z) {
+            float4_t v[4];
+#pragma unroll
+            for (int i = 0; i < 4; ++i)
+                v[i] = __builtin_bit_cast(float4_t, __builtin_amdgcn_raw_buffer_load_b128(
+                                                        rp, (unsigned)z * (kTileFloats * 4) + i * 4096u + mine, 0, kAuxDeviceScope));
+#pragma unroll
+            for (int i = 0; i < 4; ++i)
+                out[i] += v[i];
+        }
+        if (threadIdx.x == 0)
+            __hip_atomic_store(counters + tile, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    }
+
+#pragma unroll
+    for (int r = 0; r < 4; ++r)
+        finish4(a, m0 + 16 * wave + col, n0 + 16 * r + 4 * kq, out[r], params[r]);
 }
 
 }  // namespace
@@ -402,44 +448,185 @@ __global__ __launch_bounds__(256) void fcc_ragged_tile_kernel(RaggedNode a, int 
         }
     }
 
-    if (split > 1) {
-        // partial tiles are parked with device-scope stores; the last part to arrive adds them in order
-        constexpr int kAuxDeviceScope = 16;
-        constexpr unsigned kTileFloats = RG_BM * RG_BN;
-        const __amdgpu_buffer_rsrc_t rp = __builtin_amdgcn_make_buffer_rsrc(ws + (size_t)tile * split * kTileFloats, 0,
-                                                                            split * (int)(kTileFloats * 4), 0x00020000);
-        const unsigned mine = (unsigned)(wave * 64 + lane) * 16u;
-#pragma unroll
-        for (int r = 0; r < 4; ++r)
-            __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(uint4_t, out[r]), rp,
-                                                   (unsigned)part * (kTileFloats * 4) + r * 4096u + mine, 0, kAuxDeviceScope);
-        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-        __syncthreads();
-        if (threadIdx.x == 0)
-            ticket_s = __hip_atomic_fetch_add(counters + tile, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        __syncthreads();
-        if (ticket_s != (unsigned)(split - 1))
-            return;
-#pragma unroll
-        for (int r = 0; r < 4; ++r)
-            out[r] = float4_t{0.f, 0.f, 0.f, 0.f};
-        for (int z = 0; z < split; ++z) {
-            float4_t v[4];
-#pragma unroll
-            for (int r = 0; r < 4; ++r)
-                v[r] = __builtin_bit_cast(float4_t, __builtin_amdgcn_raw_buffer_load_b128(
-                                                        rp, (unsigned)z * (kTileFloats * 4) + r * 4096u + mine, 0, kAuxDeviceScope));
-#pragma unroll
-            for (int r = 0; r < 4; ++r)
-                out[r] += v[r];
-        }
-        if (threadIdx.x == 0)
-            __hip_atomic_store(counters + tile, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    }
+    finish_tile(a, ws, counters, tile, split, part, m0, n0, out, params, &ticket_s);
+}
 
+// The same tiles where rows hold an even number of halves and begin at a multiple of four bytes: the activations travel to
+// LDS by direct-to-LDS loads (RD_STAGES stages of 256-byte rows, the sixteen 16-byte chunks of row r at chunk ^ (r & 15)),
+// the weights to registers two k-blocks ahead.  A load's pieces start at any multiple of four bytes and stay inside their
+// row or, past its end, inside the activations; what they hold of the next row is set to zero when the last k-block's
+// operands are read.  Rows past M and k-blocks past the end lie beyond the descriptor's range and arrive as zeros.
+template <int BITS>
+__global__ __launch_bounds__(256, 3) void fcc_ragged_tile_dma_kernel(RaggedNode a, int kb_total, int tiles_m, int tiles,
+                                                                     int split, int kb_per_split, float* __restrict__ ws,
+                                                                     unsigned* __restrict__ counters) {
+    constexpr int NT = 4, A_BYTES = RG_BM * 256, STAGES = RD_STAGES;
+    constexpr int AL = 4;  // direct-to-LDS loads per wave and k-block, four rows each
+    constexpr int WD = BITS / 4, kStep = 64 * 4 * WD;
+    extern __shared__ __attribute__((aligned(16))) unsigned char lds[];
+    __shared__ unsigned ticket_s;
+    const lds_byte_ptr lds3 = (lds_byte_ptr)lds;
+    const int lane = threadIdx.x & 63, col = lane & 15, kq = lane >> 4;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int run = (tiles + 7) >> 3;  // tiles of an XCD, as in the kernel above
+    // (divisions and minima run on the vector ALU; told to be the same in every lane, they leave the descriptors below
+    // scalar: else each buffer load sits in a loop that looks for lanes with equal ones)
+    const int part = __builtin_amdgcn_readfirstlane((int)((blockIdx.x >> 3) / run));
+    const int tile = (int)(blockIdx.x & 7) * run + (int)(blockIdx.x >> 3) - part * run;
+    if (tile >= tiles)
+        return;
+    const int column = __builtin_amdgcn_readfirstlane(tile / tiles_m);
+    const int n0 = column * RG_BN, m0 = (tile - column * tiles_m) * RG_BM;
+    const int kb_lo = part * kb_per_split, kb_hi = min(kb_total, kb_lo + kb_per_split);
+
+    constexpr unsigned kOob = 0x80000000u;
+    constexpr int kRsrcFlags = 0x00020000;
+    // (every offset goes through the vector operand: the scalar offset of a buffer load is not range-checked)
+    const __amdgpu_buffer_rsrc_t rx = __builtin_amdgcn_make_buffer_rsrc(const_cast<half_t*>(a.x), 0, a.M * a.K * 2, kRsrcFlags);
+    const int nt0 = n0 / 16;  // channel tiles past the last one have no range
+    const int nts = __builtin_amdgcn_readfirstlane(max(0, min(4, (a.N + 15) / 16 - nt0)));
+    const __amdgpu_buffer_rsrc_t rw = __builtin_amdgcn_make_buffer_rsrc(
+        const_cast<void*>(uniform_ptr(a.w + (size_t)nt0 * kb_total * 4 * kStep)), 0, nts * kb_total * 4 * kStep, kRsrcFlags);
+    unsigned a_voff[AL];
+#pragma unroll
+    for (int i = 0; i < AL; ++i) {
+        const int r0 = 4 * AL * wave + 4 * i;
+        a_voff[i] = (unsigned)(m0 + r0 + kq) * (unsigned)a.K * 2u + ((unsigned)(col ^ kq ^ (r0 & 15)) << 4);
+    }
+    const unsigned w_voff = (unsigned)(wave * kStep + lane * 4 * WD);
+    auto dma_x = [&](int kb, int s) {
+#pragma unroll
+        for (int i = 0; i < AL; ++i) {
+            unsigned at = a_voff[i] + (unsigned)(kb * 256);
+            if (kb == kb_total - 1) {  // the piece that crosses the row's end holds the row's last eight inputs instead
+                const int past = kb * kBlockK + 8 * (col ^ kq ^ ((4 * AL * wave + 4 * i) & 15)) - (a.K - 8);
+                at -= past > 0 && past < 8 ? 2u * past : 0u;
+            }
+            __builtin_amdgcn_raw_ptr_buffer_load_lds(rx, (lds_void_ptr)(lds3 + s * A_BYTES + (AL * wave + i) * 1024), 16,
+                                                     kb < kb_hi ? at : kOob, 0, 0, 0);
+        }
+    };
+    uint32_t w[2][4][WD];
+    auto load_w = [&](int kb, uint32_t(&d)[4][WD]) {
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+            const unsigned at = kb < kb_hi ? w_voff + (unsigned)((r * kb_total + kb) * 4 * kStep) : kOob;
+            if constexpr (BITS == 8) {
+                const uint2_t v = __builtin_bit_cast(uint2_t, __builtin_amdgcn_raw_buffer_load_b64(rw, at, 0, 0));
+                d[r][0] = v.x, d[r][1] = v.y;
+            } else {
+                d[r][0] = __builtin_amdgcn_raw_buffer_load_b32(rw, at, 0, 0);
+            }
+        }
+    };
+    // (a bare barrier that waits for this wave's LDS accesses only)
+    auto barrier = [&] {
+        __builtin_amdgcn_s_waitcnt(0xC07F);
+        asm volatile("" ::: "memory");
+        __builtin_amdgcn_s_barrier();
+        asm volatile("" ::: "memory");
+    };
+    int n_of[4];
 #pragma unroll
     for (int r = 0; r < 4; ++r)
-        finish4(a, m0 + 16 * wave + col, n0 + 16 * r + 4 * kq, out[r], params[r]);
+        n_of[r] = min(n0 + 16 * r + col, a.N - 1);
+    half2_t off[4], off_hi[4];
+    zero_points<4>(a, n_of, off, off_hi);
+    dma_x(kb_lo, 0);
+    dma_x(kb_lo + 1, 1);
+    load_w(kb_lo, w[0]);
+    load_w(kb_lo + 1, w[1]);
+    float4_t acc[4][NT];  // [channel tile][row tile]
+#pragma unroll
+    for (int r = 0; r < 4; ++r)
+#pragma unroll
+        for (int t = 0; t < NT; ++t)
+            acc[r][t] = float4_t{0.f, 0.f, 0.f, 0.f};
+
+    typedef __attribute__((address_space(3))) const half8_t* lds_frag_ptr;
+    // two k-blocks per trip so that the weight registers are static; one past the end multiplies zeros
+    int s = 0;  // the k-block's stage
+    for (int kb0 = kb_lo; kb0 < kb_hi; kb0 += 2) {
+#pragma unroll
+        for (int u = 0; u < 2; ++u) {
+            const int kb = kb0 + u;
+            // this k-block's activations have landed once no more is out than what was asked for after them: its
+            // weights, activations and weights of the next one
+            __builtin_amdgcn_s_waitcnt(wait_vmcnt_imm(AL + 8));
+            barrier();  // everyone's have; everyone is done with the stage of k-block kb - 1
+            dma_x(kb + STAGES - 1, s == 0 ? STAGES - 1 : s - 1);
+            const lds_byte_ptr xs = lds3 + s * A_BYTES + col * 256 + (((4 * wave + kq) ^ col) << 4);
+            Frag8 xf[NT];
+#pragma unroll
+            for (int t = 0; t < NT; ++t)
+                xf[t].v = *(lds_frag_ptr)(xs + t * 4096);
+            if (kb >= kb_total - 1) {
+                // the row's last k-block: a piece past its end is the next row's, the one across it is moved into place
+                const int past = kb * kBlockK + 32 * wave + 8 * kq - (a.K - 8);
+                int d = past <= 0 ? 0 : min(past, 8) >> 1;  // dwords to move by; 4: nothing is left
+                asm volatile("" : "+v"(d));                 // (a branch around the moves, not selects in every k-block)
+#pragma unroll
+                for (int t = 0; t < NT; ++t)
+#pragma unroll
+                    for (int j = 0; j < 4; ++j) {
+                        uint32_t v = d == 0 ? xf[t].u[j] : 0u;
+#pragma unroll
+                        for (int i = 1; i < 4; ++i)
+                            if (j + i < 4)
+                                v = d == i ? xf[t].u[j + i] : v;
+                        xf[t].u[j] = v;
+                    }
+            }
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+                Frag8 wf;
+                unpack_ragged<BITS>(w[u][r], off[r], off_hi[r], wf);
+#pragma unroll
+                for (int t = 0; t < NT; ++t)
+                    acc[r][t] = __builtin_amdgcn_mfma_f32_16x16x32_f16(wf.v, xf[t].v, acc[r][t], 0, 0, 0);
+            }
+            load_w(kb + 2, w[u]);
+            s = s == STAGES - 1 ? 0 : s + 1;
+        }
+    }
+    ChannelParams params[4];
+#pragma unroll
+    for (int r = 0; r < 4; ++r)
+        params[r] = channel_params(a, n0 + 16 * r + 4 * kq);
+    __builtin_amdgcn_s_waitcnt(wait_vmcnt_imm(0));  // the loads past the end still target LDS
+    barrier();
+
+    // The four waves' sums over their steps meet in LDS, two channel tiles at a time: wave w finishes row tile w.
+    float4_t* hand = reinterpret_cast<float4_t*>(lds);  // [wave][3][2][64 lanes]: 24 KiB
+    float4_t out[4];
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+        if (h)
+            barrier();
+#pragma unroll
+        for (int t = 0; t < 4; ++t)
+            if (t != wave)
+#pragma unroll
+                for (int r = 0; r < 2; ++r)
+                    hand[((wave * 3 + (t > wave ? t - 1 : t)) * 2 + r) * 64 + lane] = acc[2 * h + r][t];
+        barrier();
+#pragma unroll
+        for (int r = 0; r < 2; ++r) {
+            float4_t v{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+            for (int u = 0; u < 4; ++u)  // in wave order
+                if (u == wave) {
+#pragma unroll
+                    for (int t = 0; t < 4; ++t)
+                        if (t == wave)
+                            v += acc[2 * h + r][t];
+                } else {
+                    v += hand[((u * 3 + (wave > u ? wave - 1 : wave)) * 2 + r) * 64 + lane];
+                }
+            out[2 * h + r] = v;
+        }
+    }
+    finish_tile(a, ws, counters, tile, split, part, m0, n0, out, params, &ticket_s);
 }
 
 // One thread per eight weights of the arranged node.
@@ -478,6 +665,16 @@ int launch_ragged_repack(const ovfcc_fc_desc& d, const Layout& L, const void* w,
     return (int)hipGetLastError();
 }
 
+// More than 64 KiB of LDS has to be asked for, once per kernel (the attribute is idempotent: a race only repeats it).
+static int ask_for_lds(const void* kern, std::atomic<bool>& done, int bytes) {
+    if (done.load(std::memory_order_relaxed))
+        return 0;
+    const hipError_t e = hipFuncSetAttribute(kern, hipFuncAttributeMaxDynamicSharedMemorySize, bytes);
+    if (e == hipSuccess)
+        done.store(true, std::memory_order_relaxed);
+    return (int)e;
+}
+
 int launch_ragged(const FcDeviceArgs& a, const LaunchPlan& p, void* stream) {
     hipStream_t s = static_cast<hipStream_t>(stream);
     const bool four = a.layout.bits == 4;
@@ -497,25 +694,26 @@ int launch_ragged(const FcDeviceArgs& a, const LaunchPlan& p, void* stream) {
             return (int)hipErrorInvalidValue;
         auto kern = p.tile_m == 16 ? (four ? fcc_ragged_rows_kernel<4, 1> : fcc_ragged_rows_kernel<8, 1>)
                                    : (four ? fcc_ragged_rows_kernel<4, 2> : fcc_ragged_rows_kernel<8, 2>);
-        // more than 64 KiB of LDS has to be asked for, once per kernel (the attribute is idempotent: a race only repeats it)
         static std::atomic<bool> asked[2][2] = {};
-        std::atomic<bool>& mine = asked[four ? 0 : 1][p.tile_m == 16 ? 0 : 1];
-        if (!mine.load(std::memory_order_relaxed)) {
-            const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize,
-                                                     16 * ragged_wave_lds(p.tile_m / 16));
-            if (e != hipSuccess)
-                return (int)e;
-            mine.store(true, std::memory_order_relaxed);
-        }
+        if (int e = ask_for_lds(reinterpret_cast<const void*>(kern), asked[four ? 0 : 1][p.tile_m == 16 ? 0 : 1],
+                                16 * ragged_wave_lds(p.tile_m / 16)))
+            return e;
         hipLaunchKernelGGL(kern, grid, block, p.dynamic_lds, s, r, kb);
     } else {
         const int64_t tiles = (int64_t)p.tiles_x * p.tiles_y;
         if ((int64_t)p.tiles_x * RG_BN < a.N || (int64_t)p.tiles_y * RG_BM < a.M ||
             (int64_t)p.split_k * p.kblocks_per_split < kb || p.grid[0] != (unsigned)((tiles + 7) / 8 * 8 * p.split_k))
             return (int)hipErrorInvalidValue;
-        auto kern = four ? fcc_ragged_tile_kernel<4> : fcc_ragged_tile_kernel<8>;
-        hipLaunchKernelGGL(kern, grid, block, 0, s, r, kb, p.tiles_y, (int)tiles, p.split_k, p.kblocks_per_split, a.workspace,
-                           a.counters);
+        // Straight to LDS where rows start at dwords (and offsets fit 32 bits) and some compute units get three workgroups.
+        // Up to two, where a workgroup's own latency counts, the kernel that holds its scales and bias from the start is
+        // ahead (577 x 1160 -> 1160, 384 workgroups, 11.2 us against 11.8; 256 x 1160 -> 3480, 448, 11.6 / 12.2).
+        const bool dma = a.K % 2 == 0 && a.K >= 8 && (reinterpret_cast<uintptr_t>(a.x) & 3) == 0 &&
+                         a.M * a.K * 2 < ((int64_t)1 << 31) && (int64_t)4 * kb * 2 * kTileBytes < ((int64_t)1 << 31) &&
+                         tiles * p.split_k > 2 * (int64_t)p.n_cus;
+        auto kern = dma ? (four ? fcc_ragged_tile_dma_kernel<4> : fcc_ragged_tile_dma_kernel<8>)
+                        : (four ? fcc_ragged_tile_kernel<4> : fcc_ragged_tile_kernel<8>);
+        hipLaunchKernelGGL(kern, grid, block, dma ? RD_STAGES * RG_BM * kBlockK * 2 : 0, s, r, kb, p.tiles_y, (int)tiles, p.split_k,
+                           p.kblocks_per_split, a.workspace, a.counters);
     }
     return (int)hipGetLastError();
 }

@@ -173,7 +173,7 @@ struct LaunchPlan {
     unsigned dynamic_lds = 0;   // bytes of dynamic LDS (decode kernel: the cross-wave reduction buffer)
     size_t workspace_bytes = 0;
     size_t counter_count = 0;
-    int n_cus = 0;  // routed grouped launches: the compute-unit count that the cut along K is chosen for on the device
+    int n_cus = 0;  // routed grouped launches, ragged nodes: the compute-unit count that the launch is chosen for
     const char* name = "";
 };
 

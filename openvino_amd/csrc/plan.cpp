@@ -718,6 +718,7 @@ bool plan_stream_routed(const FcDeviceArgs& a, int64_t pairs, int n_experts, int
 void plan_ragged(const FcDeviceArgs& a, int n_cus, LaunchPlan* plan) {
     LaunchPlan p;
     p.kernel = OVFCC_KERNEL_PLAIN;
+    p.n_cus = n_cus;
     const bool four = a.layout.bits == 4;
     const int64_t kb = a.layout.k_blocks;
     // The rows kernel up to 16 rows, and up to the row count at which its workgroups (32 rows each) still fit the chip

@@ -118,6 +118,46 @@ def test_rows_keep_to_themselves(dev, req):
             w.close()
 
 
+@pytest.mark.parametrize("wt,zt,N,K,M,bias", [
+    ("i8", "none", 3480, 1160, 577, True),   # rows of 16-byte pieces
+    ("u8", "u8", 3474, 394, 577, False),     # the row ends inside a piece, one dword of it left
+    ("i4", "none", 4225, 262, 514, True),    # ... three dwords left, two rows in the last row tile
+    ("u4", "u4", 4300, 388, 521, False),     # ... two
+    ("i8", "u8", 1161, 4300, 577, True),     # parts of nine k-blocks, the last of seven
+    ("u8", "none", 8300, 14, 257, False),    # one k-block, two pieces
+])
+def test_tiles_loaded_straight_to_lds_and_through_registers(oracle, dev, req, wt, zt, N, K, M, bias):
+    """Activations at a multiple of four bytes take the kernel that loads them straight to LDS, those at an odd multiple
+    of two the one that loads through registers: the same bits, and a row's result does not see its neighbours.  (The
+    first kernel takes launches of more than two workgroups to a compute unit, 512 here.)"""
+    import torch
+    c = datagen.make_case(2300 + K, M, K, N, wt, K, zt, with_bias=bias)
+    w = fc.CompressedWeights.from_case(dev, c, output_type="f32")
+
+    def run(x, shift):
+        buf = torch.zeros(M * K + 8, dtype=torch.float16, device="cuda")
+        buf[shift:shift + M * K] = torch.from_numpy(x).cuda().reshape(-1)
+        y = torch.full((M, N), float("nan"), dtype=torch.float32, device="cuda")
+        torch.cuda.synchronize()
+        req.infer_device(w, buf.data_ptr() + 2 * shift, y.data_ptr(), M)
+        req.sync()
+        assert req.last_kernel()["name"] == f"fcc_ragged_tile_w{wt[1]}"
+        return y.cpu().numpy()
+
+    try:
+        y = run(c.x, 0)
+        check_parity(oracle, y, oracle_y(oracle, c), K, f"{wt}/{zt} N={N} K={K} M={M}", output_rounding_slack=True)
+        assert np.array_equal(y, run(c.x, 2))  # four bytes further
+        assert np.array_equal(y, run(c.x, 1))  # two
+        x = c.x.copy()
+        x[1::2] = np.inf
+        x[1, 0] = np.nan
+        dirty = run(x, 0)
+        assert np.array_equal(y[0::2], dirty[0::2]) and not np.isfinite(dirty[1::2]).any()
+    finally:
+        w.close()
+
+
 def blob_fields(blob, at=0):
     """(version, flags, bytes of the weights) of the header that begins at byte `at`, as views into the blob."""
     head = int(blob[at + 12:at + 16].view(np.uint32)[0])
