@@ -2062,9 +2062,12 @@ int ovfcc_fc_run(ovfcc_request* r, const ovfcc_weights* w, const void* x_host, v
     char* hs = static_cast<char*>(r->h_stage);
     if (staged)
         std::memcpy(hs, x_host, xb);
-    HIP_TRY(hipMemcpyAsync(r->d_x, staged ? hs : x_host, xb, hipMemcpyHostToDevice, r->stream));
+    if (!staged)
+        HIP_TRY(hipMemcpyAsync(r->d_x, x_host, xb, hipMemcpyHostToDevice, r->stream));
+    else if (int e = ovfcc::launch_fetch(r->d_x, hs, xb, r->stream))
+        return hip_fail((hipError_t)e, "copy of the activations");
     // ... and the kernel writes its (write-once) output straight into the pinned memory, which is mapped into the
-    // device's address space: one copy operation less.  The activations are copied: every workgroup reads them.
+    // device's address space: one copy operation less.  The activations are copied, by a kernel: every workgroup reads them.
     rc = ovfcc_fc_run_device(r, w, r->d_x, staged ? static_cast<void*>(hs + y_off) : r->d_y, M);
     if (rc)
         return rc;

@@ -90,6 +90,29 @@ __global__ __launch_bounds__(256) void fcc_rows_kernel(uint4_t* __restrict__ dst
         dst[to + i] = src[from + i];
 }
 
+// Host memory that the device maps (src) into device memory, sixteen bytes per thread and the last few one by one.  A copy
+// command of this size goes to a copy engine, whose start and whose signal to the compute queue cost more than the
+// transfer: a call of a classifier head with 8 rows of 2048 inputs takes 29.1 us through such a
+// command and 25.0 this way, one with 83 rows of 1726 54.1 and 50.3.
+__global__ __launch_bounds__(256) void fcc_fetch_kernel(uint4_t* __restrict__ dst, const uint4_t* __restrict__ src, unsigned bytes) {
+    const unsigned i = blockIdx.x * 256 + threadIdx.x;
+    if (i < bytes / 16)
+        dst[i] = src[i];
+    const unsigned tail = bytes & ~15u;
+    if (i < bytes - tail)
+        reinterpret_cast<uint8_t*>(dst)[tail + i] = reinterpret_cast<const uint8_t*>(src)[tail + i];
+}
+
+int launch_fetch(void* dst, const void* src, size_t bytes, void* stream) {
+    if (bytes == 0)
+        return 0;
+    if (bytes > ((size_t)1 << 30) || ((reinterpret_cast<uintptr_t>(dst) | reinterpret_cast<uintptr_t>(src)) & 15))
+        return (int)hipErrorInvalidValue;
+    hipLaunchKernelGGL(fcc_fetch_kernel, dim3((unsigned)((bytes + 4095) / 4096)), dim3(256), 0, static_cast<hipStream_t>(stream),
+                       (uint4_t*)dst, (const uint4_t*)src, (unsigned)bytes);
+    return (int)hipGetLastError();
+}
+
 int launch_rows(void* dst, const void* src, const int* src_row, const int* dst_row, int rows, int row_bytes,
                 void* stream) {
     if (rows <= 0)

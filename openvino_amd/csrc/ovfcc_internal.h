@@ -379,6 +379,8 @@ int launch_i8_colsum(const void* w_tiled, const void* zp_tiled, int zp_const, in
 // weights, one group per channel, N % 256 == 0.
 int launch_prefill_i8(const FcDeviceArgs& a, const void* xq, const float* inv_scale, const int* qsum, const int* za,
                       const int* cw, void* stream);
+// Pinned host memory to device memory by a kernel; both 16-byte aligned, at most 1 GiB.
+int launch_fetch(void* dst, const void* src, size_t bytes, void* stream);
 // dst[r] = src[src_row[r]] (dst_row null) or dst[dst_row[r]] = src[r] (src_row null), rows of row_bytes % 16 == 0 bytes;
 // the caller guarantees that every index is a row of the buffer it addresses
 int launch_rows(void* dst, const void* src, const int* src_row, const int* dst_row, int rows, int row_bytes,
