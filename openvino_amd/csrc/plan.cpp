@@ -409,7 +409,8 @@ int plan_launch(const FcDeviceArgs& a, int force_kernel, int force_split, int n_
     } else {
         // The register-fed kernels with 256-channel tiles run whatever they can, however small the launch: they split K and
         // keep their loads in flight, where the square kernel waits for every k-block (u4 in groups of 128, 129 rows:
-        // 2048 -> 2048 40.8 us there against 18.7, 14336 -> 512 268 / 27; u8 2048 -> 2048 40.7 / 27.2).  Nodes under 256 KiB,
+        // 2048 -> 2048 40.8 us there against 18.7, 14336 -> 512 268 / 27; u8 2048 -> 2048 40.7 / 27.2; i8 512 -> 1152, 200
+        // rows, 13.2 / 12.2, but 384 -> 1152 11.8 / 12.2: 8-bit nodes of three k-blocks stay).  Nodes under 256 KiB,
         // which would gain too (512 -> 256 16.5 / 9.8), stay: they are what calls the square kernel by default.
         // A grouped run shares a launch only where that covers half the chip (its other slices run one by one), and
         // p.fills tells a caller that could cut the rows into decode launches.  The LDS-dequantising kernel also needs
@@ -437,7 +438,7 @@ int plan_launch(const FcDeviceArgs& a, int force_kernel, int force_split, int n_
                 reach *= 2;
         }
         p.fills = reach * 2 >= n_cus;
-        bool big = p.fills || (a.want_async && may_async) || (a.tile_rows == 0 && may_split && L.w_bytes >= ((size_t)256 << 10));
+        bool big = p.fills || (a.want_async && may_async) || (a.tile_rows == 0 && may_split && L.w_bytes >= ((size_t)256 << 10) && (L.bits == 4 || L.k_blocks >= 4));
         const int wide_env = env_int("OVFCC_PREFILL_WIDE", -1);
         if (wide_env >= 0)
             big = wide_env != 0;
