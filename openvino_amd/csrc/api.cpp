@@ -444,11 +444,16 @@ int enqueue_rows(ovfcc_request* r, const ovfcc_weights* w, const void* x, void* 
          ovfcc::env_int("OVFCC_PREFILL_WIDE", -1) == 1)) {
         if (static_scratch)
             return fail(OVFCC_EUNSUPPORTED, "a node with int8 activations needs a quantisation buffer of the request");
+        ovfcc::LaunchPlan p;
+        ovfcc::plan_prefill_i8(a, r->ctx->n_cus, &p);
+        int rc = split_buffers(r, p, static_scratch, &a);
+        if (rc)
+            return rc;
         const size_t q_bytes = ((size_t)M * w->desc.K + 255) & ~(size_t)255;
         const size_t need = q_bytes + (size_t)M * 12;
         if (need > r->quant_cap)
             HIP_TRY(hipStreamSynchronize(r->stream));
-        int rc = grow(&r->d_quant, &r->quant_cap, need);
+        rc = grow(&r->d_quant, &r->quant_cap, need);
         if (rc)
             return rc;
         char* base = static_cast<char*>(r->d_quant);
@@ -459,15 +464,11 @@ int enqueue_rows(ovfcc_request* r, const ovfcc_weights* w, const void* x, void* 
         int e = za ? ovfcc::launch_dynquant_asym(x, base, inv_scale, qsum, za, M, w->desc.K, r->stream)
                    : ovfcc::launch_dynquant(x, base, inv_scale, qsum, M, w->desc.K, r->stream);
         if (!e)
-            e = ovfcc::launch_prefill_i8(a, base, inv_scale, qsum, za, w->d_colsum, r->stream);
+            e = ovfcc::launch_prefill_i8(a, p, base, inv_scale, qsum, za, w->d_colsum, r->stream);
         if (e)
             return hip_fail((hipError_t)e, "integer kernel launch");
-        ovfcc::LaunchPlan shown;
-        shown.kernel = OVFCC_KERNEL_PREFILL;
-        shown.tile_m = 128, shown.tile_n = 256, shown.block = 512;
-        shown.grid[0] = (unsigned)(w->desc.N / 256), shown.grid[1] = (unsigned)((M + 127) / 128);
-        shown.name = za ? "fcc_prefill_i8_w8_asym" : "fcc_prefill_i8_w8";
-        record(r, shown);
+        p.name = za ? "fcc_prefill_i8_w8_asym" : "fcc_prefill_i8_w8";
+        record(r, p);
         return OVFCC_OK;
     }
     // The same permission for 4-bit weights with groups of 128 inputs (W4A8): activations per token, or per row

@@ -377,7 +377,8 @@ int launch_i8_colsum(const void* w_tiled, const void* zp_tiled, int zp_const, in
                      void* stream);
 // Integer prefill kernel over launch_dynquant's outputs (za and cw null) or launch_dynquant_asym's: tiled 8-bit
 // weights, one group per channel, N % 256 == 0.
-int launch_prefill_i8(const FcDeviceArgs& a, const void* xq, const float* inv_scale, const int* qsum, const int* za,
+void plan_prefill_i8(const FcDeviceArgs& a, int n_cus, LaunchPlan* plan);
+int launch_prefill_i8(const FcDeviceArgs& a, const LaunchPlan& p, const void* xq, const float* inv_scale, const int* qsum, const int* za,
                       const int* cw, void* stream);
 // Pinned host memory to device memory by a kernel; both 16-byte aligned, at most 1 GiB.
 int launch_fetch(void* dst, const void* src, size_t bytes, void* stream);

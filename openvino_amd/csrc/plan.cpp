@@ -28,7 +28,7 @@ namespace ovfcc {
 //            OVFCC_GEMV16_STREAM_TILES = 1 | 2 | 4 (its channel tiles per workgroup),
 //            OVFCC_STREAM = 0 | 1 (the weight-streaming kernel nowhere, wherever it can run; without it any of the
 //            overrides above keeps the kernel that they are about),
-//            OVFCC_PREFILL_{DIRECT, ASYNC, WIDE, BIG, TAIL} = 0 | 1, OVFCC_PREFILL_ROWS = 64 | 128,
+//            OVFCC_PREFILL_{DIRECT, ASYNC, WIDE, BIG, TAIL} = 0 | 1 (BIG: 256 x 256 tiles of 4-bit and of int8-activation nodes), OVFCC_PREFILL_ROWS = 64 | 128,
 //            OVFCC_MOE_HOST_ROUTING = 1, OVFCC_MLP_FUSED = 1 (an MLP node of up to four rows as one launch instead of two),
 //            OVFCC_MLP_GRID = n (its workgroups), OVFCC_MLP_SPIN_LIMIT = n (polls after which that launch's wait for its workgroups gives up; tests);
 //   logging: OVFCC_VERBOSE = 1 (one line per launch on stderr), 2 (also weights and requests as they come and go).
@@ -584,6 +584,39 @@ int rows_cap_for(const int64_t* rows, int n, bool mid_ok) {
             best_cost = total, best = caps[c];
     }
     return best;
+}
+
+// ---- 8-bit nodes over int8 activations (kernel_prefill_i8.hip) ----------------------------------------------
+
+void plan_prefill_i8(const FcDeviceArgs& a, int n_cus, LaunchPlan* plan) {
+    LaunchPlan p;
+    p.kernel = OVFCC_KERNEL_PREFILL;
+    const int64_t kb = a.layout.k_blocks;
+    const int64_t tiles128 = a.N / 256 * ((a.M + 127) / 128), tiles = a.N / 256 * ((a.M + 255) / 256);
+    const int64_t rounds128 = (tiles128 + n_cus - 1) / n_cus, rounds = (tiles + n_cus - 1) / n_cus;
+    // A round of 256 x 256 tiles over the compute units takes 1.3 times a round of 128 x 256 tiles: 16 us + 1.07 per k-block
+    // against 15 + 0.81 (u8 8192 -> 57344, 1024 rows, 7 rounds or 4, 487 us / 381; 5120 -> 10240, 1076 rows, 2 / 1, 109 / 67;
+    // 4096 -> 12288, 2000 rows, 3 / 2, 132 / 111).  Where 128-row tiles fit in one round they stay (4096 -> 16384, 500 rows,
+    // 48.5 / 56.7) unless K is so long that half of it costs less than the 38 us that parking and adding sums takes: K in two
+    // parts, 28672 -> 8192 at 1024 rows 223 / 206, 20864 -> 7936 at 835 rows 199 / 155, but 8192 -> 8192 76 / 81.
+    // OVFCC_PREFILL_BIG = 0 | 1 overrides.
+    const bool halves = tiles * 2 <= n_cus && kb >= 144;
+    const int big_env = env_int("OVFCC_PREFILL_BIG", -1);
+    if (big_env > 0 || (big_env < 0 && (rounds * 100 <= rounds128 * 75 || (rounds128 == 1 && halves)))) {
+        p.big = true;
+        p.tiles_x = (int)(a.N / 256), p.tiles_y = (int)((a.M + 255) / 256);
+        const int64_t per = halves ? (kb + 1) / 2 : kb;
+        p.split_k = halves ? 2 : 1, p.kblocks_per_split = (int)per;
+        p.grid[0] = (unsigned)(tiles * p.split_k);
+        p.block = 256;
+        p.tile_m = 256, p.tile_n = 256;
+        p.workspace_bytes = halves ? (size_t)(tiles * 2) * 256 * 256 * sizeof(int) : 0;
+        p.counter_count = halves ? (size_t)tiles : 0;
+    } else {
+        p.tile_m = 128, p.tile_n = 256, p.block = 512;
+        p.grid[0] = (unsigned)(a.N / 256), p.grid[1] = (unsigned)((a.M + 127) / 128);
+    }
+    *plan = p;
 }
 
 // ---- weight-streaming kernel (kernel_stream.hip) ----------------------------------------------------------
