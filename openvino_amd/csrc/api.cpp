@@ -438,7 +438,7 @@ int enqueue_rows(ovfcc_request* r, const ovfcc_weights* w, const void* x, void* 
     if (L0.dynquant && L0.tiled && L0.bits == 8 && L0.groups == 1 && (w->desc.N % 256) == 0 &&
         M > ovfcc::kDecodeMaxRows && (force == OVFCC_KERNEL_AUTO || force == OVFCC_KERNEL_PREFILL) &&
         M * w->desc.K < ((int64_t)1 << 31) && (M + 127) / 128 <= 65535 &&
-        // (it has no split-K: a grid that leaves half the chip idle stays with the f16 kernels, which have;
+        // (its 128-row form has no split-K: a grid that leaves half the chip idle stays with the f16 kernels, which have;
         // OVFCC_PREFILL_WIDE = 1 forces the 256-wide kernels onto small shapes, for tests)
         ((w->desc.N / 256) * ((M + 127) / 128) * 2 >= r->ctx->n_cus ||
          ovfcc::env_int("OVFCC_PREFILL_WIDE", -1) == 1)) {

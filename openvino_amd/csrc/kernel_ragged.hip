@@ -25,7 +25,7 @@
 // What a load costs the compute unit is the number of 64-byte pieces its 64 lanes name in lane order: weights read
 // where OpenVINO left them (neighbouring lanes in different rows) kept the cache's tag stage busy every cycle of the
 // launch -- 577 x 4640 -> 3480 took 61.6 us that way and takes 42.1 in operand order.
-// An encoder layer of hidden size 1160 (four nodes, 577 rows) takes 64 us where one wave per output took 7 850.
+// An encoder layer of hidden size 1160 (four nodes, 577 rows) takes 66 us where one wave per output took 7 850.
 #include <atomic>
 
 #include "device_common.h"
