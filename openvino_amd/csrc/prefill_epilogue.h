@@ -82,10 +82,8 @@ __device__ __forceinline__ void split_k_last_arrival(const __amdgpu_buffer_rsrc_
     __syncthreads();
     if (ticket_s != (unsigned)(split_k - 1))
         return;
-    if (tid == 0)  // (everyone has arrived: nobody draws from it any more)
-        __hip_atomic_store(counters + tile_id, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     if (n0 + 64 * wn >= N)
-        return;  // the node ends on half a tile
+        return;  // the node ends on half a tile (wave 0, which resets the counter, is in its first column)
     // Last arrival: every wave adds up two of its k-group pair's four channel tiles (k-group kg takes tiles 2 kg and
     // 2 kg + 1 -- a gate tile and its up tile), all row tiles, parts in ascending order.  The loads of two parts,
     // 2 x 2 NT of them, are in flight together (a part index past split_k falls outside the descriptor's range
@@ -136,6 +134,9 @@ __device__ __forceinline__ void split_k_last_arrival(const __amdgpu_buffer_rsrc_
             for (int r2 = 0; r2 < 2; ++r2)
                 finish(2 * kg + r2, t, sum[r2][t], sc[r2], bs[r2]);
     }
+    // (at the end: the loads above would wait for an earlier store)
+    if (tid == 0)
+        __hip_atomic_store(counters + tile_id, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
 // k-group 1 -> k-group 0 through LDS, two channel tiles at a time.  Without split-K k-group 0
