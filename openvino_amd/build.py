@@ -14,6 +14,10 @@ BENCH_LIB = os.path.join(PKG, "libovfcc_bench.so")
 SOURCES = ["api.cpp", "repack.cpp", "plan.cpp", "fold.cpp", "fold_data.cpp", "kernel_plain.hip", "kernel_ragged.hip", "scratch.hip", "kernel_decode.hip", "kernel_gemv.hip", "kernel_gemv16.hip", "kernel_gemv16s.hip", "kernel_mlp.hip", "kernel_batch.hip", "kernel_stream.hip", "kernel_prefill.hip", "kernel_prefill_direct.hip", "kernel_prefill_async.hip", "kernel_prefill_big.hip",
            "kernel_prefill_wide.hip", "kernel_prefill_i8.hip", "kernel_prefill_i8w4.hip"]
 BENCH_SOURCES = ["bench.cpp", "bench_probe.hip"]
+FLAGS = ["--offload-arch=gfx950", "-O3", "-std=c++17", "-fPIC",
+         # keep the compiler from forming packed-FP32 instructions
+         "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops",
+         "-I" + os.path.join(ROOT, "include"), "-I" + CSRC]
 
 
 def hipcc_path() -> str:
@@ -24,10 +28,7 @@ def hipcc_path() -> str:
 
 
 def _hipcc(sources, out, extra, verbose):
-    cmd = [hipcc_path(), "--offload-arch=gfx950", "-O3", "-std=c++17", "-fPIC", "-shared", "-pthread",
-           # keep the compiler from forming packed-FP32 instructions
-           "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops",
-           "-I" + os.path.join(ROOT, "include"), "-I" + CSRC]
+    cmd = [hipcc_path(), *FLAGS, "-shared", "-pthread"]
     cmd += [os.path.join(CSRC, s) for s in sources]
     cmd += extra + ["-o", out]
     res = subprocess.run(cmd, capture_output=True, text=True)

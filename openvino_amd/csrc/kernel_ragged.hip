@@ -494,6 +494,10 @@ __global__ __launch_bounds__(256, 3) void fcc_ragged_tile_dma_kernel(RaggedNode 
         a_voff[i] = (unsigned)(m0 + r0 + kq) * (unsigned)a.K * 2u + ((unsigned)(col ^ kq ^ (r0 & 15)) << 4);
     }
     const unsigned w_voff = (unsigned)(wave * kStep + lane * 4 * WD);
+    // The waits below count loads, so these stay in the order of the source: arithmetic and LDS accesses may move past, loads
+    // from memory may not.  (Left to itself the compiler asked for the second k-block's weights ahead of the first one's,
+    // and every second k-block then waited for the loads of the next.)
+    auto in_order = [] { __builtin_amdgcn_sched_barrier(0x0081); };
     auto dma_x = [&](int kb, int s) {
 #pragma unroll
         for (int i = 0; i < AL; ++i) {
@@ -505,6 +509,7 @@ __global__ __launch_bounds__(256, 3) void fcc_ragged_tile_dma_kernel(RaggedNode 
             __builtin_amdgcn_raw_ptr_buffer_load_lds(rx, (lds_void_ptr)(lds3 + s * A_BYTES + (AL * wave + i) * 1024), 16,
                                                      kb < kb_hi ? at : kOob, 0, 0, 0);
         }
+        in_order();
     };
     uint32_t w[2][4][WD];
     auto load_w = [&](int kb, uint32_t(&d)[4][WD]) {
@@ -518,6 +523,7 @@ __global__ __launch_bounds__(256, 3) void fcc_ragged_tile_dma_kernel(RaggedNode 
                 d[r][0] = __builtin_amdgcn_raw_buffer_load_b32(rw, at, 0, 0);
             }
         }
+        in_order();
     };
     // (a bare barrier that waits for this wave's LDS accesses only)
     auto barrier = [&] {
@@ -532,9 +538,10 @@ __global__ __launch_bounds__(256, 3) void fcc_ragged_tile_dma_kernel(RaggedNode 
         n_of[r] = min(n0 + 16 * r + col, a.N - 1);
     half2_t off[4], off_hi[4];
     zero_points<4>(a, n_of, off, off_hi);
+    in_order();
     dma_x(kb_lo, 0);
-    dma_x(kb_lo + 1, 1);
     load_w(kb_lo, w[0]);
+    dma_x(kb_lo + 1, 1);
     load_w(kb_lo + 1, w[1]);
     float4_t acc[4][NT];  // [channel tile][row tile]
 #pragma unroll
