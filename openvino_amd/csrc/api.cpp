@@ -522,7 +522,11 @@ int enqueue_rows(ovfcc_request* r, const ovfcc_weights* w, const void* x, void* 
                     ((w->desc.N % 128) != 0 && (force == OVFCC_KERNEL_AUTO || force == OVFCC_KERNEL_PREFILL)));
     if (chunked && force == OVFCC_KERNEL_AUTO && M > ovfcc::kChunkedMinPrefillRows && (w->desc.N % 256) == 0) {
         // a register-fed prefill kernel (K split; 64-row tiles for 4-bit weights) beats two or three decode
-        // launches wherever its grid fills the chip; measured on the Llama-3-8B and -70B shapes
+        // launches wherever its grid fills the chip; measured on the Llama-3-8B and -70B shapes.  Not so nodes that end on
+        // half a tile: the prefill kernels round scaled 4-bit weights to f16, the decode kernels scale their sums (4224 -> 4224,
+        // u4 in groups of 128, 128 rows, f32 results: 1.8e-4 and 7e-8 from 64 bits), and one launch is the faster one only
+        // from 97 rows, three decode launches, on (there 35.5 us against 20.4; 65 rows 21.6 / 20.4, of 4096 -> 5760 15.3 /
+        // 19.6, u8 11008 -> 4224 33.6 / 37.6).
         ovfcc::LaunchPlan p;
         if (ovfcc::plan_launch(a, OVFCC_KERNEL_PREFILL, r->force_split, r->ctx->n_cus, &p) == OVFCC_OK && p.direct && p.fills)
             chunked = false;

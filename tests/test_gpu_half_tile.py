@@ -86,3 +86,25 @@ def test_half_tile_rule(oracle, dev, req, wt, zt, N, K, G, M, name):
         check_parity(oracle, y[some], oracle_y(oracle, c, x=c.x[some]), K, name, output_rounding_slack=True)
     finally:
         w.close()
+
+
+@pytest.mark.parametrize("wt,zt,N,K,G", [("u4", "u4", 4224, 4096, 128), ("i4", "none", 6528, 2048, 64),
+                                         ("u8", "u8", 4480, 8192, 8192)])
+def test_half_tile_nodes_of_up_to_128_rows_keep_their_decode_launches(dev, req, wt, zt, N, K, G):
+    """... whose weights are not rounded after scaling: f32 results as close to 64 bits as f32 sums over K allow."""
+    c = datagen.make_case(79, 128, K, N, wt, G, zt)
+    w = fc.CompressedWeights.from_case(dev, c, output_type="f32")
+    q = c.w.astype(np.int64) if wt == "u8" else datagen.unpack_nibbles(c.w.reshape(-1), N * K).astype(np.int64)
+    q = np.where(q > 7, q - 16, q) if wt == "i4" else q
+    z = 0 if c.zp is None else c.zp.reshape(N, -1, 1) if wt == "u8" else datagen.unpack_nibbles(c.zp.reshape(-1), N * K // G).reshape(N, -1, 1)
+    full = (q.reshape(N, K // G, G) - np.asarray(z, np.int64)) * c.scale.astype(np.float64).reshape(N, -1, 1)
+    ref = c.x.astype(np.float64) @ full.reshape(N, K).T
+    try:
+        for M in (49, 96, 97, 128):
+            print(f"half tile, decode launches {wt} N={N} K={K} M={M}", flush=True)
+            y = run_guarded(req, w, c.x[:M], N, "f32")
+            assert not req.last_kernel()["name"].startswith("fcc_prefill"), req.last_kernel()
+            # a rounding of f16 weights would show as 2^-12; a sum of K terms in f32 is within sqrt(K) 2^-24 = 5.4e-6 of exact
+            assert np.linalg.norm(y - ref[:M]) < 2e-5 * np.linalg.norm(ref[:M])
+    finally:
+        w.close()
