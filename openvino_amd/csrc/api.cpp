@@ -315,8 +315,8 @@ void record(ovfcc_request* r, const ovfcc::LaunchPlan& p) {
     i.tile_n = p.tile_n;
     std::snprintf(i.name, sizeof(i.name), "%s", p.name);
     if (ovfcc::env_int("OVFCC_VERBOSE", 0) >= 1)
-        std::fprintf(stderr, "ovfcc: launch %s grid=(%u,%u,%u) block=%u tile=%dx%d split_k=%d\n", p.name, p.grid[0],
-                     p.grid[1], p.grid[2], p.block, p.tile_m, p.tile_n, p.split_k);
+        std::fprintf(stderr, "ovfcc: launch %s grid=(%u,%u,%u) block=%u tile=%dx%d split_k=%d%s\n", p.name, p.grid[0],
+                     p.grid[1], p.grid[2], p.block, p.tile_m, p.tile_n, p.split_k, p.to_lds ? " to_lds" : "");
 }
 
 // OVFCC_VERBOSE >= 2: the call is bracketed by events and waited for, and its time and algorithmic bandwidth

@@ -682,6 +682,13 @@ static int ask_for_lds(const void* kern, std::atomic<bool>& done, int bytes) {
     return (int)e;
 }
 
+// What fcc_ragged_tile_dma_kernel assumes of its operands: rows that begin at a multiple of four bytes and hold a load's
+// eight inputs, offsets into activations and into a channel tile's weights that fit the range check of a buffer load.
+bool ragged_rows_at_dwords(const FcDeviceArgs& a) {
+    return a.K % 2 == 0 && a.K >= 8 && (reinterpret_cast<uintptr_t>(a.x) & 3) == 0 && a.M * a.K * 2 < ((int64_t)1 << 31) &&
+           a.layout.k_blocks * 8 * kTileBytes < ((int64_t)1 << 31);
+}
+
 int launch_ragged(const FcDeviceArgs& a, const LaunchPlan& p, void* stream) {
     hipStream_t s = static_cast<hipStream_t>(stream);
     const bool four = a.layout.bits == 4;
@@ -711,15 +718,11 @@ int launch_ragged(const FcDeviceArgs& a, const LaunchPlan& p, void* stream) {
         if ((int64_t)p.tiles_x * RG_BN < a.N || (int64_t)p.tiles_y * RG_BM < a.M ||
             (int64_t)p.split_k * p.kblocks_per_split < kb || p.grid[0] != (unsigned)((tiles + 7) / 8 * 8 * p.split_k))
             return (int)hipErrorInvalidValue;
-        // Straight to LDS where rows start at dwords (and offsets fit 32 bits) and some compute units get three workgroups.
-        // Up to two, where a workgroup's own latency counts, the kernel that holds its scales and bias from the start is
-        // ahead (577 x 1160 -> 1160, 384 workgroups, 11.2 us against 11.8; 256 x 1160 -> 3480, 448, 11.6 / 12.2).
-        const bool dma = a.K % 2 == 0 && a.K >= 8 && (reinterpret_cast<uintptr_t>(a.x) & 3) == 0 &&
-                         a.M * a.K * 2 < ((int64_t)1 << 31) && (int64_t)4 * kb * 2 * kTileBytes < ((int64_t)1 << 31) &&
-                         tiles * p.split_k > 2 * (int64_t)p.n_cus;
-        auto kern = dma ? (four ? fcc_ragged_tile_dma_kernel<4> : fcc_ragged_tile_dma_kernel<8>)
-                        : (four ? fcc_ragged_tile_kernel<4> : fcc_ragged_tile_kernel<8>);
-        hipLaunchKernelGGL(kern, grid, block, dma ? RD_STAGES * RG_BM * kBlockK * 2 : 0, s, r, kb, p.tiles_y, (int)tiles, p.split_k,
+        if (p.to_lds && !ragged_rows_at_dwords(a))
+            return (int)hipErrorInvalidValue;
+        auto kern = p.to_lds ? (four ? fcc_ragged_tile_dma_kernel<4> : fcc_ragged_tile_dma_kernel<8>)
+                             : (four ? fcc_ragged_tile_kernel<4> : fcc_ragged_tile_kernel<8>);
+        hipLaunchKernelGGL(kern, grid, block, p.to_lds ? RD_STAGES * RG_BM * kBlockK * 2 : 0, s, r, kb, p.tiles_y, (int)tiles, p.split_k,
                            p.kblocks_per_split, a.workspace, a.counters);
     }
     return (int)hipGetLastError();

@@ -173,7 +173,8 @@ struct LaunchPlan {
     unsigned dynamic_lds = 0;   // bytes of dynamic LDS (decode kernel: the cross-wave reduction buffer)
     size_t workspace_bytes = 0;
     size_t counter_count = 0;
-    int n_cus = 0;  // routed grouped launches, ragged nodes: the compute-unit count that the launch is chosen for
+    int n_cus = 0;  // routed grouped launches: the compute-unit count that the cut along K is chosen for on the device
+    bool to_lds = false;  // ragged tile kernel: the form whose activations go straight to LDS
     const char* name = "";
 };
 
@@ -198,6 +199,7 @@ constexpr int ragged_wave_lds(int mt) {
 // launch_ragged_repack brings the constants into that layout (w as OpenVINO packs it, w_out L.w_bytes, both on the device).
 int launch_ragged_repack(const ovfcc_fc_desc& d, const Layout& L, const void* w, void* w_out, void* stream);
 void plan_ragged(const FcDeviceArgs& a, int n_cus, LaunchPlan* plan);
+bool ragged_rows_at_dwords(const FcDeviceArgs& a);  // whether the form that loads activations straight to LDS can run
 int launch_ragged(const FcDeviceArgs& a, const LaunchPlan& plan, void* stream);
 // The weight-streaming kernel for up to 48 rows of large tiled nodes (kernel_stream.hip): whether it can run a call,
 // whether it takes it from the kernel plan_launch chose, its decomposition, its launch.

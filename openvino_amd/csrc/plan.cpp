@@ -752,7 +752,6 @@ bool plan_stream_routed(const FcDeviceArgs& a, int64_t pairs, int n_experts, int
 void plan_ragged(const FcDeviceArgs& a, int n_cus, LaunchPlan* plan) {
     LaunchPlan p;
     p.kernel = OVFCC_KERNEL_PLAIN;
-    p.n_cus = n_cus;
     const bool four = a.layout.bits == 4;
     const int64_t kb = a.layout.k_blocks;
     // The rows kernel up to 16 rows, and up to the row count at which its workgroups (32 rows each) still fit the chip
@@ -782,6 +781,10 @@ void plan_ragged(const FcDeviceArgs& a, int n_cus, LaunchPlan* plan) {
         p.grid[0] = (unsigned)((tiles + 7) / 8 * 8 * split);
         p.block = 256;
         p.tile_m = kRaggedTile, p.tile_n = kRaggedTile;
+        // Activations straight to LDS where rows start at dwords (and offsets fit 32 bits) and some compute units get three
+        // workgroups.  Up to two, where a workgroup's own latency counts, the kernel that holds its scales and bias from the
+        // start is ahead (577 x 1160 -> 1160, 384 workgroups, 11.2 us against 11.8; 256 x 1160 -> 3480, 448, 11.6 / 12.2).
+        p.to_lds = ragged_rows_at_dwords(a) && tiles * split > 2 * (int64_t)n_cus;
         p.name = four ? "fcc_ragged_tile_w4" : "fcc_ragged_tile_w8";
         p.workspace_bytes = split > 1 ? (size_t)tiles * split * kRaggedTile * kRaggedTile * sizeof(float) : 0;
         p.counter_count = split > 1 ? (size_t)tiles : 0;

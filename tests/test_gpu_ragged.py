@@ -126,21 +126,25 @@ def test_rows_keep_to_themselves(dev, req):
     ("i8", "u8", 1161, 4300, 577, True),     # parts of nine k-blocks, the last of seven
     ("u8", "none", 8300, 14, 257, False),    # one k-block, two pieces
 ])
-def test_tiles_loaded_straight_to_lds_and_through_registers(oracle, dev, req, wt, zt, N, K, M, bias):
+def test_tiles_loaded_straight_to_lds_and_through_registers(oracle, dev, req, monkeypatch, capfd, wt, zt, N, K, M, bias):
     """Activations at a multiple of four bytes take the kernel that loads them straight to LDS, those at an odd multiple
     of two the one that loads through registers: the same bits, and a row's result does not see its neighbours.  (The
     first kernel takes launches of more than two workgroups to a compute unit, 512 here.)"""
     import torch
     c = datagen.make_case(2300 + K, M, K, N, wt, K, zt, with_bias=bias)
     w = fc.CompressedWeights.from_case(dev, c, output_type="f32")
+    monkeypatch.setenv("OVFCC_VERBOSE", "1")
 
     def run(x, shift):
         buf = torch.zeros(M * K + 8, dtype=torch.float16, device="cuda")
         buf[shift:shift + M * K] = torch.from_numpy(x).cuda().reshape(-1)
         y = torch.full((M, N), float("nan"), dtype=torch.float32, device="cuda")
         torch.cuda.synchronize()
+        capfd.readouterr()
         req.infer_device(w, buf.data_ptr() + 2 * shift, y.data_ptr(), M)
         req.sync()
+        launch, = [line for line in capfd.readouterr().err.splitlines() if line.startswith("ovfcc: launch")]
+        assert launch.endswith(" to_lds") == (shift % 2 == 0), launch
         assert req.last_kernel()["name"] == f"fcc_ragged_tile_w{wt[1]}"
         return y.cpu().numpy()
 
