@@ -431,6 +431,14 @@ def floors_table(dev, req, args) -> int:
                         (2, "integers -8 .. 7 as halves"), (3, "integers 0 .. 15 as subnormal halves (what the decode kernels feed)")):
         tf = max(dev.mfma_ceiling(8, 0, shape=shape) for _ in range(3))
         print(f"| {name} | {tf:.0f} | {100 * tf / 2500:.1f} % |")
+    # ... on the order in which operands meet, and what the integer form runs at
+    print("\n| matrix-core loop on registers, random operands, all compute units | one wave per SIMD, T(FL)OP/s | two |")
+    print("|---|---|---|")
+    for shape, name in ((6, "v_mfma_f32_16x16x32_f16, 4 x 8 accumulator tiles, ascending"),
+                        (7, "the same there and back: one operand changes from MFMA to MFMA"),
+                        (5, "v_mfma_i32_16x16x64_i8")):
+        print(f"| {name} | " + " | ".join(f"{max(dev.mfma_ceiling(waves, 0, 100000, shape) for _ in range(3)):.0f}"
+                                          for waves in (4, 8)) + " |")
     # how one SIMD overlaps matrix-core and vector instructions, in shader cycles: one compute unit alone, then all
     n_cus = 256
     print("\n| matrix-core loop with vector instructions after every MFMA (v_mfma_f32_16x16x32_f16, two waves per SIMD) | "

@@ -47,7 +47,10 @@ int ovfcc_bench_floor(ovfcc_ctx* ctx, const void* arena_dev, size_t arena_bytes,
  * its clock) is the ceiling the prefill kernels are measured against beside the nominal peak.  Both operands are
  * random halves; shapes 2, 3 and 4 (valu = 0) are shape 0 with the second operand looking like weights instead:
  * integers -8 .. 7 as halves, the integers 0 .. 15 as subnormal halves, integers -8 .. 7 times a scale rounded to
- * half -- the sustained rate depends on how many operand bits toggle. */
+ * half -- the sustained rate depends on how many operand bits toggle.  Shape 5 (valu = 0): eight independent
+ * v_mfma_i32_16x16x64_i8 on random bytes.  Shapes 6 and 7 (valu = 0, rounds a multiple of 4): v_mfma_f32_16x16x32_f16 over
+ * 4 x 8 accumulator tiles as a prefill kernel orders them, the four tiles of a row always ascending, or there and back
+ * again so that one operand changes from MFMA to MFMA. */
 int ovfcc_bench_mfma(ovfcc_ctx* ctx, int waves, int valu, int shape, int rounds, float* elapsed_ms, double* flops);
 
 /* How one SIMD overlaps matrix-core and vector instructions: `workgroups` workgroups (1: one compute unit alone, no

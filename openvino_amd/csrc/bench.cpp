@@ -153,7 +153,7 @@ int ovfcc_bench_copy(ovfcc_ctx* ctx, void* dst_dev, const void* src_dev, size_t 
 
 int ovfcc_bench_mfma(ovfcc_ctx* ctx, int waves, int valu, int shape, int rounds, float* elapsed_ms, double* flops) {
     if (!ctx || !elapsed_ms || !flops || rounds <= 0 || (waves != 4 && waves != 8) || valu < 0 || valu > 4 ||
-        shape < 0 || shape > 4 || (shape >= 2 && valu != 0))
+        shape < 0 || shape > 7 || (shape >= 2 && valu != 0) || (shape >= 6 && rounds % 4 != 0))
         return fail(OVFCC_EINVAL, "bad matrix-core benchmark arguments");
     HIP_TRY(hipSetDevice(ctx->device));
     Held h;
@@ -173,7 +173,8 @@ int ovfcc_bench_mfma(ovfcc_ctx* ctx, int waves, int valu, int shape, int rounds,
     HIP_TRY(hipEventElapsedTime(elapsed_ms, h.t0, h.t1));
     if (e)
         return hip_fail((hipError_t)e, "matrix-core probe launch");
-    *flops = 2.0 * 16 * 16 * 32 * 8.0 * rounds * waves * workgroups;  // either shape: 2^17 multiply-adds per round
+    // 2^16 multiply-adds per round, of bytes 2^17
+    *flops = 2.0 * 16 * 16 * (shape == 5 ? 64 : 32) * 8.0 * rounds * waves * workgroups;
     return OVFCC_OK;
 }
 

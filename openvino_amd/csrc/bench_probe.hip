@@ -196,14 +196,84 @@ __global__ __launch_bounds__(512) void fcc_mfma_pattern_probe_kernel(float* __re
     sink[blockIdx.x * blockDim.x + threadIdx.x] = s;
 }
 
+// Integer matrix cores: eight independent v_mfma_i32_16x16x64_i8 a round on random bytes.
+__global__ __launch_bounds__(512) void fcc_mfma_i8_probe_kernel(float* __restrict__ sink, int iters) {
+    uint4_t a[4], b[4];
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+        uint4_t v;
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+            unsigned h = ((threadIdx.x * 8u + i) * 4u + j) * 2654435761u;
+            h ^= h >> 15, h *= 2246822519u, h ^= h >> 13;
+            v[j] = h;
+        }
+        (i < 4 ? a[i] : b[i - 4]) = v;
+    }
+    typedef int int4_t __attribute__((ext_vector_type(4)));
+    int4_t acc[8];
+#pragma unroll
+    for (int i = 0; i < 8; ++i)
+        acc[i] = int4_t{0, 0, 0, 0};
+    for (int it = 0; it < iters; ++it) {
+#pragma unroll
+        for (int j = 0; j < 8; ++j)
+            asm volatile("v_mfma_i32_16x16x64_i8 %0, %1, %2, %0" : "+v"(acc[j]) : "v"(a[j & 3]), "v"(b[(j >> 1) & 3]));
+    }
+    int s = 0;
+#pragma unroll
+    for (int i = 0; i < 8; ++i)
+        s ^= acc[i].x ^ acc[i].y ^ acc[i].z ^ acc[i].w;
+    sink[blockIdx.x * blockDim.x + threadIdx.x] = (float)s;
+}
+
+// A product's order of operands: 4 x 8 accumulator tiles, each row tile with the four channel tiles in ascending order, or
+// (BACK) there and back again, so that only one operand changes from one MFMA to the next.
+template <bool BACK>
+__global__ __launch_bounds__(512) void fcc_mfma_order_probe_kernel(float* __restrict__ sink, int iters) {
+    half8_t a[4], b[8];
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+        a[i] = probe_operand(threadIdx.x * 12u + i);
+#pragma unroll
+    for (int i = 0; i < 8; ++i)
+        b[i] = probe_operand(threadIdx.x * 12u + 4u + i);
+    float4_t acc[4][8];
+#pragma unroll
+    for (int i = 0; i < 32; ++i)
+        acc[i & 3][i >> 2] = float4_t{0.f, 0.f, 0.f, 0.f};
+    for (int it = 0; it < iters; ++it) {
+#pragma unroll
+        for (int i = 0; i < 32; ++i) {
+            const int t = i >> 2, r = BACK && (t & 1) ? 3 - (i & 3) : i & 3;
+            asm volatile("v_mfma_f32_16x16x32_f16 %0, %1, %2, %0" : "+v"(acc[r][t]) : "v"(a[r]), "v"(b[t]));
+        }
+    }
+    float s = 0.f;
+#pragma unroll
+    for (int i = 0; i < 32; ++i)
+        s += acc[i & 3][i >> 2].x + acc[i & 3][i >> 2].y + acc[i & 3][i >> 2].z + acc[i & 3][i >> 2].w;
+    sink[blockIdx.x * blockDim.x + threadIdx.x] = s;
+}
+
 // sink: 4 * workgroups * 64 * waves bytes.  valu: 0 to 4 multiplications after every MFMA.  shape 0: 16 x 16 x 32
-// instructions, shape 1: 32 x 32 x 16; shapes 2, 3, 4: 16 x 16 x 32 with weight-operand pattern 1, 2, 3 (valu = 0).
+// instructions, shape 1: 32 x 32 x 16; shapes 2, 3, 4: 16 x 16 x 32 with weight-operand pattern 1, 2, 3 (valu = 0, here and
+// on); 5: integers; 6, 7: 4 x 8 accumulator tiles, ascending and there and back (a quarter of the rounds, each four times as long).
 int launch_mfma_probe(float* sink, int workgroups, int waves, int valu, int shape, int iters, void* stream) {
-    if (!sink || workgroups < 1 || (waves != 4 && waves != 8) || valu < 0 || valu > 4 || iters < 1 || shape < 0 || shape > 4 ||
+    if (!sink || workgroups < 1 || (waves != 4 && waves != 8) || valu < 0 || valu > 4 || iters < 1 || shape < 0 || shape > 7 ||
         (shape >= 2 && valu != 0))
         return (int)hipErrorInvalidValue;
     hipStream_t s = static_cast<hipStream_t>(stream);
     const dim3 g((unsigned)workgroups), b(64u * waves);
+    if (shape >= 5) {
+        if (shape == 5)
+            hipLaunchKernelGGL(fcc_mfma_i8_probe_kernel, g, b, 0, s, sink, iters);
+        else if (shape == 6)
+            hipLaunchKernelGGL(fcc_mfma_order_probe_kernel<false>, g, b, 0, s, sink, iters / 4);
+        else
+            hipLaunchKernelGGL(fcc_mfma_order_probe_kernel<true>, g, b, 0, s, sink, iters / 4);
+        return (int)hipGetLastError();
+    }
     if (shape >= 2) {
         hipLaunchKernelGGL(fcc_mfma_pattern_probe_kernel, g, b, 0, s, sink, iters, shape - 1);
         return (int)hipGetLastError();

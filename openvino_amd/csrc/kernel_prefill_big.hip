@@ -180,9 +180,10 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1))) voi
     };
     // Row tiles take the channel tiles there and back again (0 1 2 3, 3 2 1 0): from one MFMA to the next only one of the
     // two operands changes, and a chip at its power limit pays for every operand bit that does.  A loop of nothing but
-    // MFMAs on random halves (4 x 8 accumulator tiles, two waves per SIMD) runs 1 388 TFLOP/s starting over and 1 456
-    // this way; here it is worth 0.8 % (8B block, 2048 rows: 779 -> 773 us).  The 128-row kernels, which are not at that
-    // limit, do not gain (117 rows: 108.8 / 109.7).  The sums are the same.
+    // MFMAs on random halves (bench.py --floors; 4 x 8 accumulator tiles) runs 1 905 TFLOP/s starting over and 1 945
+    // this way; here it is worth 0.3-0.5 % (8B block, 2048 rows, three comparisons: 789.2 -> 786.1 us; runs of one side differ
+    // by 0.2 %).  The 128-row kernels, which are not at that limit, do not gain (117 rows: 108.8 / 109.7).  The sums are
+    // the same.
     auto half = [&](int stage, Frag8 (&wa)[4], Frag8 (&wb)[4], const WSlot& sa, int ja, WSlot& sb, int jb,
                     auto&& sync_next, auto&& mem) {
         auto slot = [&](int i) {
@@ -238,6 +239,9 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1))) voi
     };
 
     // ---- prologue: weights of k-blocks 0 and 1, activations of halves 0, 1, 2; first operand unpacked ----
+    // (as built, the weights, scales and zero-points are asked for behind the barrier: the compiler moves the loads and the
+    // unpacking behind the loop's test, so that a workgroup waits for memory twice before its first MFMA.  The waits below
+    // count activations and are right either way.)
     WSlot ws0, ws1;
     load_w(0, ws0);
     load_w(1, ws1);

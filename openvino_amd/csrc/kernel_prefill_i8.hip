@@ -440,8 +440,8 @@ __global__ __launch_bounds__(512) void fcc_prefill_i8_kernel(const uint4_t* __re
 //   - weights: the wave's eight tiles of a k-block, one 128-bit load per lane each, four k-blocks' worth of registers: a
 //     tile is asked for as soon as the MFMAs of the tile before it in its registers are out, seven to eight steps of 64
 //     MFMAs before its own, and its sign bits are flipped in place during the step before it is needed.
-// What bounds it: the integer matrix pipe under the chip's power limit (a loop of nothing but its MFMAs on random bytes runs
-// 2 890 TOP/s).  u8 8192 -> 57344 at 1024 rows, quantisation included: 2 520 TOP/s, 381 us; 487 with 128-row tiles, whose
+// What bounds it: the integer matrix pipe under the chip's power limit, as far as times can say (no counters were taken; a
+// loop of nothing but its MFMAs on random bytes, bench.py --floors, runs 3 940 TOP/s).  u8 8192 -> 57344 at 1024 rows, quantisation included: 2 520 TOP/s, 381 us; 487 with 128-row tiles, whose
 // matrix cores were busy 48 % of the time at 1.95 GHz, between a barrier and an LDS latency every 32 MFMAs.
 // 1-D grid: tiles times parts along K (plan_prefill_i8); a part parks its exact i32 sums.
 // ------------------------------------------------------------------------------------------------
@@ -567,6 +567,8 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1))) voi
     };
 
     // ---- prologue: weights of k-blocks 0-2 and half of 3, activations of k-blocks 0-2 ----
+    // (as built, the weights are asked for behind the barrier: the compiler moves the loads behind the loop's test, so that a
+    // workgroup waits for memory twice before its first MFMA.  The wait below counts activations and is right either way.)
 #pragma unroll
     for (int j = 0; j < 3; ++j) {
         load_w(kb_lo + j, 0, w[j][0]);
@@ -644,6 +646,8 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1))) voi
         __syncthreads();
         if (ticket_s != (unsigned)(split - 1))
             return;
+        // (as built, the loads come one to a few at a time and two accumulator tiles pass through scratch memory: the
+        // accumulation registers leave little room.  The 38 us of plan_prefill_i8 are this form's.)
         for (int z = 0; z < split; ++z) {
             if (z == part)
                 continue;
