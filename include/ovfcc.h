@@ -258,7 +258,12 @@ int ovfcc_fc_run_device(ovfcc_request* req, const ovfcc_weights* w, const void* 
  * ovfcc_init, not here), so calls from different requests and host threads are safe and simply do not overlap.  The
  * exception is a stream under graph capture, which cannot wait for an event from outside its capture: replays of
  * graphs that hold such launches, and anything else that uses the array at the same time, are the caller's to keep
- * apart. */
+ * apart.  Which launches split K is the planner's choice and may change from one version of the library to the next;
+ * ovfcc_last_kernel_info says so for each (split_k > 1).  Today: of more than 48 rows, tiled nodes whose tiles (64 or 128
+ * rows by 256 channels) cover at most half of the compute units and that hold at least 16 blocks of 128 inputs -- among them
+ * nodes whose N is an odd multiple of 128 and nodes of 256 KiB and more on grids that do not fill half the chip even with K
+ * split, which ran unsplit, on the square kernel, in earlier versions -- and nodes with one scale per channel that fit no
+ * tile, of at least eight blocks; of up to 48 rows, nodes whose channels alone do not fill the chip. */
 int ovfcc_fc_run_device_static(ovfcc_request* req, const ovfcc_weights* w, const void* x_dev, void* y_dev, int64_t M);
 
 /* Several independent nodes of one shape and weight format in one launch: the experts of a
