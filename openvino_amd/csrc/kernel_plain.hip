@@ -187,7 +187,8 @@ __global__ __launch_bounds__(256) void fcc_moe_combine_kernel(void* __restrict__
 // Bound by latency, a chain of a few waits: the expert's pointers (from the kernel arguments) and the first 256 indices
 // are asked for at the start and kept, and the counts meet in a reduction across wave 0's lanes instead of in one thread
 // that divides and adds for each expert in turn.  Block of eight experts (4096 / 14336, top two), six rows: 132.2 ->
-// 129.5 us together with the weighted sum above; the routing dispatch alone, traced, 5.7 -> 5.3.
+// 129.5 us together with the weighted sum above (131.2 -> 128.5 and 141.2 -> 138.2 on other boxes; runs of one side can differ
+// by as much); the routing dispatch alone, traced, 5.7 -> 5.3.
 // ------------------------------------------------------------------------------------------------
 __global__ __launch_bounds__(256) void fcc_moe_route_kernel(const int* __restrict__ indices, int R, int M, int top_k,
                                                             int n_experts, int a_batches, int inverse, int cap,

@@ -440,9 +440,12 @@ __global__ __launch_bounds__(512) void fcc_prefill_i8_kernel(const uint4_t* __re
 //   - weights: the wave's eight tiles of a k-block, one 128-bit load per lane each, four k-blocks' worth of registers: a
 //     tile is asked for as soon as the MFMAs of the tile before it in its registers are out, seven to eight steps of 64
 //     MFMAs before its own, and its sign bits are flipped in place during the step before it is needed.
-// What bounds it: the integer matrix pipe under the chip's power limit, as far as times can say (no counters were taken; a
-// loop of nothing but its MFMAs on random bytes, bench.py --floors, runs 3 940 TOP/s).  u8 8192 -> 57344 at 1024 rows, quantisation included: 2 520 TOP/s, 381 us; 487 with 128-row tiles, whose
-// matrix cores were busy 48 % of the time at 1.95 GHz, between a barrier and an LDS latency every 32 MFMAs.
+// u8 8192 -> 57344 at 1024 rows, quantisation included: 2 520 TOP/s, 381 us; 487 with 128-row tiles, whose matrix cores were
+// busy 48 % of the time at 1.95 GHz, between a barrier and an LDS latency every 32 MFMAs.  What bounds it: the integer
+// matrix pipe where the chip stays busy (67-69 % of the busy cycles by the counters in nodes of one round of tiles), under a
+// clock that falls with its load; with 3.5 rounds (57344 channels) the pipe is busy 57 %: every tile starts with two
+// latencies of memory, and the last round is half empty.  A loop of nothing but its MFMAs on random bytes (bench.py
+// --floors) runs 3 940 TOP/s.
 // 1-D grid: tiles times parts along K (plan_prefill_i8); a part parks its exact i32 sums.
 // ------------------------------------------------------------------------------------------------
 constexpr int PIB_BM = 256, PIB_BN = 256, PIB_STAGES = 4, PIB_XQ = 8, PIB_AL = 8;

@@ -20,8 +20,12 @@
 //   fcc_ragged_tile_dma_kernel  the same tiles where rows start at dwords: the activations go to LDS without registers
 //                           or LDS stores.  577 x 1160 -> 3480 (552 tiles) 18.1 -> 15.2 us, 1160 -> 4300 18.4 -> 15.7, 4300
 //                           -> 1160 23.2 -> 18.9, 1500 x 1600 -> 4800 51.5 -> 46.1; a k-block of three workgroups takes 0.97 us
-//                           against 0.32 of matrix-core work: 32 load instructions a workgroup, 16 cycles of the
-//                           address path each, are 0.64.  A fourth stage leaves room for two workgroups only (17.8).
+//                           against 0.32 of matrix-core work (by the counters their pipe is busy 20 % of the launch and
+//                           waves wait 36-39 % of their cycles).  What takes the rest: a wave's k-block holds 143 vector
+//                           instructions (32 to unpack; the rest offsets, selects and moves for the row's last k-block), 11
+//                           branches and 11 waits around its 16 MFMAs, and 32 load instructions a workgroup at 16
+//                           cycles of the address path each would be 0.64 us (counted, not measured).  A fourth stage
+//                           leaves room for two workgroups only (17.8).
 // What a load costs the compute unit is the number of 64-byte pieces its 64 lanes name in lane order: weights read
 // where OpenVINO left them (neighbouring lanes in different rows) kept the cache's tag stage busy every cycle of the
 // launch -- 577 x 4640 -> 3480 took 61.6 us that way and takes 42.1 in operand order.

@@ -410,8 +410,9 @@ int plan_launch(const FcDeviceArgs& a, int force_kernel, int force_split, int n_
         // The register-fed kernels with 256-channel tiles run whatever they can, however small the launch: they split K and
         // keep their loads in flight, where the square kernel waits for every k-block (u4 in groups of 128, 129 rows:
         // 2048 -> 2048 40.8 us there against 18.7, 14336 -> 512 268 / 27; u8 2048 -> 2048 40.7 / 27.2; i8 512 -> 1152, 200
-        // rows, 13.2 / 12.2, but 384 -> 1152 11.8 / 12.2: 8-bit nodes of three k-blocks stay).  Nodes under 256 KiB,
-        // which would gain too (512 -> 256 16.5 / 9.8), stay: they are what calls the square kernel by default.
+        // rows, 13.2 / 12.2, but 384 -> 1152 11.8 / 12.2: 8-bit nodes of three k-blocks stay).  The line at 256 KiB is not
+        // where the kernels cross: smaller nodes would gain too (129 rows, u4 in groups of 128: 512 -> 256 15.5 / 8.7, 1024 ->
+        // 384 23.0 / 12.2; u8 512 -> 256 15.4 / 13.0) and stay only because tests check the square kernel through their calls.
         // A grouped run shares a launch only where that covers half the chip (its other slices run one by one), and
         // p.fills tells a caller that could cut the rows into decode launches.  The LDS-dequantising kernel also needs
         // K % 256 == 0.  OVFCC_PREFILL_WIDE = 0 | 1 and OVFCC_PREFILL_DIRECT = 0 | 1 override for experiments.
