@@ -686,13 +686,6 @@ static int ask_for_lds(const void* kern, std::atomic<bool>& done, int bytes) {
     return (int)e;
 }
 
-// What fcc_ragged_tile_dma_kernel assumes of its operands: rows that begin at a multiple of four bytes and hold a load's
-// eight inputs, offsets into activations and into a channel tile's weights that fit the range check of a buffer load.
-bool ragged_rows_at_dwords(const FcDeviceArgs& a) {
-    return a.K % 2 == 0 && a.K >= 8 && (reinterpret_cast<uintptr_t>(a.x) & 3) == 0 && a.M * a.K * 2 < ((int64_t)1 << 31) &&
-           a.layout.k_blocks * 8 * kTileBytes < ((int64_t)1 << 31);
-}
-
 int launch_ragged(const FcDeviceArgs& a, const LaunchPlan& p, void* stream) {
     hipStream_t s = static_cast<hipStream_t>(stream);
     const bool four = a.layout.bits == 4;

@@ -750,6 +750,13 @@ bool plan_stream_routed(const FcDeviceArgs& a, int64_t pairs, int n_experts, int
 
 // ---- nodes with one scale per channel that fit no tile (kernel_ragged.hip) ---------------------------------
 
+// What fcc_ragged_tile_dma_kernel assumes of its operands: rows that begin at a multiple of four bytes and hold a load's
+// eight inputs, offsets into activations and into a channel tile's weights that fit the range check of a buffer load.
+bool ragged_rows_at_dwords(const FcDeviceArgs& a) {
+    return a.K % 2 == 0 && a.K >= 8 && (reinterpret_cast<uintptr_t>(a.x) & 3) == 0 && a.M * a.K * 2 < ((int64_t)1 << 31) &&
+           a.layout.k_blocks * 8 * kTileBytes < ((int64_t)1 << 31);
+}
+
 void plan_ragged(const FcDeviceArgs& a, int n_cus, LaunchPlan* plan) {
     LaunchPlan p;
     p.kernel = OVFCC_KERNEL_PLAIN;
