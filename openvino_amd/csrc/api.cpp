@@ -574,7 +574,7 @@ int enqueue_rows(ovfcc_request* r, const ovfcc_weights* w, const void* x, void* 
 // ---- mixture-of-experts layers with the routing done on the device --------------------------------------------
 // The grouped launch whose slices the routing kernel cuts: tiled 4-bit experts that the all-asynchronous prefill
 // kernel runs, at most kMaxGroupItems of them (their pointers travel in the routing kernel's arguments).  The
-// slice height is fixed from the average bucket (the counts stay on the device; rows_cap_for).  How many slices the buckets make is known on the device only, where
+// slice height is fixed (the counts stay on the device).  How many slices the buckets make is known on the device only, where
 // the routing kernel also chooses the cut along K for that count; grid, workspace and counters are sized for the
 // worst count up to ceil(R / cap) + n_experts, and workgroups beyond the header's grid return at once.
 struct RoutedLaunch {
@@ -587,11 +587,11 @@ bool plan_routed(ovfcc_request* r, const ovfcc_weights* w0, int64_t R, int n_exp
     if (n_experts > ovfcc::kMaxGroupItems || !w0->layout.tiled || w0->layout.bits != 4 ||
         r->force_kernel != OVFCC_KERNEL_AUTO || R <= 0)
         return false;
-    // the counts stay on the device: plan for buckets of the average size plus twice its square root (what random
-    // routing stays under)
-    const double avg = (double)R / n_experts;
-    const int64_t likely = (int64_t)std::ceil(avg + 2.0 * std::sqrt(avg));
-    int cap = ovfcc::rows_cap_for(&likely, 1, w0->layout.groups_per_kblock == 1);
+    // The counts stay on the device.  A slice costs what its own rows need, so slices are cut as high as the kernel goes
+    // (256 rows over eight experts, top two, one bucket of more than 80 rows: 285 us in slices of up to 80 rows, 245 in slices
+    // of up to 128); groups of 32 inputs with a zero-point table, whose higher forms run alone on a compute unit, stop at 80.
+    const int64_t tallest = w0->layout.groups_per_kblock == 4 && w0->layout.zp_table ? 80 : ovfcc::kPrefillGroupRows;
+    int cap = ovfcc::rows_cap_for(&tallest, 1, true);
     const int64_t n = (R + cap - 1) / cap + n_experts;
     if (n * cap * w0->desc.K * 2 >= ((int64_t)1 << 31) || n > 65535)
         return false;
@@ -1604,7 +1604,7 @@ int ovfcc_fc_run_grouped_device(ovfcc_request* r, const ovfcc_group_item* items,
         std::vector<int64_t> rows(n_items);
         for (int i = 0; i < n_items; ++i)
             rows[i] = items[i].M;
-        rows_cap = ovfcc::rows_cap_for(rows.data(), n_items, w0->layout.groups_per_kblock == 1);
+        rows_cap = ovfcc::rows_cap_for(rows.data(), n_items, true);
     }
     ovfcc::FcDeviceArgs a;
     std::vector<ovfcc::BatchGroupItem> work;

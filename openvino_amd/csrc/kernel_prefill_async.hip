@@ -1,13 +1,10 @@
 // Prefill kernel for 4-bit weights with register-fed matrix-core operands and fully asynchronous data
 // movement: 128 x 256 output tile per workgroup (NT = 8 row tiles of 16), 8 waves; also built with 64 x 256
-// tiles (NT = 4) for grids that 128-row tiles would underfill and, for grouped runs whose slices have between 64
-// and 128 rows (the experts of a mixture-of-experts layer), with 80 and 96 rows (NT = 5, 6; four stages of
-// weights).  The text below describes NT = 8.
+// tiles (NT = 4) for grids that 128-row tiles would underfill.  The text below describes NT = 8.
 //
 // 1-D grid, block = 512: workgroup -> (tile, part of K) by tile_work (device_common.h); the first full_tiles
 // workgroups own whole tiles in XCD-aware order, the others one of split_k parts of a tile (deterministic
-// split-K, prefill_epilogue.h).  K advances one k-block (128 inputs) per step.  The grouped kernel at the end of
-// the file runs the same body over a table of nodes, one tile row per node.
+// split-K, prefill_epilogue.h).  K advances one k-block (128 inputs) per step.
 //
 // Every operand of a k-block travels HBM/L2 -> LDS with buffer loads that write LDS directly (no registers,
 // no LDS store instructions), 16 bytes per lane:
@@ -61,18 +58,12 @@ constexpr int PA_STAGES = 3;
 constexpr int PA_XQ = 3;  // activation operands in registers: the one in use and PA_XQ - 1 on their way from LDS
 constexpr int PA_W_BYTES = 16 * kTileBytes;    // 16 KiB per stage
 constexpr int PA_P_BYTES = 1024;               // per group of a k-block: scales (512) + zero-points (256)
-// Tiles of 80 and 96 rows stage 96 rows of activations (24 KiB instead of 32) and spend the room on more stages of
-// weights and parameters: their weights come from memory rather than from L2 (every slice of a grouped run has its
-// own) and need the longer lead.
-constexpr int pa_a_bytes(int nt) { return nt == 5 || nt == 6 ? 96 * PA_BK * 2 : PA_BM * PA_BK * 2; }
-constexpr int pa_w_stages(int nt) { return nt == 5 || nt == 6 ? 4 : PA_STAGES; }
-// 128- and 64-row tiles: 147 KiB with one group per k-block, 150 and 156 KiB with two and four
-constexpr unsigned pa_lds_bytes(int nt, int gpb) {
-    return (unsigned)(PA_STAGES * pa_a_bytes(nt) + pa_w_stages(nt) * (PA_W_BYTES + PA_P_BYTES * gpb));
+// 147 KiB with one group per k-block, 150 and 156 KiB with two and four
+constexpr unsigned pa_lds_bytes(int gpb) {
+    return (unsigned)(PA_STAGES * (PA_BM * PA_BK * 2 + PA_W_BYTES + PA_P_BYTES * gpb));
 }
 
-// The whole kernel for one workgroup's share of one node.  The two kernels below differ only in where the node's
-// operands come from.
+// The whole kernel for one workgroup's share of one node.
 // GPB: groups per k-block.  With groups of 64 or 32 inputs (GPB = 2 or 4) a staged k-block carries GPB scales and
 // zero-points per channel, stored [tile][channel][group]; a wave's k-group kg and step js contract inputs
 // 32 (2 kg + js) ..+32 of the k-block, that is group kg (GPB = 2) or 2 kg + js (GPB = 4).
@@ -82,18 +73,17 @@ __device__ __forceinline__ void prefill_async_body(const uint4_t* __restrict__ w
                                                    const half_t* __restrict__ bias, void* __restrict__ y,
                                                    float* __restrict__ ws, unsigned* __restrict__ counters, int M, int N,
                                                    int K, int kb_total, int kb_per_group, int ng, int zp_const,
-                                                   int out_f32, int glu, const TileWork wk,
-                                                   const int* __restrict__ row_map = nullptr, int x_rows = 0) {
-    static_assert(NT == 8 || NT == 6 || NT == 5 || NT == 4, "tiles of 128, 96, 80 or 64 rows");
+                                                   int out_f32, int glu, const TileWork wk) {
+    static_assert(NT == 8 || NT == 4, "tiles of 128 or 64 rows");
     static_assert(GPB == 1 || ((GPB == 2 || GPB == 4) && PRESCALE), "several groups per k-block: scales go into the weights");
     constexpr int PB = PA_P_BYTES * GPB;  // parameter bytes per stage
-    constexpr int WS = pa_w_stages(NT);   // stages of weights and parameters
+    constexpr int WS = PA_STAGES;         // stages of weights and parameters
     // LDS: parameters first, then weights, then activations -- the small, scattered reads of scales and zero-points
     // keep their offsets within the 16 bits of an LDS instruction's immediate
-    constexpr int PA_A_BYTES = pa_a_bytes(NT), PA_W_OFF = WS * PB, PA_A_OFF = PA_W_OFF + WS * PA_W_BYTES;
+    constexpr int PA_A_BYTES = PA_BM * PA_BK * 2, PA_W_OFF = WS * PB, PA_A_OFF = PA_W_OFF + WS * PA_W_BYTES;
     constexpr int ZOFF = 512 * GPB;       // zero-points follow the scales
     constexpr int NOPS = 5 + 4 + (PRESCALE ? 4 : 0);  // unpack micro-operations per dword
-    constexpr int AL = (NT + 1) / 2;                    // activation loads per wave and k-block (32 AL rows staged)
+    constexpr int AL = NT / 2;                          // activation loads per wave and k-block (32 AL rows staged)
     constexpr int S = 4 * NT;                           // MFMA slots per step (a wave's two steps make a k-block)
     extern __shared__ __attribute__((aligned(16))) unsigned char lds_raw[];
     const lds_byte_ptr lds3 = (lds_byte_ptr)lds_raw;
@@ -107,7 +97,6 @@ __device__ __forceinline__ void prefill_async_body(const uint4_t* __restrict__ w
     // split-K: this workgroup contracts k-blocks [kb_lo, kb_hi); loads of k-blocks past kb_hi are sent out of range
     const int kb_lo = wk.kb_lo, kb_hi = wk.kb_hi;
 
-    constexpr unsigned kOob = 0x80000000u;
     constexpr int kRsrcFlags = 0x00020000;
     // Buffer loads: the per-lane part of an offset (row, chunk, lane) is computed once and travels in the vector
     // operand, which the hardware checks against the descriptor's range (rows >= M read zeros); the part that
@@ -119,7 +108,7 @@ __device__ __forceinline__ void prefill_async_body(const uint4_t* __restrict__ w
     const int w_len = 2 * wave < nts ? 16 * kb_total * kTileBytes : 0;  // (the tiles 2 wave, 2 wave + 1 that the wave copies)
     auto live = [&](int kb, int bytes) { return kb < kb_hi ? bytes : 0; };
 #define PA_DESC_X(kb) \
-    __builtin_amdgcn_make_buffer_rsrc(const_cast<half_t*>(x), 0, live(kb, (row_map ? x_rows : M) * K * 2), kRsrcFlags)
+    __builtin_amdgcn_make_buffer_rsrc(const_cast<half_t*>(x), 0, live(kb, M * K * 2), kRsrcFlags)
 #define PA_DESC_W(kb) \
     __builtin_amdgcn_make_buffer_rsrc(const_cast<uint4_t*>(wt + (size_t)nt0 * kb_total * 64), 0, live(kb, w_len), kRsrcFlags)
 #define PA_DESC_S(kb) \
@@ -132,22 +121,13 @@ __device__ __forceinline__ void prefill_async_body(const uint4_t* __restrict__ w
     // ---- activations: direct-to-LDS load i of the wave covers rows 4 AL wave + 4 i .. +3 of the tile (AL loads per
     // wave; 16 wave + 4 i with 128-row tiles); lane -> row (lane >> 4) of those, LDS slot lane & 15 of that row,
     // which holds global chunk (lane & 15) ^ (row & 15).  4 AL wave + 4 i is a multiple of four, so
-    // row & 15 = ((4 AL wave + 4 i) & 15) ^ (lane >> 4).  80-row tiles stage 96 rows; the loads of rows past the
-    // tile go out of range. ----
+    // row & 15 = ((4 AL wave + 4 i) & 15) ^ (lane >> 4).  ----
     unsigned a_voff[4];  // AL entries in use (a bound that depends on NT does not pass the host pass)
 #pragma unroll
     for (int i = 0; i < AL; ++i) {
         const int r0 = 4 * AL * wave + 4 * i;  // first of the load's four rows, uniform
-        int row = m0 + r0 + (lane >> 4);
-        unsigned dead = r0 >= 16 * NT ? kOob : 0u;
-        if (row_map) {
-            // the slice gathers its rows itself: row_map[.] names the row of x; rows past the slice and entries that
-            // name no row are switched off here (the descriptor spans the whole of x)
-            const int src = row < M ? row_map[row] : -1;
-            dead |= src < 0 ? kOob : 0u;
-            row = src < 0 ? 0 : src;
-        }
-        a_voff[i] = ((unsigned)(row * K) * 2u + ((unsigned)((lane & 15) ^ (lane >> 4) ^ (r0 & 15)) << 4)) | dead;
+        const int row = m0 + r0 + (lane >> 4);
+        a_voff[i] = (unsigned)(row * K) * 2u + ((unsigned)((lane & 15) ^ (lane >> 4) ^ (r0 & 15)) << 4);
     }
     auto dma_a = [&](int kb, int stage, int i) {
         { const __amdgpu_buffer_rsrc_t d_ = PA_DESC_X(kb); __builtin_amdgcn_raw_ptr_buffer_load_lds(d_,
@@ -211,9 +191,8 @@ __device__ __forceinline__ void prefill_async_body(const uint4_t* __restrict__ w
     // Per k-block a wave issues, in this order: AL activation loads (for k-block + 2), then 2 weight
     // loads and at most one parameter load (for k-block + WS).  The wait at the top of a k-block needs the
     // activations of this k-block and the weights and parameters of the next; the instructions issued after those
-    // are one k-block's worth, at least AL + 2; with more than three stages the weights of the next k-block were
-    // requested before the activations of this one, and the two weight loads that followed those may be in flight too.
-    constexpr int kWaitTop = WS == 3 ? AL + 2 : AL + 4;
+    // are one k-block's worth, at least AL + 2.
+    constexpr int kWaitTop = AL + 2;
 
     // ---- the wave's share of a staged k-block of weights: 8 bytes per tile, plus scale and zero-point ----
     typedef __attribute__((address_space(3))) const uint2_t* lds_u2_ptr;
@@ -401,7 +380,7 @@ __device__ __forceinline__ void prefill_async_body(const uint4_t* __restrict__ w
 
     // ---- epilogue (prefill_epilogue.h): the k-groups exchange halves, scale / bias / gated linear unit, split-K fix-up ----
     __builtin_amdgcn_s_waitcnt(wait_vmcnt_imm(0));  // the out-of-range loads of the last trips still target LDS
-    static_assert(pa_lds_bytes(NT, GPB) >= 8u * 4u * ((NT + 1) / 2) * 1024u, "the epilogue's exchange buffer");
+    static_assert(pa_lds_bytes(GPB) >= 8u * 4u * ((NT + 1) / 2) * 1024u, "the epilogue's exchange buffer");
     tile_epilogue_shared<PRESCALE, NT>(acc, lds_raw, st, bias, y, ws, counters, M, N, n0, m0, split_k, wk.z, tile_id,
                                        out_f32, glu);
 }
@@ -426,46 +405,6 @@ __global__ __launch_bounds__(512) void fcc_prefill_async_kernel(const uint4_t* _
                                                     kb_per_group, ng, zp_const, out_f32, glu, wk);
 }
 
-// Grouped launch: tile row tile_y is item tile_y of the table, a node of the common shape and format with at most
-// 128 rows of its own (the experts of a mixture-of-experts layer over their gathered rows).  Workgroups of one
-// item sit together in a super-tile and share its activations in L2.
-template <bool ZP_TABLE, bool PRESCALE, int NT, int GPB>
-__global__ __launch_bounds__(512) void fcc_prefill_async_grouped_kernel(const BatchGroupTable tab,
-                                                                        const BatchGroupItem* __restrict__ dev_tab,
-                                                                        const RoutedHeader* __restrict__ dev_hdr,
-                                                                        float* __restrict__ ws,
-                                                                        unsigned* __restrict__ counters, int N, int K,
-                                                                        int kb_total, int kb_per_group, int ng,
-                                                                        int zp_const, int out_f32, int glu,
-                                                                        int tiles_x, int tiles_y, int full_tiles,
-                                                                        int tail_split, int kb_per_split,
-                                                                        const int* __restrict__ row_map, int x_rows) {
-    // the table travels in the kernel arguments, or -- when the rows were bucketed on the device -- lies in memory,
-    // with the slice count and the cut along K that the routing kernel chose for it
-    if (dev_tab) {
-        const RoutedHeader h = *dev_hdr;
-        if ((int)blockIdx.x >= h.grid)
-            return;
-        tiles_y = h.tiles_y, tail_split = h.split_k, kb_per_split = h.kb_per_split, full_tiles = h.full_tiles;
-    }
-    TileWork wk = tile_work(tiles_x, tiles_y, full_tiles, tail_split, kb_per_split, kb_total, 16 * NT, PA_BN / 2);
-    BatchGroupItem it = dev_tab ? dev_tab[wk.tile_y] : tab.item[wk.tile_y];
-    // The item is the same for every lane, but the compiler cannot tell: without this, every buffer load of the body
-    // sits in a loop that looks for lanes with equal descriptors (six vector instructions and a branch per load).
-    it.w = uniform_ptr(it.w), it.scale = uniform_ptr(it.scale), it.zp = uniform_ptr(it.zp);
-    it.bias = uniform_ptr(it.bias), it.x = uniform_ptr(it.x), it.y = const_cast<void*>(uniform_ptr(it.y));
-    it.M = __builtin_amdgcn_readfirstlane(it.M);
-    if (it.M <= 0)
-        return;
-    wk.m0 = 0;
-    prefill_async_body<ZP_TABLE, PRESCALE, NT, GPB>((const uint4_t*)it.w, (const half_t*)it.scale,
-                                                    (const uint8_t*)it.zp, (const half_t*)it.x, (const half_t*)it.bias,
-                                                    it.y, ws, counters, it.M, N, K, kb_total, kb_per_group, ng, zp_const,
-                                                    out_f32, glu, wk,
-                                                    row_map ? row_map + __builtin_amdgcn_readfirstlane(it.reserved) : nullptr,
-                                                    x_rows);
-}
-
 template <typename Kern>
 static int allow_lds(Kern kern, bool* done, unsigned bytes) {
     if (*done)
@@ -481,7 +420,7 @@ static int allow_lds(Kern kern, bool* done, unsigned bytes) {
 // remaining tile, parts that cover K.
 static bool async_plan_ok(const FcDeviceArgs& a, const LaunchPlan& p) {
     const int64_t tiles = (int64_t)p.tiles_x * p.tiles_y;
-    return (p.tile_m == 128 || p.tile_m == 96 || p.tile_m == 80 || p.tile_m == 64) && p.tiles_x == (a.N + PA_BN - 1) / PA_BN && a.N % (PA_BN / 2) == 0 && p.tiles_y >= 1 && p.full_tiles >= 0 && p.full_tiles <= tiles && p.split_k >= 1 &&
+    return (p.tile_m == 128 || p.tile_m == 64) && p.tiles_x == (a.N + PA_BN - 1) / PA_BN && a.N % (PA_BN / 2) == 0 && p.tiles_y >= 1 && p.full_tiles >= 0 && p.full_tiles <= tiles && p.split_k >= 1 &&
            (int64_t)p.kblocks_per_split * p.split_k >= a.layout.k_blocks && (p.full_tiles == tiles || p.kblocks_per_split >= 1) &&
            p.grid[0] == (unsigned)(p.full_tiles + (tiles - p.full_tiles) * p.split_k) && p.grid[1] == 1 && p.grid[2] == 1 &&
            (p.split_k == 1 || (a.workspace && a.counters));
@@ -492,9 +431,9 @@ static int launch_async_gpb(const FcDeviceArgs& a, const LaunchPlan& p, hipStrea
     const Layout& L = a.layout;
     auto kern = fcc_prefill_async_kernel<ZPT, PRE, NT, GPB>;
     static bool attr_set = false;  // per instantiation
-    if (int e = allow_lds(kern, &attr_set, pa_lds_bytes(NT, GPB)))
+    if (int e = allow_lds(kern, &attr_set, pa_lds_bytes(GPB)))
         return e;
-    hipLaunchKernelGGL(kern, dim3(p.grid[0], p.grid[1], p.grid[2]), dim3(512), pa_lds_bytes(NT, GPB), s, (const uint4_t*)a.w,
+    hipLaunchKernelGGL(kern, dim3(p.grid[0], p.grid[1], p.grid[2]), dim3(512), pa_lds_bytes(GPB), s, (const uint4_t*)a.w,
                        (const half_t*)a.scale, (const uint8_t*)a.zp, (const half_t*)a.x, (const half_t*)a.bias, a.y,
                        a.workspace, a.counters, (int)a.M, (int)a.N, (int)a.K, (int)L.k_blocks,
                        (int)L.kblocks_per_group, (int)L.groups, L.zp_const, a.out_f32, L.glu, p.tiles_x,
@@ -511,35 +450,6 @@ static int launch_async_impl(const FcDeviceArgs& a, const LaunchPlan& p, hipStre
             return launch_async_gpb<ZPT, PRE, NT, 4>(a, p, s);
     }
     return launch_async_gpb<ZPT, PRE, NT, 1>(a, p, s);
-}
-
-template <bool ZPT, bool PRE, int NT, int GPB>
-static int launch_async_grouped_gpb(const BatchGroupTable& tab, const BatchGroupItem* dev_tab,
-                                    const RoutedHeader* dev_hdr, const FcDeviceArgs& a, const LaunchPlan& p,
-                                    hipStream_t s) {
-    const Layout& L = a.layout;
-    auto kern = fcc_prefill_async_grouped_kernel<ZPT, PRE, NT, GPB>;
-    static bool attr_set = false;  // per instantiation
-    if (int e = allow_lds(kern, &attr_set, pa_lds_bytes(NT, GPB)))
-        return e;
-    hipLaunchKernelGGL(kern, dim3(p.grid[0], p.grid[1], p.grid[2]), dim3(512), pa_lds_bytes(NT, GPB), s, tab, dev_tab,
-                       dev_hdr, a.workspace, a.counters, (int)a.N, (int)a.K, (int)L.k_blocks, (int)L.kblocks_per_group, (int)L.groups,
-                       L.zp_const, a.out_f32, L.glu, p.tiles_x, p.tiles_y, p.full_tiles, p.split_k,
-                       p.kblocks_per_split, a.row_map, (int)a.x_rows);
-    return (int)hipGetLastError();
-}
-
-template <bool ZPT, bool PRE, int NT>
-static int launch_async_grouped_impl(const BatchGroupTable& tab, const BatchGroupItem* dev_tab,
-                                     const RoutedHeader* dev_hdr, const FcDeviceArgs& a, const LaunchPlan& p,
-                                     hipStream_t s) {
-    if constexpr (PRE) {
-        if (a.layout.groups_per_kblock == 2)
-            return launch_async_grouped_gpb<ZPT, PRE, NT, 2>(tab, dev_tab, dev_hdr, a, p, s);
-        if (a.layout.groups_per_kblock == 4)
-            return launch_async_grouped_gpb<ZPT, PRE, NT, 4>(tab, dev_tab, dev_hdr, a, p, s);
-    }
-    return launch_async_grouped_gpb<ZPT, PRE, NT, 1>(tab, dev_tab, dev_hdr, a, p, s);
 }
 
 // dispatch on zero-point table, per-group scales and tile height
@@ -559,52 +469,6 @@ int launch_prefill_async(const FcDeviceArgs& a, const LaunchPlan& p, void* strea
     return OVFCC_ASYNC_DISPATCH(launch_async_impl, a, p, s);
 }
 
-// p plans one node of n_items * tile_m rows: its tile rows are the items of the table.  dev_tab and dev_hdr
-// (optional, both or none): table and header in device memory, written by the routing kernel earlier on the same
-// stream -- at most n_items entries of at most tile_m rows each; how many are in use and how K is cut for them is
-// the header's word, and p only sizes the launch: a 1-D grid, workspace and counters that hold
-// routed_header(tiles_x, t, k_blocks, .).grid workgroups for every t <= n_items.  `tab` is then ignored and n_items
-// is not limited to kMaxGroupItems.
-int launch_prefill_async_grouped(const BatchGroupTable& tab, int n_items, const FcDeviceArgs& a, const LaunchPlan& p,
-                                 void* stream, const BatchGroupItem* dev_tab, const RoutedHeader* dev_hdr) {
-    hipStream_t s = static_cast<hipStream_t>(stream);
-    const Layout& L = a.layout;
-    if (L.bits != 4 || n_items < 1 || p.tiles_y != n_items || !dev_tab != !dev_hdr ||
-        (a.row_map && (!dev_tab || a.x_rows < 1 || a.x_rows * a.K * 2 >= ((int64_t)1 << 31))))
-        return (int)hipErrorInvalidValue;
-    if (!dev_tab) {
-        if (!async_plan_ok(a, p) || n_items > kMaxGroupItems)
-            return (int)hipErrorInvalidValue;
-        for (int i = 0; i < n_items; ++i)
-            if (tab.item[i].M < 1 || tab.item[i].M > p.tile_m)
-                return (int)hipErrorInvalidValue;
-    } else {
-        if ((p.tile_m != 128 && p.tile_m != 96 && p.tile_m != 80 && p.tile_m != 64) || p.tiles_x != a.N / PA_BN || p.grid[1] != 1 || p.grid[2] != 1)
-            return (int)hipErrorInvalidValue;
-        for (int t = 1; t <= n_items; ++t) {
-            const RoutedHeader h = routed_header(p.tiles_x, t, (int)L.k_blocks, p.n_cus);
-            if ((unsigned)h.grid > p.grid[0] ||
-                (h.split_k > 1 && (!a.workspace || !a.counters ||
-                                   (size_t)routed_parked_tiles(h, p.tiles_x) * p.tile_m * PA_BN * sizeof(float) > p.workspace_bytes ||
-                                   (size_t)p.tiles_x * t > p.counter_count)))
-                return (int)hipErrorInvalidValue;
-        }
-    }
-    if (p.tile_m == 80 || p.tile_m == 96) {
-        // slices of 80 and 96 rows: one group per k-block only
-        if (L.groups_per_kblock != 1)
-            return (int)hipErrorInvalidValue;
-        const bool nt5 = p.tile_m == 80;
-#define OVFCC_ASYNC_MID(ZPT, PRE)                                                                          \
-    (nt5 ? launch_async_grouped_gpb<ZPT, PRE, 5, 1>(tab, dev_tab, dev_hdr, a, p, s)                         \
-         : launch_async_grouped_gpb<ZPT, PRE, 6, 1>(tab, dev_tab, dev_hdr, a, p, s))
-        return L.groups == 1 ? (L.zp_table ? OVFCC_ASYNC_MID(true, false) : OVFCC_ASYNC_MID(false, false))
-                             : (L.zp_table ? OVFCC_ASYNC_MID(true, true) : OVFCC_ASYNC_MID(false, true));
-#undef OVFCC_ASYNC_MID
-    }
-    const bool nt8 = p.tile_m == PA_BM;
-    return OVFCC_ASYNC_DISPATCH(launch_async_grouped_impl, tab, dev_tab, dev_hdr, a, p, s);
-}
 #undef OVFCC_ASYNC_DISPATCH
 
 }  // namespace ovfcc

@@ -464,8 +464,8 @@ int plan_launch(const FcDeviceArgs& a, int force_kernel, int force_split, int n_
                 rows = env_rows;
             if (a.tile_rows == 64 || a.tile_rows == 128)
                 rows = a.tile_rows;
-            // (80 and 96 rows: grouped runs only, one group per k-block)
-            if ((a.tile_rows == 80 || a.tile_rows == 96) && L.groups_per_kblock == 1)
+            // (80 and 96 rows: grouped runs only)
+            if (a.tile_rows == 80 || a.tile_rows == 96)
                 rows = a.tile_rows;
             if (rows != 128) {
                 p.tile_m = rows == 80 || rows == 96 ? rows : 64;
