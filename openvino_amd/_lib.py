@@ -210,8 +210,8 @@ def load() -> ctypes.CDLL:
 # every override the library's table holds (csrc/plan.cpp)
 ENV_NAMES = tuple("OVFCC_" + n for n in (
     "DECODE_WAVES DECODE_RT DECODE_XLDS DECODE_BATCH GEMV GEMV_C GEMV16 GEMV16_GRID GEMV16_SPLIT GEMV16_STREAM "
-    "GEMV16_STREAM_TILES STREAM PREFILL_DIRECT PREFILL_ASYNC PREFILL_WIDE PREFILL_BIG PREFILL_TAIL PREFILL_ROWS "
-    "MOE_HOST_ROUTING MLP_FUSED MLP_SPIN_LIMIT MLP_GRID VERBOSE").split())
+    "GEMV16_STREAM_TILES STREAM PREFILL_DIRECT PREFILL_ASYNC PREFILL_WIDE PREFILL_BIG PREFILL_PAIR PREFILL_TAIL "
+    "PREFILL_ROWS MOE_HOST_ROUTING MLP_FUSED MLP_SPIN_LIMIT MLP_GRID VERBOSE").split())
 # os.environ decodes every entry it hands out: at 18 us a look it cost more than a decode launch.  The mapping
 # underneath it holds the encoded entries, and a handful of lookups there take 1 us.
 _env_raw = getattr(os.environ, "_data", None)

@@ -316,7 +316,7 @@ void record(ovfcc_request* r, const ovfcc::LaunchPlan& p) {
     std::snprintf(i.name, sizeof(i.name), "%s", p.name);
     if (ovfcc::env_int("OVFCC_VERBOSE", 0) >= 1)
         std::fprintf(stderr, "ovfcc: launch %s grid=(%u,%u,%u) block=%u tile=%dx%d split_k=%d%s\n", p.name, p.grid[0],
-                     p.grid[1], p.grid[2], p.block, p.tile_m, p.tile_n, p.split_k, p.to_lds ? " to_lds" : "");
+                     p.grid[1], p.grid[2], p.block, p.tile_m, p.tile_n, p.split_k, p.to_lds ? " to_lds" : p.pair ? " pair" : "");
 }
 
 // OVFCC_VERBOSE >= 2: the call is bracketed by events and waited for, and its time and algorithmic bandwidth
@@ -383,13 +383,21 @@ int enqueue(ovfcc_request* r, const ovfcc_weights* w, const void* x, void* y, in
     return OVFCC_OK;
 }
 
-// The plan of one launch: plan_launch's, or the weight-streaming kernel's where that takes the call and nothing forces
-// another (OVFCC_STREAM, or an override about the kernel that plan_launch chose).
+// The plan of one launch: plan_launch's, or that of the weight-streaming kernel or of the prefill kernel with two workgroups per
+// compute unit where those take the call and nothing forces another (OVFCC_STREAM, OVFCC_PREFILL_PAIR, or an override about the
+// kernel that plan_launch chose).
 int plan_call(const ovfcc_request* r, const ovfcc::FcDeviceArgs& a, int force, ovfcc::LaunchPlan* p) {
     int rc = ovfcc::plan_launch(a, force, r->force_split, r->ctx->n_cus, p);
-    if (rc || (force != OVFCC_KERNEL_AUTO && force != OVFCC_KERNEL_DECODE) || r->force_split != 0 ||
-        p->kernel != OVFCC_KERNEL_DECODE)
+    if (rc || r->force_split != 0)
         return rc;
+    if (p->kernel == OVFCC_KERNEL_PREFILL) {
+        const int wish = ovfcc::env_int("OVFCC_PREFILL_PAIR", -1);
+        if (wish == 1 ? ovfcc::pair_applies(a, *p) : wish != 0 && ovfcc::pair_preferred(a, *p, r->ctx->n_cus))
+            (void)ovfcc::plan_pair(a, r->ctx->n_cus, p);
+        return OVFCC_OK;
+    }
+    if ((force != OVFCC_KERNEL_AUTO && force != OVFCC_KERNEL_DECODE) || p->kernel != OVFCC_KERNEL_DECODE)
+        return OVFCC_OK;
     const int wish = ovfcc::env_int("OVFCC_STREAM", -1);
     if (wish == 1 ? ovfcc::stream_applies(a) : wish != 0 && !ovfcc::decode_overridden() && ovfcc::stream_preferred(a, *p, r->ctx->n_cus))
         ovfcc::plan_stream(a, r->ctx->n_cus, p);
@@ -397,7 +405,9 @@ int plan_call(const ovfcc_request* r, const ovfcc::FcDeviceArgs& a, int force, o
 }
 
 int launch_call(const ovfcc::FcDeviceArgs& a, const ovfcc::LaunchPlan& p, void* stream) {
-    return p.stream ? ovfcc::launch_stream(a, p, stream) : ovfcc::launch_fc(a, p, stream);
+    return p.stream ? ovfcc::launch_stream(a, p, stream)
+           : p.pair ? ovfcc::launch_prefill_pair(a, p, stream)
+                    : ovfcc::launch_fc(a, p, stream);
 }
 
 // plan_call for a call of the node on its own (fill_args's arguments, nothing set by a grouped run), through the
@@ -556,6 +566,13 @@ int enqueue_rows(ovfcc_request* r, const ovfcc_weights* w, const void* x, void* 
     }
     ovfcc::LaunchPlan p;
     int rc = cached_plan(r, w, a, force, &p);
+    // a launch that needs no scratch array otherwise does not come to share it (replays of graphs would have to be kept apart)
+    if (rc == OVFCC_OK && static_scratch && p.pair && p.split_k > 1) {
+        ovfcc::LaunchPlan other;
+        rc = ovfcc::plan_launch(a, force, r->force_split, r->ctx->n_cus, &other);
+        if (rc == OVFCC_OK && other.split_k == 1)
+            p = other;
+    }
     if (rc)
         return rc;
     rc = split_buffers(r, p, static_scratch, &a);
@@ -1660,6 +1677,14 @@ int ovfcc_fc_run_grouped_device(ovfcc_request* r, const ovfcc_group_item* items,
             a.tile_rows = (int)rows_cap;
             rc = ovfcc::plan_launch(a, OVFCC_KERNEL_PREFILL, r->force_split, r->ctx->n_cus, &p);
             grouped = !rc && p.async_dma && p.tiles_y == n;
+            if (grouped && r->force_split <= 0) {  // K is cut as it is for slices that the device counts: the same bits
+                const ovfcc::RoutedHeader h = ovfcc::routed_header(p.tiles_x, n, (int)w0->layout.k_blocks, r->ctx->n_cus);
+                p.split_k = h.split_k, p.kblocks_per_split = h.kb_per_split, p.full_tiles = h.full_tiles;
+                p.grid[0] = (unsigned)h.grid;
+                const size_t parked = (size_t)ovfcc::routed_parked_tiles(h, p.tiles_x);
+                p.workspace_bytes = parked * p.tile_m * ovfcc::kPrefillWideN * sizeof(float);
+                p.counter_count = parked ? (size_t)p.tiles_x * n - h.full_tiles : 0;
+            }
         }
         if (!grouped) {
             if (first == 0)

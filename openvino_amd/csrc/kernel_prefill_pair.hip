@@ -1,5 +1,6 @@
 // Prefill kernels for 4-bit weights that run two workgroups on a compute unit: tiles of 64 to 128 rows x 256 channels,
-// four waves of 256 registers each.  The grouped form runs the slices of a mixture-of-experts layer.
+// four waves of 256 registers each.  They run the slices of a mixture-of-experts layer and single nodes (pair_preferred in
+// plan.cpp draws the line against the 8-wave and the 256 x 256 kernel).
 //
 // Against the 8-wave kernel (kernel_prefill_async.hip), which has a compute unit to itself: the two workgroups share no
 // barrier, so one contracts while the other starts, waits or stores, and on every SIMD the vector ALU unpacks for one
@@ -8,7 +9,9 @@
 // unpacking beside the matrix cores -- 258 vector instructions (4 cycles each) to 80 MFMAs (16 cycles) per wave and k-block at
 // 80 rows; without the subtraction and the scaling the 256 rows below take 43 us less, without the barriers 3, without the
 // activation loads 16.  Expert block of eight experts, 4096 / 14336, top two, u4 in groups of 128 with zero-points, against
-// the 8-wave kernel's slices: 256 rows 282 -> 244 us, 330 rows 350 -> 275, 400 rows 363 -> 325, 1000 rows 808 -> 643.
+// the 8-wave kernel's slices: 256 rows 282 -> 244 us, 330 rows 350 -> 275, 400 rows 363 -> 325, 1000 rows 808 -> 643; with K cut
+// for two workgroups on a compute unit 295 -> 247 at 256 rows, another card.  Single nodes: pair_preferred's comment; 4096 -> 28672
+// with a gated linear unit at 2048 rows 358 us, 1.34 PFLOP/s, against 430 in 256 x 256 tiles.
 //
 // 1-D grid, block = 256: workgroup -> (tile, part of K) by tile_work (device_common.h).  A tile has the height that its rows
 // need (64, 80, 96 or 128: a branch per workgroup), whatever the launch's tile height is.
@@ -34,6 +37,9 @@ namespace ovfcc {
 
 constexpr int PP_BN = 256;
 constexpr int pp_half_bytes(int nt) { return nt * 16 * 128; }  // 64 inputs of a tile's rows
+// The order of a k-block's steps (each of its halves on its own): any is as good as another, results that sit on a tie of f16
+// move with it.
+constexpr int pp_dword(int step) { return step ^ 1; }
 // stages of activations: three k-blocks, with 128-row tiles four halves of one
 constexpr bool pp_by_halves(int nt) { return nt == 8; }
 constexpr unsigned pp_lds_bytes(int nt) { return (unsigned)((pp_by_halves(nt) ? 4 : 6) * pp_half_bytes(nt)); }
@@ -192,7 +198,7 @@ __device__ __forceinline__ void prefill_pair_body(const uint4_t* __restrict__ wt
             if constexpr (ZP_TABLE && (GPB != 1 || !PRESCALE))
                 spread(raw_z, pz_n);
         } else {
-            offsets(pz_n, piece - 3, 0, lo_n, hi_n);
+            offsets(pz_n, piece - 3, GPB == 4 ? pp_dword(0) : 0, lo_n, hi_n);
         }
     };
     auto commit = [&]() {
@@ -254,7 +260,7 @@ __device__ __forceinline__ void prefill_pair_body(const uint4_t* __restrict__ wt
         const int kb = __builtin_amdgcn_readfirstlane(kb_);
         auto x_at = [&](int n) {  // operand n: step n / NT, row tile n % NT
             const int js = n / NT, t = n % NT;
-            return *(lds_frag_ptr)(((js & 1) ? xa1 : xa0) + stage * 2 * HB + (js >> 1) * HB + t * 2048);
+            return *(lds_frag_ptr)(((pp_dword(js) & 1) ? xa1 : xa0) + stage * 2 * HB + (js >> 1) * HB + t * 2048);
         };
         half8_t xq[XQ];
         auto slot = [&](int js, int i) {
@@ -277,14 +283,14 @@ __device__ __forceinline__ void prefill_pair_body(const uint4_t* __restrict__ wt
             if ((GPB == 4 && js < 3 && i == 0) || (GPB == 2 && js == 1 && i == 0)) {
 #pragma unroll
                 for (int rr = 0; rr < 4; ++rr)
-                    offsets(pz, rr, GPB == 4 ? js + 1 : 1, off_lo, off_hi);
+                    offsets(pz, rr, GPB == 4 ? pp_dword(js + 1) : 1, off_lo, off_hi);
             }
 #pragma unroll
             for (int g = i * 4 * NOPS / S; g < (i + 1) * 4 * NOPS / S; ++g) {
                 if (js < 3)
-                    unpack_op(sa, g / NOPS, js + 1, g % NOPS, wf[(js & 1) ^ 1][g / NOPS]);
+                    unpack_op(sa, g / NOPS, pp_dword(js + 1), g % NOPS, wf[(js & 1) ^ 1][g / NOPS]);
                 else
-                    unpack_op(sb, g / NOPS, 0, g % NOPS, wf[0][g / NOPS]);
+                    unpack_op(sb, g / NOPS, pp_dword(0), g % NOPS, wf[0][g / NOPS]);
             }
             // activations two k-blocks ahead (three halves), into the stage that the barrier freed
             if constexpr (HALVES) {
@@ -377,7 +383,7 @@ __device__ __forceinline__ void prefill_pair_body(const uint4_t* __restrict__ wt
     for (int r = 0; r < 4; ++r)
 #pragma unroll
         for (int op = 0; op < NOPS; ++op)
-            unpack_op(ws0, r, 0, op, wf[0][r]);
+            unpack_op(ws0, r, pp_dword(0), op, wf[0][r]);
     __builtin_amdgcn_sched_barrier(0);
 
     // As many k-blocks per trip as there are slots, so that slots and stages are static; the rest behind the loop, at 128 rows
@@ -578,7 +584,7 @@ __device__ __forceinline__ void prefill_pair_body(const uint4_t* __restrict__ wt
 #undef PP_DESC_S
 #undef PP_DESC_Z
 
-// Grouped launch: tile row tile_y is item tile_y of the table, a node of the common shape and format with at most
+// Grouped launch: tile row tile_y is item tile_y of the table (of the one node that it holds, rows from tile_y tile_rows on), a node of the common shape and format with at most
 // tile_rows rows of its own (the experts of a mixture-of-experts layer over their gathered rows).  Workgroups of one
 // item sit together in a super-tile and share its activations in L2.
 template <bool ZP_TABLE, bool PRESCALE, int NT, int GPB>
@@ -586,7 +592,7 @@ __global__ __launch_bounds__(256, pp_waves(NT, GPB, ZP_TABLE)) void fcc_prefill_
     const BatchGroupTable tab, const BatchGroupItem* __restrict__ dev_tab, const RoutedHeader* __restrict__ dev_hdr,
     float* __restrict__ ws, unsigned* __restrict__ counters, int N, int K, int kb_total, int kb_per_group, int ng,
     int zp_const, int out_f32, int glu, int tiles_x, int tiles_y, int tile_rows, int full_tiles, int tail_split, int kb_per_split,
-    const int* __restrict__ row_map, int x_rows) {
+    const int* __restrict__ row_map, int x_rows, int one_node) {
     // the table travels in the kernel arguments, or -- when the rows were bucketed on the device -- lies in memory,
     // with the slice count and the cut along K that the routing kernel chose for it
     if (dev_tab) {
@@ -596,7 +602,12 @@ __global__ __launch_bounds__(256, pp_waves(NT, GPB, ZP_TABLE)) void fcc_prefill_
         tiles_y = h.tiles_y, tail_split = h.split_k, kb_per_split = h.kb_per_split, full_tiles = h.full_tiles;
     }
     TileWork wk = tile_work(tiles_x, tiles_y, full_tiles, tail_split, kb_per_split, kb_total, tile_rows, PP_BN / 2);
-    BatchGroupItem it = dev_tab ? dev_tab[wk.tile_y] : tab.item[wk.tile_y];
+    BatchGroupItem it = dev_tab ? dev_tab[wk.tile_y] : tab.item[one_node ? 0 : wk.tile_y];
+    if (one_node) {  // its rows wk.m0 .. + tile_rows
+        it.x = static_cast<const half_t*>(it.x) + (size_t)wk.m0 * K;
+        it.y = static_cast<char*>(it.y) + (size_t)wk.m0 * (glu ? N / 2 : N) * (out_f32 ? 4 : 2);
+        it.M = min(tile_rows, it.M - wk.m0);
+    }
     // The item and its share of the work are the same for every lane, but the compiler cannot tell: without this, every
     // buffer load of the body sits in a loop that looks for lanes with equal descriptors (six vector instructions and a
     // branch per load).
@@ -637,7 +648,7 @@ static int allow_lds(Kern kern, bool* done) {
 
 template <bool ZPT, bool PRE, int NT, int GPB>
 static int launch_grouped_impl(const BatchGroupTable& tab, const BatchGroupItem* dev_tab, const RoutedHeader* dev_hdr,
-                               const FcDeviceArgs& a, const LaunchPlan& p, hipStream_t s) {
+                               const FcDeviceArgs& a, const LaunchPlan& p, hipStream_t s, int one_node) {
     const Layout& L = a.layout;
     auto kern = fcc_prefill_async_grouped_kernel<ZPT, PRE, NT, GPB>;
     static bool attr_set = false;  // per instantiation
@@ -646,8 +657,26 @@ static int launch_grouped_impl(const BatchGroupTable& tab, const BatchGroupItem*
     hipLaunchKernelGGL(kern, dim3(p.grid[0], 1, 1), dim3(256), PP_LDS, s, tab, dev_tab, dev_hdr, a.workspace, a.counters,
                        (int)a.N, (int)a.K, (int)L.k_blocks, (int)L.kblocks_per_group, (int)L.groups, L.zp_const, a.out_f32,
                        L.glu, p.tiles_x, p.tiles_y, p.tile_m, p.full_tiles, p.split_k, p.kblocks_per_split, a.row_map,
-                       (int)a.x_rows);
+                       (int)a.x_rows, one_node);
     return (int)hipGetLastError();
+}
+
+static int launch_pair(const BatchGroupTable& tab, const BatchGroupItem* dev_tab, const RoutedHeader* dev_hdr, const FcDeviceArgs& a,
+                       const LaunchPlan& p, hipStream_t s, int one_node) {
+    const Layout& L = a.layout;
+    if (L.groups_per_kblock == 2)
+        return L.zp_table ? launch_grouped_impl<true, true, 8, 2>(tab, dev_tab, dev_hdr, a, p, s, one_node)
+                          : launch_grouped_impl<false, true, 8, 2>(tab, dev_tab, dev_hdr, a, p, s, one_node);
+    if (L.groups_per_kblock == 4 && L.zp_table)
+        return p.tile_m <= 80 ? launch_grouped_impl<true, true, 5, 4>(tab, dev_tab, dev_hdr, a, p, s, one_node)
+                              : launch_grouped_impl<true, true, 8, 4>(tab, dev_tab, dev_hdr, a, p, s, one_node);
+    if (L.groups_per_kblock == 4)
+        return launch_grouped_impl<false, true, 8, 4>(tab, dev_tab, dev_hdr, a, p, s, one_node);
+    if (L.groups == 1)
+        return L.zp_table ? launch_grouped_impl<true, false, 8, 1>(tab, dev_tab, dev_hdr, a, p, s, one_node)
+                          : launch_grouped_impl<false, false, 8, 1>(tab, dev_tab, dev_hdr, a, p, s, one_node);
+    return L.zp_table ? launch_grouped_impl<true, true, 8, 1>(tab, dev_tab, dev_hdr, a, p, s, one_node)
+                      : launch_grouped_impl<false, true, 8, 1>(tab, dev_tab, dev_hdr, a, p, s, one_node);
 }
 
 // The launch must be what tile_work assumes: a 1-D grid of full_tiles whole tiles plus split_k parts of each remaining
@@ -693,19 +722,17 @@ int launch_prefill_async_grouped(const BatchGroupTable& tab, int n_items, const 
                 return (int)hipErrorInvalidValue;
         }
     }
-    if (L.groups_per_kblock == 2)
-        return L.zp_table ? launch_grouped_impl<true, true, 8, 2>(tab, dev_tab, dev_hdr, a, p, s)
-                          : launch_grouped_impl<false, true, 8, 2>(tab, dev_tab, dev_hdr, a, p, s);
-    if (L.groups_per_kblock == 4 && L.zp_table)
-        return p.tile_m <= 80 ? launch_grouped_impl<true, true, 5, 4>(tab, dev_tab, dev_hdr, a, p, s)
-                              : launch_grouped_impl<true, true, 8, 4>(tab, dev_tab, dev_hdr, a, p, s);
-    if (L.groups_per_kblock == 4)
-        return launch_grouped_impl<false, true, 8, 4>(tab, dev_tab, dev_hdr, a, p, s);
-    if (L.groups == 1)
-        return L.zp_table ? launch_grouped_impl<true, false, 8, 1>(tab, dev_tab, dev_hdr, a, p, s)
-                          : launch_grouped_impl<false, false, 8, 1>(tab, dev_tab, dev_hdr, a, p, s);
-    return L.zp_table ? launch_grouped_impl<true, true, 8, 1>(tab, dev_tab, dev_hdr, a, p, s)
-                      : launch_grouped_impl<false, true, 8, 1>(tab, dev_tab, dev_hdr, a, p, s);
+    return launch_pair(tab, dev_tab, dev_hdr, a, p, s, 0);
+}
+
+// One node of any number of rows, as plan_pair plans it: the grouped kernel over the node's own row tiles.
+int launch_prefill_pair(const FcDeviceArgs& a, const LaunchPlan& p, void* stream) {
+    if (a.layout.bits != 4 || a.M < 1 || a.M * a.K * 2 >= ((int64_t)1 << 31) || (int64_t)p.tiles_y * p.tile_m < a.M ||
+        (p.tile_m != 128 && p.tile_m != 96 && p.tile_m != 80 && p.tile_m != 64) || !pair_plan_ok(a, p))
+        return (int)hipErrorInvalidValue;
+    BatchGroupTable tab = {};
+    tab.item[0] = BatchGroupItem{a.w, a.scale, a.zp, a.bias, a.x, a.y, (int)a.M, 0};
+    return launch_pair(tab, nullptr, nullptr, a, p, static_cast<hipStream_t>(stream), 1);
 }
 
 }  // namespace ovfcc

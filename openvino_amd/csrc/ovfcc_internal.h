@@ -158,6 +158,7 @@ struct LaunchPlan {
     bool x_in_lds = false;      // decode kernel: activations staged in LDS
     bool direct = false;        // prefill family: the kernels that feed weights from registers
     bool async_dma = false;     // ... and of those the one whose operands all travel by direct-to-LDS loads
+    bool pair = false;          // ... or the one that runs two workgroups on a compute unit (single nodes; launched by launch_prefill_pair, not launch_fc)
     bool fills = false;         // ... and whether their grid covers half the chip
     bool big = false;           // prefill family: the 4-bit kernel with 256 x 256 tiles (whole tiles, no split-K)
     bool batch = false;         // decode family: the small-batch kernel (waves own channel tiles)
@@ -261,19 +262,21 @@ struct RoutedHeader {
     int full_tiles;    // tiles that one workgroup each computes whole; the rest are split
     int pad[3];        // the slice table follows the header: keeps it 8-byte aligned
 };
-// K is split while the tiles alone leave compute units idle and every part keeps at least eight k-blocks (the
-// planner's rule for the register-fed prefill kernels).  With more tiles than compute units, the tiles of a last
-// round that would fill at most half of them are split instead, so that the launch ends with a full round of shorter
-// workgroups rather than a half-empty round of whole tiles (tile_work, device_common.h).
+// K is split while the tiles alone leave places idle (two workgroups to a compute unit) and every part keeps at least eight
+// k-blocks.  With more tiles than places, the tiles of a last round that would fill at most half of them are split
+// instead, so that the launch ends with a full round of shorter workgroups rather than a half-empty round of whole
+// tiles (tile_work, device_common.h).  (Counted with one workgroup to a compute unit: expert block 4096 / 14336 of eight, top
+// two, 256 rows 2 % slower -- 239 us against 276 of the kernel before, now 247 against 295.)
 OVFCC_HOST_DEVICE inline RoutedHeader routed_header(int tiles_x, int slices, int kb_total, int n_cus) {
     const long long tiles = (long long)tiles_x * slices;
+    const int slots = 2 * n_cus;
     int split = 1;
-    while (split < 8 && tiles * split * 2 <= n_cus && kb_total / (split * 2) >= 8)
+    while (split < 8 && tiles * split * 2 <= slots && kb_total / (split * 2) >= 8)
         split *= 2;
     long long full = split == 1 ? tiles : 0;
-    const long long rest = tiles % n_cus;
-    if (split == 1 && tiles > n_cus && rest != 0) {
-        while (split < 8 && rest * split * 2 <= n_cus && kb_total / (split * 2) >= 8)
+    const long long rest = tiles % slots;
+    if (split == 1 && tiles > slots && rest != 0) {
+        while (split < 8 && rest * split * 2 <= slots && kb_total / (split * 2) >= 8)
             split *= 2;
         if (split > 1)
             full = tiles - rest;
@@ -292,6 +295,12 @@ OVFCC_HOST_DEVICE inline long long routed_parked_tiles(const RoutedHeader& h, in
 }
 // Slice height (64, 80, 96 or 128 rows) of a grouped prefill launch over items of these row counts (plan.cpp).
 int rows_cap_for(const int64_t* rows, int n, bool mid_ok);
+// The kernel with two workgroups on a compute unit over one node: whether it can run a call that plan_launch planned, whether it
+// is faster there, its launch (plan holds plan_launch's, the result is a time in us) and that launch.
+bool pair_applies(const FcDeviceArgs& a, const LaunchPlan& plan);
+bool pair_preferred(const FcDeviceArgs& a, const LaunchPlan& plan, int n_cus);
+double plan_pair(const FcDeviceArgs& a, int n_cus, LaunchPlan* plan, double shared = 0.82);
+int launch_prefill_pair(const FcDeviceArgs& a, const LaunchPlan& plan, void* stream);
 int launch_prefill_async_grouped(const BatchGroupTable& tab, int n_items, const FcDeviceArgs& a, const LaunchPlan& plan,
                                  void* stream, const BatchGroupItem* dev_tab = nullptr,
                                  const RoutedHeader* dev_hdr = nullptr);

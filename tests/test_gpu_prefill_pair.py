@@ -4,7 +4,7 @@ import numpy as np
 import pytest
 
 from openvino_amd import datagen, fc
-from parity import check_parity, oracle_y
+from parity import check_parity, glu_reference, oracle_y
 
 pytestmark = pytest.mark.gpu
 
@@ -50,3 +50,36 @@ def test_slices_of_every_height(oracle, dev, req, monkeypatch, wt, zt, G, bias, 
     finally:
         for w in ws:
             w.close()
+
+
+@pytest.mark.parametrize("wt,zt,G,N,kb,out,glu", [
+    ("u4", "u4", 128, 768, 7, "f16", None), ("i4", "none", 128, 640, 8, "f32", None),   # (640: ends on half a tile)
+    ("u4", "u8", 384, 512, 9, "f16", None), ("i4", "none", 64, 512, 16, "f16", "swish"),
+    ("u4", "u4", 64, 896, 5, "f32", None), ("u4", "u4", 32, 512, 12, "f16", None), ("i4", "none", 32, 1152, 4, "f16", "gelu_tanh")])
+def test_one_node(oracle, dev, req, monkeypatch, wt, zt, G, N, kb, out, glu):
+    """Rows that end on, before and behind the tiles, K whole and in parts, half a tile of channels at the end: the oracle,
+    the 8-wave kernel (the same weights, rounded the same way: sums of K products in another order differ by at most K 2^-24
+    of the largest sum of magnitudes, below 1e-4 of the 2-norm here also after a tie of the f16 result has moved), and
+    repeated launches."""
+    K = 128 * kb
+    c = datagen.make_case(1400 + kb, 700, K, N, wt, G, zt, with_bias=True)
+    w = fc.CompressedWeights.from_case(dev, c, output_type=out, **({"glu": glu} if glu else {}))
+    seen = set()
+    try:
+        for M in (129, 160, 161, 255, 385, 640, 700):
+            print(f"pair node {wt}/{zt} G={G} N={N} K={K} M={M}", flush=True)
+            monkeypatch.setenv("OVFCC_PREFILL_PAIR", "1")
+            y = req.infer(w, c.x[:M])
+            info = req.last_kernel()
+            assert info["name"] == "fcc_prefill_async_w4" and info["block"] == 256, info
+            seen.add((info["tile_m"], info["split_k"] > 1))
+            assert np.array_equal(req.infer(w, c.x[:M]).view(np.uint8), y.view(np.uint8))
+            ref, scale = glu_reference(oracle, c, glu, x=c.x[:M]) if glu else (oracle_y(oracle, c, x=c.x[:M]), 1.0)
+            check_parity(oracle, y, ref, K, f"{info}", output_rounding_slack=True, limit_scale=scale)
+            monkeypatch.setenv("OVFCC_PREFILL_PAIR", "0")
+            other = req.infer(w, c.x[:M])
+            assert req.last_kernel()["block"] == 512
+            assert oracle.rel_l2(y, other.astype(np.float32)) < 1e-4
+        assert len(seen) > 1, seen
+    finally:
+        w.close()
