@@ -13,6 +13,12 @@
 // for two workgroups on a compute unit 295 -> 247 at 256 rows, another card.  Single nodes: pair_preferred's comment; 4096 -> 28672
 // with a gated linear unit at 2048 rows 358 us, 1.34 PFLOP/s, against 430 in 256 x 256 tiles.
 //
+// Tiles of 128 channels (R = 2 channel tiles a wave; single nodes): a wave alone on its SIMD pays 5 cycles for every vector
+// instruction beyond two per MFMA, and at R = 4 and 64 rows it has four.  The same MFMAs as 128 rows x 128 channels have half
+// of the unpacking: a k-block takes 1.02 us against 1.03, of 64 rows 0.62 (4096 -> 6144 at 117 rows 20.7 -> 16.9 us, 14336 -> 4096
+// 29.7 -> 25.8).  Against that, an operand read from LDS meets two MFMAs and not four, which is more than half of what LDS gives;
+// long launches keep 256 channels (plan_pair).
+//
 // 1-D grid, block = 256: workgroup -> (tile, part of K) by tile_work (device_common.h).  A tile has the height that its rows
 // need (64, 80, 96 or 128: a branch per workgroup), whatever the launch's tile height is.
 //
@@ -35,7 +41,8 @@
 
 namespace ovfcc {
 
-constexpr int PP_BN = 256;
+constexpr int pp_bn(int r) { return 64 * r; }  // channels of a tile: four waves of r channel tiles each
+constexpr int PP_BN = pp_bn(4);
 constexpr int pp_half_bytes(int nt) { return nt * 16 * 128; }  // 64 inputs of a tile's rows
 // The order of a k-block's steps (each of its halves on its own): any is as good as another, results that sit on a tie of f16
 // move with it.
@@ -47,7 +54,7 @@ constexpr unsigned pp_lds_bytes(int nt) { return (unsigned)((pp_by_halves(nt) ? 
 constexpr int pp_waves(int nt, int gpb, bool zp_table) { return nt == 8 && gpb == 4 && zp_table ? 1 : 2; }
 constexpr unsigned PP_LDS = pp_lds_bytes(6);  // the largest of the four heights: 72 KiB, twice on a compute unit
 
-template <bool ZP_TABLE, bool PRESCALE, int NT, int GPB>
+template <bool ZP_TABLE, bool PRESCALE, int NT, int GPB, int R>
 __device__ __forceinline__ void prefill_pair_body(const uint4_t* __restrict__ wt, const half_t* __restrict__ st,
                                                    const uint8_t* __restrict__ zt, const half_t* __restrict__ x,
                                                    const half_t* __restrict__ bias, void* __restrict__ y,
@@ -56,10 +63,11 @@ __device__ __forceinline__ void prefill_pair_body(const uint4_t* __restrict__ wt
                                                    int out_f32, int glu, const TileWork wk,
                                                    const int* __restrict__ row_map, int x_rows, int park_rows) {
     constexpr bool HALVES = pp_by_halves(NT);
-    constexpr bool BURST = NT >= 6;  // no registers for a second set of parameters
+    constexpr bool BURST = R == 4 && NT >= 6;  // no registers for a second set of parameters
     static_assert(GPB == 1 || ((GPB == 2 || GPB == 4) && PRESCALE), "several groups per k-block: scales go into the weights");
     constexpr int HB = pp_half_bytes(NT);
-    constexpr int S = 4 * NT;                           // MFMAs of a step (32 inputs)
+    constexpr int S = R * NT;                           // MFMAs of a step (32 inputs)
+    constexpr int BN = pp_bn(R);
     constexpr int NOPS = 5 + 4 + (PRESCALE ? 4 : 0);    // unpack operations per weight dword
     extern __shared__ __attribute__((aligned(16))) unsigned char lds_raw[];
     const lds_byte_ptr lds3 = (lds_byte_ptr)lds_raw;
@@ -69,13 +77,13 @@ __device__ __forceinline__ void prefill_pair_body(const uint4_t* __restrict__ wt
     const int lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int col = lane & 15, kq = lane >> 4;
-    const int n0 = wk.tile_x * PP_BN, m0 = wk.m0, split_k = wk.split_k;
+    const int n0 = wk.tile_x * BN, m0 = wk.m0, split_k = wk.split_k;
     const int kb_lo = wk.kb_lo, kb_hi = wk.kb_hi;
     constexpr unsigned kOob = 0x80000000u;
     constexpr int kRsrcFlags = 0x00020000;
 
-    const int nt0 = n0 / 16 + 4 * wave;
-    const int nts = n0 + 64 * wave < N ? 4 : 0;  // the wave's channel tiles: none where the node ends on half a tile
+    const int nt0 = n0 / 16 + R * wave;
+    const int nts = n0 + 16 * R * wave < N ? R : 0;  // the wave's channel tiles: none where the node ends on half a tile
     auto live = [&](int kb, int bytes) { return kb < kb_hi ? bytes : 0; };
 #define PP_DESC_X(kb) \
     __builtin_amdgcn_make_buffer_rsrc(const_cast<half_t*>(x), 0, live(kb, (row_map ? x_rows : M) * K * 2), kRsrcFlags)
@@ -121,7 +129,7 @@ __device__ __forceinline__ void prefill_pair_body(const uint4_t* __restrict__ wt
     };
     // ---- weights of one k-block ----
     struct WSlot {
-        uint4_t w[4];
+        uint4_t w[R];
         uint32_t s[GPB == 4 ? 2 : 1];  // scales (and, with one group per k-block, zero-points) of tile kq, channel col
         uint32_t z;
     };
@@ -131,7 +139,7 @@ __device__ __forceinline__ void prefill_pair_body(const uint4_t* __restrict__ wt
     };
     // (all as whole dwords: two channels' scales, four, two or one channels' zero-points; prepare picks the lane's)
     constexpr int ZB = GPB;  // bytes of a channel's zero-points in a k-block
-    const unsigned p_voff = (unsigned)(kq * (GPB == 1 ? ng : kb_total) * 16 + col) * GPB;
+    const unsigned p_voff = (unsigned)((kq & (R - 1)) * (GPB == 1 ? ng : kb_total) * 16 + col) * GPB;
     const unsigned s_shift = GPB == 1 ? 16u * (col & 1) : 0u, z_shift = 8u * ((col * ZB) & 3);
     auto load_p = [&](int kb, WSlot& s, int which) {
         const int g = GPB == 1 ? kb * g_one + (int)__umulhi((unsigned)kb, g_mul) : kb;
@@ -150,7 +158,7 @@ __device__ __forceinline__ void prefill_pair_body(const uint4_t* __restrict__ wt
             s.z = __builtin_amdgcn_raw_buffer_load_b32(d_, p_voff & ~3u, g * (16 * GPB), 0);
         }
     };
-    constexpr int LW = 4 + (PRESCALE ? 1 : 0) + (ZP_TABLE ? 1 : 0);
+    constexpr int LW = R + (PRESCALE ? 1 : 0) + (ZP_TABLE ? 1 : 0);
 
     // ---- parameters of the slot being unpacked, one register per channel tile ----
     uint32_t ps[GPB == 4 ? 2 : 1][4], pz[4];
@@ -235,9 +243,9 @@ __device__ __forceinline__ void prefill_pair_body(const uint4_t* __restrict__ wt
         }
     };
 
-    float4_t acc[4][NT];
+    float4_t acc[R][NT];
 #pragma unroll
-    for (int r = 0; r < 4; ++r)
+    for (int r = 0; r < R; ++r)
 #pragma unroll
         for (int t = 0; t < NT; ++t)
             acc[r][t] = float4_t{0.f, 0.f, 0.f, 0.f};
@@ -256,7 +264,7 @@ __device__ __forceinline__ void prefill_pair_body(const uint4_t* __restrict__ wt
     };
     // One k-block (stage: its number among the stages): step js multiplies wf[js & 1] with the row tiles while dword
     // js + 1 of slot sa (dword 0 of sb in the last step) is unpacked into the other set
-    auto block = [&](int kb_, int stage, Frag8 (&wf)[2][4], WSlot& sa, WSlot& sb) {
+    auto block = [&](int kb_, int stage, Frag8 (&wf)[2][R], WSlot& sa, WSlot& sb) {
         const int kb = __builtin_amdgcn_readfirstlane(kb_);
         auto x_at = [&](int n) {  // operand n: step n / NT, row tile n % NT
             const int js = n / NT, t = n % NT;
@@ -264,7 +272,7 @@ __device__ __forceinline__ void prefill_pair_body(const uint4_t* __restrict__ wt
         };
         half8_t xq[XQ];
         auto slot = [&](int js, int i) {
-            const int t = i >> 2, r = i & 3, n = js * NT + t;
+            const int t = i / R, r = i % R, n = js * NT + t;
             constexpr int last = 4 * NT;
             const int limit = HALVES && js < 2 ? 2 * NT : last;
             if (r == 0 && n + XQ - 1 < limit)
@@ -282,11 +290,11 @@ __device__ __forceinline__ void prefill_pair_body(const uint4_t* __restrict__ wt
             }
             if ((GPB == 4 && js < 3 && i == 0) || (GPB == 2 && js == 1 && i == 0)) {
 #pragma unroll
-                for (int rr = 0; rr < 4; ++rr)
+                for (int rr = 0; rr < R; ++rr)
                     offsets(pz, rr, GPB == 4 ? pp_dword(js + 1) : 1, off_lo, off_hi);
             }
 #pragma unroll
-            for (int g = i * 4 * NOPS / S; g < (i + 1) * 4 * NOPS / S; ++g) {
+            for (int g = i * R * NOPS / S; g < (i + 1) * R * NOPS / S; ++g) {
                 if (js < 3)
                     unpack_op(sa, g / NOPS, pp_dword(js + 1), g % NOPS, wf[(js & 1) ^ 1][g / NOPS]);
                 else
@@ -294,16 +302,16 @@ __device__ __forceinline__ void prefill_pair_body(const uint4_t* __restrict__ wt
             }
             // activations two k-blocks ahead (three halves), into the stage that the barrier freed
             if constexpr (HALVES) {
-                if (!(js & 1) && (i & 7) == 2)
-                    dma_h(2 * kb + (js >> 1) + 3, (2 * stage + (js >> 1) + 3) & 3, i >> 3);
-            } else if (js < 3 && (i & 7) == 2) {
-                const int q = js * ((NT + 2) / 3) + (i >> 3);
-                if ((i >> 3) < (NT + 2) / 3 && q < NT)
+                if (!(js & 1) && i % (2 * R) == 2)
+                    dma_h(2 * kb + (js >> 1) + 3, (2 * stage + (js >> 1) + 3) & 3, i / (2 * R));
+            } else if (js < 3 && i % (2 * R) == 2) {
+                const int q = js * ((NT + 2) / 3) + i / (2 * R);
+                if (i / (2 * R) < (NT + 2) / 3 && q < NT)
                     dma_a(kb + 2, (stage + 2) % 3, q);
             }
             // weights and parameters NS k-blocks ahead, into this k-block's own registers, unpacked by then
             if (js == 3) {
-                if ((i & 3) == 1 && (i >> 2) < 4)
+                if ((i & 3) == 1 && (i >> 2) < R)
                     load_w(kb + NS, sa, i >> 2);
                 if (i == 3)
                     load_p(kb + NS, sa, 0);
@@ -342,7 +350,7 @@ __device__ __forceinline__ void prefill_pair_body(const uint4_t* __restrict__ wt
     WSlot ws0, ws1, ws2;
     auto load_all = [&](int kb, WSlot& s) {
 #pragma unroll
-        for (int r = 0; r < 4; ++r)
+        for (int r = 0; r < R; ++r)
             load_w(kb, s, r);
         load_p(kb, s, 0);
         load_p(kb, s, 1);
@@ -374,13 +382,13 @@ __device__ __forceinline__ void prefill_pair_body(const uint4_t* __restrict__ wt
         dma_all(kb_lo + 1, 1);
         load_all(kb_lo + 2, ws2);
     }
-    Frag8 wf[2][4];
+    Frag8 wf[2][R];
 #pragma unroll
     for (int i = 0; i < 7; ++i)
         prepare(ws0, i);
     commit();
 #pragma unroll
-    for (int r = 0; r < 4; ++r)
+    for (int r = 0; r < R; ++r)
 #pragma unroll
         for (int op = 0; op < NOPS; ++op)
             unpack_op(ws0, r, pp_dword(0), op, wf[0][r]);
@@ -411,7 +419,7 @@ __device__ __forceinline__ void prefill_pair_body(const uint4_t* __restrict__ wt
     // that unpacks them, and the counted waits above would count loads that were not issued.
     auto hold = [&](const WSlot& s) {
 #pragma unroll
-        for (int r = 0; r < 4; ++r)
+        for (int r = 0; r < R; ++r)
             asm volatile("" ::"v"(s.w[r]));
         if constexpr (PRESCALE)
             asm volatile("" ::"v"(s.s[0]));
@@ -424,7 +432,7 @@ __device__ __forceinline__ void prefill_pair_body(const uint4_t* __restrict__ wt
     if constexpr (!HALVES)
         hold(ws2);
 #pragma unroll
-    for (int r = 0; r < 4; ++r)
+    for (int r = 0; r < R; ++r)
         asm volatile("" ::"v"(wf[0][r].v));  // (the same for the first step's operands, unpacked a k-block ahead)
 
     // (the lane's coordinates once more, so that nothing derived from them lives through the loop)
@@ -435,12 +443,12 @@ __device__ __forceinline__ void prefill_pair_body(const uint4_t* __restrict__ wt
     // ---- split-K: park, draw a ticket, the last arrival adds the parts in order ----
     if (split_k > 1) {
         constexpr int kAuxDeviceScope = 16;
-        constexpr unsigned kParkBytes = 4 * (4 * NT) * 64 * 16;
+        constexpr unsigned kParkBytes = 4 * (R * NT) * 64 * 16;
         const __amdgpu_buffer_rsrc_t rp = __builtin_amdgcn_make_buffer_rsrc(
-            reinterpret_cast<char*>(ws) + (size_t)wk.park_slot * split_k * park_rows * (PP_BN * 4), 0, split_k * (int)kParkBytes, kRsrcFlags);
-        const unsigned at = (unsigned)(wave * 4 * NT * 64 + lane_e) * 16u;
+            reinterpret_cast<char*>(ws) + (size_t)wk.park_slot * split_k * park_rows * (BN * 4), 0, split_k * (int)kParkBytes, kRsrcFlags);
+        const unsigned at = (unsigned)(wave * R * NT * 64 + lane_e) * 16u;
 #pragma unroll
-        for (int r = 0; r < 4; ++r)
+        for (int r = 0; r < R; ++r)
 #pragma unroll
             for (int t = 0; t < NT; ++t)
                 __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(uint4_t, acc[r][t]), rp,
@@ -456,13 +464,13 @@ __device__ __forceinline__ void prefill_pair_body(const uint4_t* __restrict__ wt
         if (nts == 0)
             return;  // (wave 0, which resets the counter, is never beyond the node's end)
 #pragma unroll
-        for (int r = 0; r < 4; ++r)
+        for (int r = 0; r < R; ++r)
 #pragma unroll
             for (int t = 0; t < NT; ++t)
                 acc[r][t] = float4_t{0.f, 0.f, 0.f, 0.f};
         for (int z = 0; z < split_k; ++z) {
 #pragma unroll
-            for (int r0 = 0; r0 < 4; r0 += 2) {  // (half of a part's loads in flight at a time: all of them do not fit)
+            for (int r0 = 0; r0 < R; r0 += 2) {  // (half of a part's loads in flight at a time: all of them do not fit)
                 float4_t part[2][NT];
 #pragma unroll
                 for (int r = 0; r < 2; ++r)
@@ -487,7 +495,7 @@ __device__ __forceinline__ void prefill_pair_body(const uint4_t* __restrict__ wt
     // ---- scale, bias, gated linear unit, stores ----
     if (nts == 0)
         return;
-    const int nw = n0 + 64 * wave;
+    const int nw = n0 + 16 * R * wave;
     auto channel_params = [&](int r, float (&sc)[4], float (&bs)[4]) {
         const int n = nw + 16 * r + 4 * kq_e;
 #pragma unroll
@@ -513,16 +521,16 @@ __device__ __forceinline__ void prefill_pair_body(const uint4_t* __restrict__ wt
             *reinterpret_cast<half4_t*>(static_cast<half_t*>(y) + idx) =
                 half4_t{to_half_rne(o[0]), to_half_rne(o[1]), to_half_rne(o[2]), to_half_rne(o[3])};
     };
-    float sc[4][4], bs[4][4];
+    float sc[R][4], bs[R][4];
 #pragma unroll
-    for (int r = 0; r < 4; ++r)
+    for (int r = 0; r < R; ++r)
         channel_params(r, sc[r], bs[r]);
     if (glu) {
 #pragma unroll
         for (int t = 0; t < NT; ++t) {
             const int m = m0 + 16 * t + col_e;
 #pragma unroll
-            for (int j = 0; j < 2; ++j) {
+            for (int j = 0; j < R / 2; ++j) {
                 const float4_t g = acc[2 * j][t], u = acc[2 * j + 1][t];
                 const float o[4] = {
                     glu_value(glu, g.x * sc[2 * j][0] + bs[2 * j][0], u.x * sc[2 * j + 1][0] + bs[2 * j + 1][0]),
@@ -535,6 +543,7 @@ __device__ __forceinline__ void prefill_pair_body(const uint4_t* __restrict__ wt
         }
         return;
     }
+    if constexpr (R == 4) {
     if (!out_f32 && (reinterpret_cast<uintptr_t>(y) & 15) == 0) {
         half_t* yh = static_cast<half_t*>(y);
 #pragma unroll
@@ -566,11 +575,12 @@ __device__ __forceinline__ void prefill_pair_body(const uint4_t* __restrict__ wt
         }
         return;
     }
+    }
 #pragma unroll
     for (int t = 0; t < NT; ++t) {
         const int m = m0 + 16 * t + col_e;
 #pragma unroll
-        for (int r = 0; r < 4; ++r) {
+        for (int r = 0; r < R; ++r) {
             const float4_t v = acc[r][t];
             const float o[4] = {v.x * sc[r][0] + bs[r][0], v.y * sc[r][1] + bs[r][1], v.z * sc[r][2] + bs[r][2],
                                 v.w * sc[r][3] + bs[r][3]};
@@ -587,8 +597,8 @@ __device__ __forceinline__ void prefill_pair_body(const uint4_t* __restrict__ wt
 // Grouped launch: tile row tile_y is item tile_y of the table (of the one node that it holds, rows from tile_y tile_rows on), a node of the common shape and format with at most
 // tile_rows rows of its own (the experts of a mixture-of-experts layer over their gathered rows).  Workgroups of one
 // item sit together in a super-tile and share its activations in L2.
-template <bool ZP_TABLE, bool PRESCALE, int NT, int GPB>
-__global__ __launch_bounds__(256, pp_waves(NT, GPB, ZP_TABLE)) void fcc_prefill_async_grouped_kernel(
+template <bool ZP_TABLE, bool PRESCALE, int NT, int GPB, int R>
+__global__ __launch_bounds__(256, pp_waves(NT, GPB, R == 4 && ZP_TABLE)) void fcc_prefill_async_grouped_kernel(
     const BatchGroupTable tab, const BatchGroupItem* __restrict__ dev_tab, const RoutedHeader* __restrict__ dev_hdr,
     float* __restrict__ ws, unsigned* __restrict__ counters, int N, int K, int kb_total, int kb_per_group, int ng,
     int zp_const, int out_f32, int glu, int tiles_x, int tiles_y, int tile_rows, int full_tiles, int tail_split, int kb_per_split,
@@ -601,7 +611,7 @@ __global__ __launch_bounds__(256, pp_waves(NT, GPB, ZP_TABLE)) void fcc_prefill_
             return;
         tiles_y = h.tiles_y, tail_split = h.split_k, kb_per_split = h.kb_per_split, full_tiles = h.full_tiles;
     }
-    TileWork wk = tile_work(tiles_x, tiles_y, full_tiles, tail_split, kb_per_split, kb_total, tile_rows, PP_BN / 2);
+    TileWork wk = tile_work(tiles_x, tiles_y, full_tiles, tail_split, kb_per_split, kb_total, tile_rows, pp_bn(R) / 2);
     BatchGroupItem it = dev_tab ? dev_tab[wk.tile_y] : tab.item[one_node ? 0 : wk.tile_y];
     if (one_node) {  // its rows wk.m0 .. + tile_rows
         it.x = static_cast<const half_t*>(it.x) + (size_t)wk.m0 * K;
@@ -621,7 +631,7 @@ __global__ __launch_bounds__(256, pp_waves(NT, GPB, ZP_TABLE)) void fcc_prefill_
     wk.split_k = __builtin_amdgcn_readfirstlane(wk.split_k), wk.park_slot = __builtin_amdgcn_readfirstlane(wk.park_slot);
     wk.kb_lo = __builtin_amdgcn_readfirstlane(wk.kb_lo), wk.kb_hi = __builtin_amdgcn_readfirstlane(wk.kb_hi);
     auto body = [&](auto rows) {
-        prefill_pair_body<ZP_TABLE, PRESCALE, decltype(rows)::value, GPB>(
+        prefill_pair_body<ZP_TABLE, PRESCALE, decltype(rows)::value, GPB, R>(
             (const uint4_t*)it.w, (const half_t*)it.scale, (const uint8_t*)it.zp, (const half_t*)it.x, (const half_t*)it.bias,
             it.y, ws, counters, it.M, N, K, kb_total, kb_per_group, ng, zp_const, out_f32, glu, wk,
             row_map ? row_map + __builtin_amdgcn_readfirstlane(it.reserved) : nullptr, x_rows, tile_rows);
@@ -646,11 +656,11 @@ static int allow_lds(Kern kern, bool* done) {
     return (int)e;
 }
 
-template <bool ZPT, bool PRE, int NT, int GPB>
+template <bool ZPT, bool PRE, int NT, int GPB, int R = 4>
 static int launch_grouped_impl(const BatchGroupTable& tab, const BatchGroupItem* dev_tab, const RoutedHeader* dev_hdr,
                                const FcDeviceArgs& a, const LaunchPlan& p, hipStream_t s, int one_node) {
     const Layout& L = a.layout;
-    auto kern = fcc_prefill_async_grouped_kernel<ZPT, PRE, NT, GPB>;
+    auto kern = fcc_prefill_async_grouped_kernel<ZPT, PRE, NT, GPB, R>;
     static bool attr_set = false;  // per instantiation
     if (int e = allow_lds(kern, &attr_set))
         return e;
@@ -664,6 +674,18 @@ static int launch_grouped_impl(const BatchGroupTable& tab, const BatchGroupItem*
 static int launch_pair(const BatchGroupTable& tab, const BatchGroupItem* dev_tab, const RoutedHeader* dev_hdr, const FcDeviceArgs& a,
                        const LaunchPlan& p, hipStream_t s, int one_node) {
     const Layout& L = a.layout;
+    if (p.tile_n == PP_BN / 2) {
+        if (!one_node || L.groups == 1)
+            return (int)hipErrorInvalidValue;
+        if (L.groups_per_kblock == 2)
+            return L.zp_table ? launch_grouped_impl<true, true, 8, 2, 2>(tab, dev_tab, dev_hdr, a, p, s, 1)
+                              : launch_grouped_impl<false, true, 8, 2, 2>(tab, dev_tab, dev_hdr, a, p, s, 1);
+        if (L.groups_per_kblock == 4)
+            return L.zp_table ? launch_grouped_impl<true, true, 8, 4, 2>(tab, dev_tab, dev_hdr, a, p, s, 1)
+                              : launch_grouped_impl<false, true, 8, 4, 2>(tab, dev_tab, dev_hdr, a, p, s, 1);
+        return L.zp_table ? launch_grouped_impl<true, true, 8, 1, 2>(tab, dev_tab, dev_hdr, a, p, s, 1)
+                          : launch_grouped_impl<false, true, 8, 1, 2>(tab, dev_tab, dev_hdr, a, p, s, 1);
+    }
     if (L.groups_per_kblock == 2)
         return L.zp_table ? launch_grouped_impl<true, true, 8, 2>(tab, dev_tab, dev_hdr, a, p, s, one_node)
                           : launch_grouped_impl<false, true, 8, 2>(tab, dev_tab, dev_hdr, a, p, s, one_node);
@@ -683,7 +705,7 @@ static int launch_pair(const BatchGroupTable& tab, const BatchGroupItem* dev_tab
 // tile, parts that cover K.
 static bool pair_plan_ok(const FcDeviceArgs& a, const LaunchPlan& p) {
     const int64_t tiles = (int64_t)p.tiles_x * p.tiles_y;
-    return p.tiles_x == (a.N + PP_BN - 1) / PP_BN && a.N % (PP_BN / 2) == 0 && p.tiles_y >= 1 && p.full_tiles >= 0 &&
+    return (p.tile_n == PP_BN || p.tile_n == PP_BN / 2) && p.tiles_x == (a.N + p.tile_n - 1) / p.tile_n && a.N % (PP_BN / 2) == 0 && p.tiles_y >= 1 && p.full_tiles >= 0 &&
            p.full_tiles <= tiles && p.split_k >= 1 && (int64_t)p.kblocks_per_split * p.split_k >= a.layout.k_blocks &&
            (p.full_tiles == tiles || (p.kblocks_per_split >= 1 && (int64_t)p.kblocks_per_split * (p.split_k - 1) < a.layout.k_blocks)) &&
            p.grid[0] == (unsigned)(p.full_tiles + (tiles - p.full_tiles) * p.split_k) && p.grid[1] == 1 && p.grid[2] == 1 &&

@@ -570,50 +570,56 @@ int launch_fc(const FcDeviceArgs& a, const LaunchPlan& p, void* stream) {
 
 // Time of a prefill launch, us: its start and end, the k-blocks that a compute unit goes through, and the sums of parts of K --
 // parked, and added by the last part to arrive alone.  Fitted to calls of 4096 -> 6144 / 4096 / 28672 and 14336 -> 4096, i4 in
-// groups of 64 and u4 in groups of 128, 140 to 2048 rows (off by 12 % at most): a k-block of a tile that has a compute unit to
-// itself takes 1.03 / 1.20 / 1.34 / 1.66 us at 64 / 80 / 96 / 128 rows, of tiles that share it `shared` of that each.
-static double prefill_us(int64_t tiles, int64_t kb, int split, int rows, double kblock_us, double shared, int n_cus) {
+// groups of 64 and u4 in groups of 128, 66 to 2048 rows (off by 12 % at most): kblock_us is what a k-block of a tile that has
+// a compute unit to itself takes; of tiles that share it, each takes `shared` of that.  cost: rows x 256 channels of a tile.
+static double prefill_us(int64_t tiles, int64_t kb, int split, double cost, double kblock_us, double shared, int n_cus) {
     const int64_t rounds = (tiles * split + n_cus - 1) / n_cus;
     return 4.0 + (double)((kb + split - 1) / split) * kblock_us * (rounds == 1 ? 1.0 : shared * (double)rounds) +
-           (split > 1 ? 1.0 + 2e-4 * (double)(tiles * split * rows) + 0.01 * split * rows : 0.0);
+           (split > 1 ? 1.0 + 2e-4 * (double)(tiles * split) * cost + 0.01 * split * cost : 0.0);
 }
 
 // Whether it can run a call that plan_launch gave to another of the 4-bit kernels.  (Not with one scale per channel: the others
 // keep such weights exact and add the halves of two wave groups, this one sums K in one chain.)
 bool pair_applies(const FcDeviceArgs& a, const LaunchPlan& p) {
     return p.kernel == OVFCC_KERNEL_PREFILL && p.async_dma && a.layout.groups > 1 && a.tile_rows == 0 && !a.want_async &&
-           a.M > kChunkedMaxRows;
+           a.M > kDecodeMaxRows;
 }
 
-// Its best launch by prefill_us.  K is cut only to fill the chip once: beyond, parts cost more than they fill (14336 -> 4096 at
-// 1000 rows 106 us in 256 or in 512 workgroups, 4096 -> 4096 36 in 256 and 42 in 512).  That also keeps the parked sums within 32 MiB.
+// Its best launch by prefill_us.  Tiles of 128 channels do half the unpacking per row of their k-block and take 0.6 of the time of
+// tiles of 256: they win where one round of tiles covers the call, the others where the work is long (activations cross LDS half as
+// often per product).  4096 -> 4096, 117 rows 18.9 / 14.4 us, 600 rows 32 / 27; 4096 -> 28672, 80 rows 33 / 27.5, but 371 rows 82 / 90.
+// K is cut only to fill the chip once: beyond, parts cost more than they fill (14336 -> 4096 at 1000 rows 106 us in 256 or in 512
+// workgroups of 256 channels, 4096 -> 4096 36 in 256 and 42 in 512).  That also keeps the parked sums within 32 MiB.
 double plan_pair(const FcDeviceArgs& a, int n_cus, LaunchPlan* plan, double shared) {
     static const int heights[4] = {128, 96, 80, 64};
-    static const double kblock_us[4] = {1.66, 1.34, 1.20, 1.03};
+    static const double kblock_us[2][4] = {{1.66, 1.34, 1.20, 1.06}, {1.02, 0.81, 0.74, 0.62}};  // 256 channels, 128
+    static const double share[2][4] = {{1.00, 1.00, 1.00, 1.00}, {1.10, 1.00, 0.98, 1.10}};
     const Layout& L = a.layout;
     LaunchPlan p = *plan;
-    // four waves instead of eight apply a gated linear unit (4096 -> 28672, 220 rows 53 / 58.8 us); two zero-points a step
-    const double more = (L.glu ? 1.06 : 1.0) * (L.groups_per_kblock == 4 && L.zp_table ? 1.04 : 1.0);
+    // four waves instead of eight apply a gated linear unit (4096 -> 28672, 220 rows 53 / 58.8 us); with two zero-points a
+    // step the 8-wave kernel is the slower one (3200 -> 18176, 1509 rows 208 / 186)
+    const double more = (L.glu ? 1.06 : 1.0) * (L.groups_per_kblock == 4 && L.zp_table ? 0.95 : 1.0);
     double best = -1.0;
-    for (int h = 0; h < 4; ++h) {
-        const int rows = heights[h];
-        if (rows > 80 && L.groups_per_kblock == 4 && L.zp_table)
+    for (int h = 0; h < 8; ++h) {
+        const int rows = heights[h & 3], channels = h < 4 ? kPrefillWideN : kPrefillWideN / 2;
+        if (rows > 80 && channels == kPrefillWideN && L.groups_per_kblock == 4 && L.zp_table)
             continue;  // (these run alone on a compute unit)
-        const int64_t nx = (a.N + kPrefillWideN - 1) / kPrefillWideN, ny = (a.M + rows - 1) / rows, tiles = nx * ny;
+        const int64_t nx = (a.N + channels - 1) / channels, ny = (a.M + rows - 1) / rows, tiles = nx * ny;
+        const double cost = (double)rows * channels / kPrefillWideN;
         for (int want = 1; want <= 8; ++want) {
             const int64_t per = (L.k_blocks + want - 1) / want;
             const int split = (int)((L.k_blocks + per - 1) / per);
-            if (split != want || (split > 1 && (per < 4 || tiles * split > n_cus)))
+            if (split != want || (split > 1 && (per < 8 || tiles * split > n_cus)))
                 continue;
-            const double us = prefill_us(tiles, L.k_blocks, split, rows, more * kblock_us[h], shared, n_cus);
+            const double us = prefill_us(tiles, L.k_blocks, split, cost, more * kblock_us[h >> 2][h & 3], shared * share[h >> 2][h & 3], n_cus);
             if (best >= 0.0 && us >= best)
                 continue;
             best = us;
-            p.tile_m = rows, p.tiles_x = (int)nx, p.tiles_y = (int)ny;
+            p.tile_m = rows, p.tile_n = channels, p.tiles_x = (int)nx, p.tiles_y = (int)ny;
             p.split_k = split, p.kblocks_per_split = (int)per;
             p.full_tiles = split == 1 ? (int)tiles : 0;
             p.grid[0] = (unsigned)(tiles * split), p.grid[1] = p.grid[2] = 1;
-            p.workspace_bytes = split > 1 ? (size_t)tiles * split * rows * kPrefillWideN * sizeof(float) : 0;
+            p.workspace_bytes = split > 1 ? (size_t)tiles * split * rows * channels * sizeof(float) : 0;
             p.counter_count = split > 1 ? (size_t)tiles : 0;
         }
     }
@@ -638,11 +644,11 @@ bool pair_preferred(const FcDeviceArgs& a, const LaunchPlan& p, int n_cus) {
     // where the two workgroups gain less.  4096 -> 28672 with the unit, 2048 rows 430 / 358 us, 5003 rows 991 / 888; without it
     // 4096 -> 14336, 5003 rows 465 / 434, but 8192 rows 682 / 688; 14336 -> 4096, 8192 rows 667 / 689.
     if (p.big)
-        return plan_pair(a, n_cus, &pair, 0.90) < prefill_us(tiles, kb, 1, 256, a.layout.glu ? 3.4 : 2.95, 1.0, n_cus);
+        return plan_pair(a, n_cus, &pair, 0.90) < prefill_us(tiles, kb, 1, 256.0, a.layout.glu ? 3.4 : 2.95, 1.0, n_cus);
     // The 8-wave kernel, which has a compute unit to itself: ahead where its tiles fit one round (7936 -> 7936 in groups of 32, 970
     // rows 117 / 133 us; 4096 -> 4096, 914 rows 39 / 43), behind where they do not or a lower or finer cut fits better
     // (4096 -> 28672, 371 rows 109 / 80; 14336 -> 4096, 600 rows 106 / 73; 4096 -> 6144, 3000 rows 174 / 127).
-    return plan_pair(a, n_cus, &pair) < prefill_us(tiles, kb, p.split_k, p.tile_m, p.tile_m == 64 ? 1.02 : 1.52, 1.0, n_cus);
+    return plan_pair(a, n_cus, &pair) < prefill_us(tiles, kb, p.split_k, p.tile_m, p.tile_m == 64 ? 1.05 : 1.52, 1.0, n_cus);
 }
 
 // Slice height of a grouped prefill launch over items of these row counts: every item is cut into equal slices of
