@@ -596,9 +596,9 @@ double plan_pair(const FcDeviceArgs& a, int n_cus, LaunchPlan* plan, double shar
     static const double share[2][4] = {{1.00, 1.00, 1.00, 1.00}, {1.10, 1.00, 0.98, 1.10}};
     const Layout& L = a.layout;
     LaunchPlan p = *plan;
-    // four waves instead of eight apply a gated linear unit (4096 -> 28672, 220 rows 53 / 58.8 us); with two zero-points a
-    // step the 8-wave kernel is the slower one (3200 -> 18176, 1509 rows 208 / 186)
-    const double more = (L.glu ? 1.06 : 1.0) * (L.groups_per_kblock == 4 && L.zp_table ? 0.95 : 1.0);
+    // four waves instead of eight apply a gated linear unit (4096 -> 28672, 220 rows 53 / 58.8 us in tiles of 256 channels); with
+    // two zero-points a step the 8-wave kernel is the slower one (3200 -> 18176, 1509 rows 208 / 186)
+    const double unit = L.glu ? 1.06 : 1.0, more = L.groups_per_kblock == 4 && L.zp_table ? 0.95 : 1.0;
     double best = -1.0;
     for (int h = 0; h < 8; ++h) {
         const int rows = heights[h & 3], channels = h < 4 ? kPrefillWideN : kPrefillWideN / 2;
@@ -611,7 +611,7 @@ double plan_pair(const FcDeviceArgs& a, int n_cus, LaunchPlan* plan, double shar
             const int split = (int)((L.k_blocks + per - 1) / per);
             if (split != want || (split > 1 && (per < 8 || tiles * split > n_cus)))
                 continue;
-            const double us = prefill_us(tiles, L.k_blocks, split, cost, more * kblock_us[h >> 2][h & 3], shared * share[h >> 2][h & 3], n_cus);
+            const double us = prefill_us(tiles, L.k_blocks, split, cost, (h < 4 ? unit * more : more) * kblock_us[h >> 2][h & 3], shared * share[h >> 2][h & 3], n_cus);
             if (best >= 0.0 && us >= best)
                 continue;
             best = us;
